@@ -571,7 +571,9 @@ __global__ __launch_bounds__(TILE_THREADS) void gemm_tile_kernel(GemmProblem p)
             // therefore start at the (aligned) beginning of the whole scale array.
             const int idx = (wave & 3) * 64 + lane;
             if (wave < 4) {
-                c.rs_sc = make_rsrc(p.sa, (uint32_t)min((int64_t)(p.T - 1) * psa + p.sld, (int64_t)lim));
+                // (rounded up to the dword that the last row's last scale lies in: the bounds check drops a dword that the
+                // size cuts, and an odd number of rows of an odd number of byte pairs ends inside one)
+                c.rs_sc = make_rsrc(p.sa, (uint32_t)min(((int64_t)(p.T - 1) * psa + p.sld + 3) & ~(int64_t)3, (int64_t)lim));
                 c.off_sc = ((uint32_t)(c.m0 + min(tile_row_of(idx), c.rows - 1)) * (uint32_t)psa) & ~3u;
             } else if (TB) {
                 c.rs_sc = make_rsrc(p.sb, (uint32_t)min((int64_t)p.num_groups * p.N * p.sld, (int64_t)lim));
