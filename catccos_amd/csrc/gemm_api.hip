@@ -26,6 +26,7 @@ static int run(const GemmProblem &prob, int kind, int epi, hipStream_t stream)
     GemmProblem p = prob;
     const int order = g_tile_order.load();
     p.tile_order = order >= 0 ? order : 2;
+    p.tile_kernel_only = order >= 0;
     p.i8_fp16_step = g_i8_fp16_step.load() != 0;
     const int nto = g_nt_out.load();
     p.nt_out = nto >= 0 ? nto : (kind == KIND_F4);

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "catccos_hip.h"
@@ -52,9 +53,17 @@ struct GemmProblem {
     int64_t b_stride;        // bytes between experts in b
     int64_t sb_stride;       // bytes between experts in sb
     int nt_out;              // tiled kernels: output stores carry the non-temporal hint
+    int tile_kernel_only;    // an order of its tiles was asked for: the 256 x 256 kernel, whatever the size
     int tile_order;          // tiled kernels: 0 = row-major over (row tile, column tile); 1 = runs of consecutive tiles per XCD;
                              // 2 = a block of 4 row tiles x 8 column tiles per XCD where the shape allows (else 1 for groups, 0 without)
 };
+
+// Upper bound of the row tiles of a problem whose group sizes only the device knows.
+inline int64_t row_tiles_bound(const GemmProblem &p, int tm)
+{
+    if (!p.group_sizes) return (p.T + tm - 1) / tm;
+    return p.T / tm + std::min<int64_t>(p.num_groups, p.T);
+}
 
 // Row ranges and tile counts of the groups, kept in LDS by every workgroup.
 //   row_start[g] .. row_start[g+1]   rows of group g (g == num_groups: rows past the last group,

@@ -1,0 +1,9 @@
+// Instantiates the weight-streaming GEMM template: MXFP8 kernels (plain epilogue), B stored [K, N] and [N, K].
+#include "gemm_stream_kernel.h"
+
+namespace cch {
+template int launch_stream_t<KIND_F8, EPI_PLAIN, CCH_FMT_E4M3, 0>(const GemmProblem &, int, hipStream_t);
+template int launch_stream_t<KIND_F8, EPI_PLAIN, CCH_FMT_E4M3, 1>(const GemmProblem &, int, hipStream_t);
+template int launch_stream_t<KIND_F8, EPI_PLAIN, CCH_FMT_E5M2, 0>(const GemmProblem &, int, hipStream_t);
+template int launch_stream_t<KIND_F8, EPI_PLAIN, CCH_FMT_E5M2, 1>(const GemmProblem &, int, hipStream_t);
+}  // namespace cch

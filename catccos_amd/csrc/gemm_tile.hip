@@ -1,17 +1,26 @@
 // Tiled MFMA GEMM family for gfx950: which problems the kernels take, and the choice of the instantiation.
 // The kernel template is gemm_tile_kernel.h; gemm_tile_<kind>_<layout>.hip instantiate it.
 #include <algorithm>
+#include <cmath>
 
 #include "common.h"
 #include "gemm_common.h"
+#include "gemm_mid.h"
+#include "gemm_stream.h"
 #include "gemm_tile_shape.h"
 
 namespace cch {
 
 template <int KIND, int EPI, int FMT, int TB> int launch_tile_t(const GemmProblem &p, hipStream_t stream);
+template <int KIND, int EPI, int FMT, int TB> int launch_stream_t(const GemmProblem &p, int waves, hipStream_t stream);
+template <int KIND, int EPI, int FMT, int TB> int launch_mid_t(const GemmProblem &p, int rows, int cols, hipStream_t stream);
 #define CCH_TILE_FAMILY(KIND, EPI, FMT) \
     extern template int launch_tile_t<KIND, EPI, FMT, 0>(const GemmProblem &, hipStream_t); \
-    extern template int launch_tile_t<KIND, EPI, FMT, 1>(const GemmProblem &, hipStream_t);
+    extern template int launch_tile_t<KIND, EPI, FMT, 1>(const GemmProblem &, hipStream_t); \
+    extern template int launch_stream_t<KIND, EPI, FMT, 0>(const GemmProblem &, int, hipStream_t); \
+    extern template int launch_stream_t<KIND, EPI, FMT, 1>(const GemmProblem &, int, hipStream_t); \
+    extern template int launch_mid_t<KIND, EPI, FMT, 0>(const GemmProblem &, int, int, hipStream_t); \
+    extern template int launch_mid_t<KIND, EPI, FMT, 1>(const GemmProblem &, int, int, hipStream_t);
 CCH_TILE_FAMILY(KIND_I8, EPI_DEQUANT, 0)
 CCH_TILE_FAMILY(KIND_I8, EPI_DEQUANT_SWIGLU, 0)
 CCH_TILE_FAMILY(KIND_F8, EPI_PLAIN, CCH_FMT_E4M3)
@@ -64,25 +73,98 @@ const char *gemm_tile_unsupported(const GemmProblem &p, int kind, int epi)
     return nullptr;
 }
 
+// ---- which of the kernels takes a problem
+//
+// The 256 x 256 tiles have the fewest bytes through L2 and LDS per product, and one persistent workgroup per CU; the smaller
+// tiles of the others fill more CUs, in shorter steps.  What decides is how many tiles there are to a CU and how long K is, so
+// each kernel has an estimate of its time,
+//     us = start + max(steps * max(step_alone, step_full * fill) + finish * fill, weights * per_mb),
+//     steps: 128-byte steps of K one wave walks, fill: tiles / CUs, weights: MB of right-hand operands,
+// and the smallest one wins (the 256 x 256 kernel unless another is estimated 8 % faster).  With one workgroup to a CU a last,
+// partly empty round costs at least half a full one: fill counts as floor(fill) + 0.5 + 0.5 * the rest.  The constants are a fit of
+// this form to the times of all kernels on 1200 problems (dense and grouped, all kinds and layouts, 1 to 16384 rows, K and N from
+// 256 to 8192) in which the choices count, not the times, which are off by 11 to 17 % each: the choices are within 1.5 % of the
+// best ones in the geometric mean, and 1.83 times faster than the 256 x 256 kernel on all of them (dense 2.1, grouped 1.6).
+enum GemmPath { PATH_TILE, PATH_MID1, PATH_MID2, PATH_MID3, PATH_STREAM4, PATH_STREAM8, NUM_PATHS };
+struct PathModel {
+    int tm, tn, waves_k;    // rows and columns of B per tile, waves that share a tile's K
+    bool rounds;            // one workgroup per CU
+    double start, step_alone, step_full, finish;
+    double per_mb[3];       // B as [N, K], as [K, N], and as [K, N] with gate and up columns apart (narrower pieces of a row)
+};
+static const PathModel PATH_MODEL[NUM_PATHS] = {
+    {256, 256, 1, true, 9.7, 1.27, 1.66, 3.9, {0.30, 0.20, 0.21}},
+    {64, 128, 1, false, 4.5, 0.37, 0.50, 1.55, {0.18, 0.22, 0.22}},
+    {128, 128, 1, false, 5.75, 0.48, 0.65, 1.55, {0.19, 0.22, 0.27}},
+    {128, 256, 1, true, 5.6, 0.69, 1.07, 4.9, {0.20, 0.22, 0.205}},
+    {STREAM_TM, STREAM_TN, 4, false, 3.35, 0.95, 1.09, 1.05, {0.245, 0.29, 0.30}},
+    {STREAM_TM, STREAM_TN, 8, false, 3.7, 1.24, 1.92, 2.0, {0.21, 0.255, 0.46}},
+};
+
+static GemmPath choose_path(const GemmProblem &p, int kind, int epi, int cus)
+{
+    const int epb = kind == KIND_F4 ? 2 : 1;
+    const bool swiglu = epi == EPI_DEQUANT_SWIGLU || epi == EPI_SWIGLU;
+    if (p.tile_kernel_only) return PATH_TILE;
+    // the smaller kernels add up to 512 K-rows of a [K, N] operand to offsets below 2^31
+    if (!p.trans_b && p.N / epb >= 1 << 21) return PATH_TILE;
+    const double steps = (p.K / epb + BKB - 1) / BKB;
+    const double groups = std::min<int64_t>(p.num_groups, p.T);   // that can have rows
+    const double weights = groups * (double)p.N * (p.K / epb) * 1e-6;
+    const int layout = p.trans_b ? 0 : swiglu ? 2 : 1;
+    GemmPath best = PATH_TILE;
+    double best_us = 0.0;
+    for (int i = 0; i < NUM_PATHS; i++) {
+        const PathModel &m = PATH_MODEL[i];
+        // a group's last row tile is half full on average; groups of a few rows have one tile each
+        const double row_tiles = p.group_sizes ? std::max<double>(groups, (double)p.T / m.tm + 0.5 * groups) : (double)((p.T + m.tm - 1) / m.tm);
+        const int tn_out = swiglu ? m.tn / 2 : m.tn;
+        const double fill = row_tiles * ((p.n_out + tn_out - 1) / tn_out) / cus, whole = std::floor(fill);
+        const double rounds = m.rounds && fill > 1.0 && fill > whole ? whole + 0.5 + 0.5 * (fill - whole) : fill;
+        const double us = m.start + std::max(steps / m.waves_k * std::max(m.step_alone, m.step_full * rounds) + m.finish * fill, weights * m.per_mb[layout]);
+        if (i == PATH_TILE) {
+            best_us = 0.92 * us;
+        } else if (us < best_us) {
+            best = (GemmPath)i;
+            best_us = us;
+        }
+    }
+    return best;
+}
+
+template <int KIND, int EPI, int FMT>
+static int launch_family(const GemmProblem &p, hipStream_t stream)
+{
+    int dev = 0, cus = 0;
+    CCH_HIP(hipGetDevice(&dev));
+    CCH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    const GemmPath path = choose_path(p, KIND, EPI, cus);
+    switch (path) {
+    case PATH_MID1:
+    case PATH_MID2:
+    case PATH_MID3: {
+        const int rows = PATH_MODEL[path].tm, cols = PATH_MODEL[path].tn;
+        return p.trans_b ? launch_mid_t<KIND, EPI, FMT, 1>(p, rows, cols, stream) : launch_mid_t<KIND, EPI, FMT, 0>(p, rows, cols, stream);
+    }
+    case PATH_STREAM4:
+    case PATH_STREAM8: {
+        const int waves = path == PATH_STREAM4 ? 4 : 8;
+        return p.trans_b ? launch_stream_t<KIND, EPI, FMT, 1>(p, waves, stream) : launch_stream_t<KIND, EPI, FMT, 0>(p, waves, stream);
+    }
+    default: return p.trans_b ? launch_tile_t<KIND, EPI, FMT, 1>(p, stream) : launch_tile_t<KIND, EPI, FMT, 0>(p, stream);
+    }
+}
+
 int launch_gemm_tile(const GemmProblem &p, int kind, int epi, hipStream_t stream)
 {
-    const bool tb = p.trans_b != 0;
-    if (kind == KIND_I8 && epi == EPI_DEQUANT)
-        return tb ? launch_tile_t<KIND_I8, EPI_DEQUANT, 0, 1>(p, stream) : launch_tile_t<KIND_I8, EPI_DEQUANT, 0, 0>(p, stream);
-    if (kind == KIND_I8 && epi == EPI_DEQUANT_SWIGLU)
-        return tb ? launch_tile_t<KIND_I8, EPI_DEQUANT_SWIGLU, 0, 1>(p, stream) : launch_tile_t<KIND_I8, EPI_DEQUANT_SWIGLU, 0, 0>(p, stream);
-    if (kind == KIND_F8 && epi == EPI_PLAIN && p.fmt == CCH_FMT_E4M3)
-        return tb ? launch_tile_t<KIND_F8, EPI_PLAIN, CCH_FMT_E4M3, 1>(p, stream) : launch_tile_t<KIND_F8, EPI_PLAIN, CCH_FMT_E4M3, 0>(p, stream);
-    if (kind == KIND_F8 && epi == EPI_PLAIN && p.fmt == CCH_FMT_E5M2)
-        return tb ? launch_tile_t<KIND_F8, EPI_PLAIN, CCH_FMT_E5M2, 1>(p, stream) : launch_tile_t<KIND_F8, EPI_PLAIN, CCH_FMT_E5M2, 0>(p, stream);
-    if (kind == KIND_F4 && epi == EPI_PLAIN)
-        return tb ? launch_tile_t<KIND_F4, EPI_PLAIN, CCH_FMT_E2M1, 1>(p, stream) : launch_tile_t<KIND_F4, EPI_PLAIN, CCH_FMT_E2M1, 0>(p, stream);
-    if (kind == KIND_F8 && epi == EPI_SWIGLU && p.fmt == CCH_FMT_E4M3)
-        return tb ? launch_tile_t<KIND_F8, EPI_SWIGLU, CCH_FMT_E4M3, 1>(p, stream) : launch_tile_t<KIND_F8, EPI_SWIGLU, CCH_FMT_E4M3, 0>(p, stream);
-    if (kind == KIND_F8 && epi == EPI_SWIGLU && p.fmt == CCH_FMT_E5M2)
-        return tb ? launch_tile_t<KIND_F8, EPI_SWIGLU, CCH_FMT_E5M2, 1>(p, stream) : launch_tile_t<KIND_F8, EPI_SWIGLU, CCH_FMT_E5M2, 0>(p, stream);
-    if (kind == KIND_F4 && epi == EPI_SWIGLU)
-        return tb ? launch_tile_t<KIND_F4, EPI_SWIGLU, CCH_FMT_E2M1, 1>(p, stream) : launch_tile_t<KIND_F4, EPI_SWIGLU, CCH_FMT_E2M1, 0>(p, stream);
+    if (kind == KIND_I8 && epi == EPI_DEQUANT) return launch_family<KIND_I8, EPI_DEQUANT, 0>(p, stream);
+    if (kind == KIND_I8 && epi == EPI_DEQUANT_SWIGLU) return launch_family<KIND_I8, EPI_DEQUANT_SWIGLU, 0>(p, stream);
+    if (kind == KIND_F8 && epi == EPI_PLAIN && p.fmt == CCH_FMT_E4M3) return launch_family<KIND_F8, EPI_PLAIN, CCH_FMT_E4M3>(p, stream);
+    if (kind == KIND_F8 && epi == EPI_PLAIN && p.fmt == CCH_FMT_E5M2) return launch_family<KIND_F8, EPI_PLAIN, CCH_FMT_E5M2>(p, stream);
+    if (kind == KIND_F4 && epi == EPI_PLAIN) return launch_family<KIND_F4, EPI_PLAIN, CCH_FMT_E2M1>(p, stream);
+    if (kind == KIND_F8 && epi == EPI_SWIGLU && p.fmt == CCH_FMT_E4M3) return launch_family<KIND_F8, EPI_SWIGLU, CCH_FMT_E4M3>(p, stream);
+    if (kind == KIND_F8 && epi == EPI_SWIGLU && p.fmt == CCH_FMT_E5M2) return launch_family<KIND_F8, EPI_SWIGLU, CCH_FMT_E5M2>(p, stream);
+    if (kind == KIND_F4 && epi == EPI_SWIGLU) return launch_family<KIND_F4, EPI_SWIGLU, CCH_FMT_E2M1>(p, stream);
     return fail(CCH_ENOSUP, "no tiled GEMM kernel for kind %d with epilogue %d, trans_b %d", kind, epi, p.trans_b);
 }
 

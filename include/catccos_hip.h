@@ -339,7 +339,8 @@ int cch_dyn_quant_i8_rows_smooth(const void *x, const int32_t *src_rows, const f
  * over (row tile, column tile), 1 = each XCD takes a run of consecutive tiles of every round (whole
  * row tiles next to each other: fewer token and weight panels per L2), 2 = each XCD takes a block of
  * 4 row tiles x 8 column tiles of every round (where 8, 16, 32 or 64 column tiles and 256 workgroups
- * allow it; else 1 for grouped problems and 0 for dense ones), -1 (default) = 2;
+ * allow it; else 1 for grouped problems and 0 for dense ones), -1 (default) = 2; an order set here also keeps problems of every
+ * size on those kernels (by default the ones too small for 256 x 256 tiles go to kernels with smaller tiles);
  * "i8_epilogue_fp16_step" = 1 makes the int8 epilogues (cch_gemm_i8_dequant*, cch_gmm_i8_dequant*, both kernel paths)
  * round acc * per_channel to IEEE half before the per-token factor, as the reference's device kernel does
  * (include/catccos/epilogue/block/block_epilogue_per_token_dequant_swiglu.hpp:348-361: the matrix unit's output stage
