@@ -51,6 +51,19 @@ def test_routing_one_workgroup_equals_three_launches(case):
                 assert np.array_equal(a, w)
 
 
+@pytest.mark.parametrize("rows", [1023, 1024, 1025, 2048, 2049, 4096, 4097, 8191, 8192])
+@pytest.mark.parametrize("e", [1, 64, 65, 256])
+def test_routing_one_workgroup_edges(rows, e):
+    """The one-workgroup kernel is instantiated on the 64-row groups of a wave (1, 2, 4, 8) and scans experts 64 at a time:
+    the row counts and expert counts on either side of each limit, with dropped routes (which leave -1 behind the last)."""
+    rng = np.random.default_rng(rows * 31 + e)
+    idx = rng.integers(-1, e + 1, rows).astype(np.int32)
+    for cumsum in (False, True):
+        got = [t.cpu().numpy() for t in cc.moe_init_routing(torch.from_numpy(idx).cuda(), e, cumsum)]
+        for a, w in zip(got, orc.moe_init_routing(idx, e, cumsum)):
+            assert np.array_equal(a, w)
+
+
 def test_routing_skewed_and_sorted_inputs():
     for idx in (np.zeros(5000, np.int32), np.arange(5000, dtype=np.int32) % 7, np.sort(np.arange(5000, dtype=np.int32) % 7)[::-1].copy()):
         d2s, s2d, cnt = cc.moe_init_routing(torch.from_numpy(idx).cuda(), 7)
