@@ -1,6 +1,6 @@
 // Per-token dynamic int8 quantiser with row gather: the step that turns bf16 tokens into the
 // int8 rows and per-token scales the MoE grouped GEMM consumes.  Streaming, HBM-bound: one wave
-// owns one output row (two or four waves share a row longer than 4096 columns), keeps it in
+// owns one output row (up to eight waves share a row of few or a long one), keeps it in
 // registers (16-byte non-temporal loads, up to 16384 columns), reduces |x| across the wave(s), and
 // writes 8 int8 per lane per chunk.  Longer rows are read twice.
 //
@@ -21,6 +21,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int DQ_THREADS = 256;   // 4 rows per workgroup
+constexpr int DQ_FEW_ROWS = 256;  // rows that get a workgroup (of up to eight waves) each
 constexpr int DQ_MAX_CHUNKS = 32; // 32 x 512 columns held in registers, by up to four waves
 
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v)
@@ -78,16 +79,17 @@ __device__ __forceinline__ int quant_one(float v, const RowDivisor &d)
 // registers per wave for full occupancy, and the grid has WPR times as many, shorter, pieces of
 // work.  The partial maxima meet in LDS.  SMOOTH: every element is first multiplied by the row's
 // fp32 smoothing vector (vector `smooth_rows[row]`, or vector 0 without that list).
+constexpr int dq_threads(int wpr) { return wpr * 64 > DQ_THREADS ? wpr * 64 : DQ_THREADS; }
 template <int MODE, int CHUNKS, int WPR = 1, bool SMOOTH = false>
-__global__ __launch_bounds__(DQ_THREADS) void dyn_quant_rows_kernel(const uint16_t *__restrict__ x, const int32_t *__restrict__ src,
+__global__ __launch_bounds__(dq_threads(WPR)) void dyn_quant_rows_kernel(const uint16_t *__restrict__ x, const int32_t *__restrict__ src,
                                                                    const float *__restrict__ smooth,
                                                                    const int32_t *__restrict__ smooth_rows, int num_smooth,
                                                                    int8_t *__restrict__ q, float *__restrict__ scale, int rows_in,
                                                                    int T, int K, int topk)
 {
-    constexpr int ROWS_PER_WG = DQ_THREADS / 64 / WPR;
+    constexpr int ROWS_PER_WG = dq_threads(WPR) / 64 / WPR;
     constexpr int NW = SMOOTH ? 8 : 4;   // registers per chunk: fp32 products or bf16 pairs
-    __shared__ uint32_t part[DQ_THREADS / 64];
+    __shared__ uint32_t part[dq_threads(WPR) / 64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int share = wave % WPR;   // which part of the row this wave owns
@@ -198,16 +200,25 @@ static int launch_dq(const void *x, const int32_t *src, const float *smooth, con
     const int chunks = vec ? (int)((k + 511) / 512) : DQ_MAX_CHUNKS + 1;
 #define CCH_DQ_LAUNCH(C, W)                                                                                                \
     do {                                                                                                                   \
-        constexpr int rows_per_wg = DQ_THREADS / 64 / W;                                                                   \
+        constexpr int rows_per_wg = dq_threads(W) / 64 / W;                                                                \
         const unsigned grid = (unsigned)((t + rows_per_wg - 1) / rows_per_wg);                                             \
-        hipLaunchKernelGGL((dyn_quant_rows_kernel<MODE, C, W, SMOOTH>), dim3(grid), dim3(DQ_THREADS), 0, stream,           \
+        hipLaunchKernelGGL((dyn_quant_rows_kernel<MODE, C, W, SMOOTH>), dim3(grid), dim3(dq_threads(W)), 0, stream,        \
                            static_cast<const uint16_t *>(x), src, smooth, smooth_rows, num_smooth, static_cast<int8_t *>(q), \
                            scale, (int)rows_in, (int)t, (int)k, topk);                                                     \
     } while (0)
     // four chunks per wave where the row allows: few registers (full occupancy) and many short
     // pieces of work measured fastest (5.8 TB/s at K = 7168 against 5.4 with two waves per row
     // and 5.0 with one)
-    if (chunks <= 4) CCH_DQ_LAUNCH(4, 1);
+    // Few rows (a decode step): up to DQ_FEW_ROWS of them are on the chip at a time whatever the split, so the
+    // time is one wave's chain of instructions, and a row is shared by as many waves as it has chunks.
+    // Measured (two and four waves of four chunks -> this): 64 x 4096 4.3 -> 3.2 us, 96 x 2048 4.0 -> 3.1, 64 x 7168 4.2 -> 3.6,
+    // 256 x 4096 4.4 -> 3.4, 256 x 8192 4.9 -> 4.3; from 512 rows on the split below is as fast or faster.
+    if (t <= DQ_FEW_ROWS && chunks <= 16) {
+        if (chunks <= 1) CCH_DQ_LAUNCH(1, 1);
+        else if (chunks <= 4) CCH_DQ_LAUNCH(1, 4);
+        else if (chunks <= 8) CCH_DQ_LAUNCH(1, 8);
+        else CCH_DQ_LAUNCH(2, 8);
+    } else if (chunks <= 4) CCH_DQ_LAUNCH(4, 1);
     else if (chunks <= 8) CCH_DQ_LAUNCH(4, 2);
     else if (chunks <= 16) CCH_DQ_LAUNCH(4, 4);
     else if (chunks <= 32) CCH_DQ_LAUNCH(8, 4);

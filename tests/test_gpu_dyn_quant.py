@@ -34,6 +34,24 @@ def test_dyn_quant_bit_exact(shape, mode):
     assert np.array_equal(q.cpu().numpy(), wq)
 
 
+@pytest.mark.parametrize("mode", [cc.DQ_DEVICE, cc.DQ_GOLDEN])
+@pytest.mark.parametrize("k", [8, 512, 520, 2048, 2056, 4096, 4104, 8192])
+@pytest.mark.parametrize("rows", [256, 257])
+def test_dyn_quant_either_side_of_the_few_rows_limit(rows, k, mode):
+    """Up to 256 rows a row is shared by as many waves as it has 512-column chunks, beyond that by fewer: the same bytes at
+    the edges of every split, with a gather that drops and repeats rows."""
+    rng = np.random.default_rng(rows * 17 + k + mode)
+    xb = rand_rows(rng, rows, k, 2.5)
+    xb[3] = 0
+    src = rng.integers(-1, rows + 1, rows).astype(np.int32)
+    for rm in (None, src):
+        q, s = cc.dynamic_quant_i8(dev_bf16(xb), None if rm is None else torch.from_numpy(rm).cuda(), 1, mode)
+        xs = xb if rm is None else np.where(((rm >= 0) & (rm < rows))[:, None], xb[np.clip(rm, 0, rows - 1)], np.uint16(0))
+        wq, ws = orc.dyn_quant_i8_rows(xs, mode=mode)
+        assert np.array_equal(s.cpu().numpy(), ws)
+        assert np.array_equal(q.cpu().numpy(), wq)
+
+
 def test_dyn_quant_ties_and_extremes():
     # rows built so that x / scale lands on .5 boundaries and on half-precision truncation edges
     k = 512
