@@ -46,7 +46,7 @@ def test_scatter_vector_path(shape, fmt):
 @pytest.mark.parametrize("fmt", ["e4m3", "e2m1"])
 @pytest.mark.parametrize("shape", [(11, 64, 2), (5, 100, 3), (9, 31, 2), (6, 1000, 5), (3, 8200, 1)])
 def test_scatter_byte_path_and_ragged_k(shape, fmt):
-    # packed rows of these K are not multiples of 8 bytes (or K is ragged): byte stores
+    # packed rows of these K are not multiples of 8 bytes (vector stores off their alignment), or K is ragged (byte stores)
     tokens, k, topk = shape
     run_case(tokens, k, topk, fmt, cc.ROUND_RNE, tokens * 3 + k)
 
