@@ -9,6 +9,7 @@ Outputs (git-ignored, shipped as built files):
     catccos_amd/libcatccos_host.so     C++ operator surface  (catccos_amd/csrc/host/)
     catccos_amd/catccos_run            command-line driver over the operator surface
     catccos_amd/libcatccos_torch.so    torch.ops.catccos.* (C++ TORCH_LIBRARY, catccos_amd/csrc/torch/)
+    catccos_amd/_direct.so             native form of the entry points of ops.py (CPython module, catccos_amd/csrc/torch/)
 """
 import argparse
 import concurrent.futures
@@ -25,6 +26,7 @@ LIB = os.path.join(PKG, "libcatccos_hip.so")
 HOST_LIB = os.path.join(PKG, "libcatccos_host.so")
 DRIVER = os.path.join(PKG, "catccos_run")
 TORCH_LIB = os.path.join(PKG, "libcatccos_torch.so")
+DIRECT = os.path.join(PKG, "_direct.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_FLAGS = [
@@ -83,20 +85,27 @@ def build_host():
     return HOST_LIB
 
 
-def build_torch():
-    """torch.ops.catccos.* as a C++ TORCH_LIBRARY (catccos_amd/csrc/torch/torch_bindings.cpp): host code only, against
-    this interpreter's PyTorch and the HIP library above."""
+def _torch_cmd(src, out, extra):
     import torch
     from torch.utils import cpp_extension as ce
-    src = os.path.join(CSRC, "torch", "torch_bindings.cpp")
     tlib = ce.library_paths()[0]
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unused-function",
-           # the platform macro the HIP runtime headers ask for, and PyTorch's switch for its ROCm headers
-           "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
-           "-I" + os.path.join(ROOT, "include"), "-I/opt/rocm/include"] + ["-isystem" + d for d in ce.include_paths()] + [
-           src, "-o", TORCH_LIB, "-L" + tlib, "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_hip", "-L" + PKG, "-lcatccos_hip",
-           "-Wl,-rpath,$ORIGIN", "-Wl,-rpath," + tlib]
-    _run(cmd)
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unused-function",
+            # the platform macro the HIP runtime headers ask for, and PyTorch's switch for its ROCm headers
+            "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
+            "-I" + os.path.join(ROOT, "include"), "-I/opt/rocm/include"] + ["-isystem" + d for d in ce.include_paths()] + [
+            src, "-o", out, "-L" + tlib, "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_hip"] + extra + [
+            "-L" + PKG, "-lcatccos_hip", "-Wl,-rpath,$ORIGIN", "-Wl,-rpath," + tlib]
+
+
+def build_torch():
+    """torch.ops.catccos.* as a C++ TORCH_LIBRARY (catccos_amd/csrc/torch/torch_bindings.cpp) and the CPython module behind
+    ops.py (direct_calls.cpp): host code only, against this interpreter's PyTorch and the HIP library above."""
+    import sysconfig
+    tdir = os.path.join(CSRC, "torch")
+    cmds = [_torch_cmd(os.path.join(tdir, "torch_bindings.cpp"), TORCH_LIB, []),
+            _torch_cmd(os.path.join(tdir, "direct_calls.cpp"), DIRECT, ["-isystem" + sysconfig.get_paths()["include"], "-ltorch_python"])]
+    with concurrent.futures.ThreadPoolExecutor(max_workers=2) as ex:
+        list(ex.map(_run, cmds))
     return TORCH_LIB
 
 

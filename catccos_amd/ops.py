@@ -3,7 +3,12 @@
 make inputs contiguous, allocate the output, take the current stream, call the C ABI.
 
 torch is used for device memory and streams only; all arithmetic happens in the HIP library.
+
+The entry points of a serving program's inner loop first offer the call to their native form (csrc/torch/direct_calls.cpp), which
+takes plain contiguous GPU tensors of the right types and shapes and answers NotImplemented to everything else.
 """
+import importlib as _importlib
+
 import torch
 
 from . import _abi
@@ -39,6 +44,22 @@ def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
+class _Direct:
+    """The native forms, loaded with the first call (like the library, whose absence is an error too)."""
+
+    def __getattr__(self, name):
+        try:
+            mod = _importlib.import_module("._direct", __package__)
+        except ImportError as e:
+            raise FileNotFoundError("catccos_amd/_direct.so is missing or does not load (build it with `python -m catccos_amd.build`): %s" % e) from e
+        for f in ("mx_quant", "dynamic_quant_i8", "moe_init_routing", "w8a8_matmul_dequant", "gmm_i8", "mx_matmul", "mx_grouped_matmul", "moe_ffn_mxfp8"):
+            setattr(self, f, getattr(mod, f))
+        return getattr(mod, name)
+
+
+_direct = _Direct()
+
+
 def scale_cols(k):
     """E8M0 bytes per row for a K extent: block count padded to even."""
     return 2 * ((k + 63) // 64)
@@ -49,6 +70,9 @@ def mx_quant(x, fmt="e4m3", rounding=ROUND_RNE):
 
     Returns (payload uint8 [M, K] or [M, ceil(K/2)] for FP4, scales uint8 [M, scale_cols(K)]).
     """
+    r = _direct.mx_quant(x, fmt, rounding)
+    if r is not NotImplemented:
+        return r
     fmt = _fmt(fmt)
     _require_gpu(x)
     if x.dim() != 2 or x.dtype not in (torch.bfloat16, torch.float16):
@@ -131,6 +155,10 @@ def dynamic_quant_i8(x, src_rows=None, topk=1, mode=DQ_DEVICE, smooth=None, smoo
     smooth_rows[i] (vector 0 without `smooth_rows`).  Returns (q int8 [T, K], scale float32 [T])
     with scale = amax(row) / 127.
     """
+    if smooth is None and smooth_rows is None:
+        r = _direct.dynamic_quant_i8(x, src_rows, topk, mode)
+        if r is not NotImplemented:
+            return r
     _require_gpu(x)
     if x.dim() != 2 or x.dtype != torch.bfloat16:
         raise ValueError("dynamic_quant_i8 expects a 2-D bfloat16 tensor")
@@ -175,6 +203,9 @@ def moe_init_routing(expert_idx, num_experts, cumsum=False):
     Returns (dst_to_src, src_to_dst, expert_tokens): the flat entry at every sorted position (-1 past
     the routed entries), the sorted position of every flat entry (-1 if dropped), and the entries
     per expert (their running sum with cumsum=True)."""
+    r = _direct.moe_init_routing(expert_idx, num_experts, cumsum)
+    if r is not NotImplemented:
+        return r
     _require_gpu(expert_idx)
     if expert_idx.dtype != torch.int32:
         raise ValueError("expert_idx must be an int32 tensor")
@@ -233,6 +264,9 @@ def _check_2d(name, t, dtype):
 
 def w8a8_matmul_dequant(a, b, per_tok, per_ch, trans_b=0, out_dtype=torch.bfloat16):
     """int8 [M,K] x int8 [K,N] (or [N,K] with trans_b=1) -> bf16 (or half) [M,N], scaled per token and per channel."""
+    r = _direct.w8a8_matmul_dequant(a, b, per_tok, per_ch, trans_b, out_dtype)
+    if r is not NotImplemented:
+        return r
     code = _out_code(out_dtype)
     _require_gpu(a, b, per_tok, per_ch)
     _check_2d("a", a, torch.int8)
@@ -271,6 +305,10 @@ def gmm_dequant_swiglu_mx(x, w, group_sizes, per_tok, per_ch, trans_b=0, fmt="e4
 
 
 def _gmm_i8(x, w, group_sizes, per_tok, per_ch, trans_b, swiglu, out_dtype=torch.bfloat16, mx_fmt=None):
+    if mx_fmt is None:
+        r = _direct.gmm_i8(x, w, group_sizes, per_tok, per_ch, trans_b, swiglu, out_dtype)
+        if r is not NotImplemented:
+            return r
     code = _out_code(out_dtype)
     _require_gpu(x, w, group_sizes, per_tok, per_ch)
     _check_2d("x", x, torch.int8)
@@ -332,6 +370,9 @@ def _mx_shapes(a, sa, b, sb, fmt, trans_b, grouped):
 
 def mx_matmul(a, sa, b, sb, fmt="e4m3", trans_b=0, out_dtype=torch.bfloat16):
     """MX dense GEMM: payload/scales as produced by mx_quant (a) and mx_quant_b (b); bf16 (or half) [M,N]."""
+    r = _direct.mx_matmul(a, sa, b, sb, fmt, trans_b, out_dtype)
+    if r is not NotImplemented:
+        return r
     code = _out_code(out_dtype)
     _require_gpu(a, sa, b, sb)
     a, sa, b, sb = a.contiguous(), sa.contiguous(), b.contiguous(), sb.contiguous()
@@ -344,6 +385,9 @@ def mx_matmul(a, sa, b, sb, fmt="e4m3", trans_b=0, out_dtype=torch.bfloat16):
 def mx_grouped_matmul(a, sa, b, sb, group_sizes, fmt="e4m3", trans_b=0, out_dtype=torch.bfloat16):
     """MX grouped GEMM: rows of a grouped by expert (group_sizes int32 [E] on the device),
     b [E,...] / sb [E,...] one operand per expert; bf16 (or, with out_dtype=torch.float16, half) [T,N]."""
+    r = _direct.mx_grouped_matmul(a, sa, b, sb, group_sizes, fmt, trans_b, out_dtype)
+    if r is not NotImplemented:
+        return r
     _require_gpu(a, sa, b, sb, group_sizes)
     if group_sizes.dtype != torch.int32 or group_sizes.dim() != 1:
         raise ValueError("group_sizes must be a 1-D int32 tensor")
@@ -448,6 +492,9 @@ def moe_ffn_mxfp8(x, expert_idx, probs, w1, sw1, w2, sw2, trans_b=1):
     x bf16 [m, k]; expert_idx int32 [m, top_k]; probs float32 [m, top_k]; w1 / sw1 and w2 / sw2 E4M3 payload and E8M0 scales
     of the experts' up ([k, n], gate columns first) and down ([n/2, k]) projections in the layout `trans_b` names
     (1, as the reference's files hold them: [E, n, k] and [E, k, n/2]).  Returns bf16 [m, k]."""
+    r = _direct.moe_ffn_mxfp8(x, expert_idx, probs, w1, sw1, w2, sw2, trans_b)
+    if r is not NotImplemented:
+        return r
     _require_gpu(x, expert_idx, probs, w1, sw1, w2, sw2)
     if x.dim() != 2 or x.dtype != torch.bfloat16:
         raise ValueError("x must be a 2-D bfloat16 tensor")
