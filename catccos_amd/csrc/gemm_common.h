@@ -16,6 +16,7 @@ enum GemmKind { KIND_I8 = 0, KIND_F8 = 1, KIND_F4 = 2 };
 enum GemmEpilogue { EPI_PLAIN = 0, EPI_DEQUANT = 1, EPI_DEQUANT_SWIGLU = 2, EPI_SWIGLU = 3 };
 
 constexpr int MAX_GROUPS = 256;
+constexpr int TAIL_TILES = 512;   // most tiles that the second launch of a grouped problem may have (gemm_tail.h): one round of its kernel
 
 // One (dense or grouped) problem: out[T, n_out] = epilogue(A[T,K] x B_e[K,N]).
 struct GemmProblem {
@@ -52,6 +53,8 @@ struct GemmProblem {
     int sld;                 // scale bytes per row: 2*ceil(K/64)
     int64_t b_stride;        // bytes between experts in b
     int64_t sb_stride;       // bytes between experts in sb
+    int tail_cus;            // grouped problems, 256 x 256 kernel: CUs, if a second launch takes the last rows of some groups
+                             // (gemm_tail.h); 0: it takes them all itself
     int nt_out;              // tiled kernels: output stores carry the non-temporal hint
     int tile_kernel_only;    // an order of its tiles was asked for: the 256 x 256 kernel, whatever the size
     int tile_order;          // tiled kernels: 0 = row-major over (row tile, column tile); 1 = runs of consecutive tiles per XCD;

@@ -1,7 +1,8 @@
 // What happens to eight neighbouring results of one row at the end of a tile: shared by the kernels whose accumulators pass
 // through LDS as fp32 (int32) rows.
 #pragma once
-#include "gemm_device.h"
+#include "gemm_mid.h"
+#include "gemm_tail.h"
 
 namespace cch {
 
@@ -134,6 +135,42 @@ __device__ __forceinline__ GroupPlace find_place(const GemmProblem &p, int tile,
     }
     g.used = (int)min(before, (uint32_t)p.T);
     g.total = tiles_before * n_tiles;
+    return g;
+}
+
+// The same for the second launch of a problem (gemm_tail.h): the groups' rows are those that the first left out.
+template <bool SWIGLU>
+__device__ __forceinline__ GroupPlace find_tail(const GemmProblem &p, int block, int tm, int n_tiles, int round_size)
+{
+    GroupPlace g = {};
+    const GroupRows rows = group_rows(p);
+    const uint32_t key = tail_key<SWIGLU>(p, rows);
+    int tiles_before = 0, tiles[GroupRows::NB], start[GroupRows::NB];
+#pragma unroll
+    for (int b = 0; b < GroupRows::NB; b++) {
+        tiles[b] = start[b] = 0;
+        if (b * 64 < p.num_groups) {
+            tiles[b] = in_tail(rows, b, key) ? (((rows.hi[b] - rows.lo[b]) & (BM - 1)) + tm - 1) / tm : 0;
+            const int incl = (int)wave_scan_sat((uint32_t)tiles[b]);
+            start[b] = (tiles_before + incl - tiles[b]) * n_tiles;
+            tiles_before += __builtin_amdgcn_readlane(incl, 63);
+        }
+    }
+    g.total = tiles_before * n_tiles;
+    const int tile = mid_tile_of(block, g.total, round_size);
+#pragma unroll
+    for (int b = 0; b < GroupRows::NB; b++) {
+        const uint64_t hit = __ballot(tile >= start[b] && tile < start[b] + tiles[b] * n_tiles);
+        if (hit != 0) {
+            const int l = __builtin_ctzll(hit);
+            g.found = true;
+            g.e = b * 64 + l;
+            g.hi = __builtin_amdgcn_readlane(rows.hi[b], l);
+            g.lo = g.hi - ((g.hi - __builtin_amdgcn_readlane(rows.lo[b], l)) & (BM - 1));
+            g.rel = tile - __builtin_amdgcn_readlane(start[b], l);
+            g.rt = __builtin_amdgcn_readlane(tiles[b], l);
+        }
+    }
     return g;
 }
 

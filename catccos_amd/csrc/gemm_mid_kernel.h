@@ -65,6 +65,14 @@ __global__ __launch_bounds__(128 * WN, 2) void gemm_mid_kernel(GemmProblem p)
         rt = (p.T + TM - 1) / TM;
         rel = mid_tile_of((int)blockIdx.x, rt * n_tiles, mid_round(WN));
         if (rel < 0) return;
+    } else if (MB == 1 && p.tail_cus) {
+        const GroupPlace at = find_tail<SWIGLU>(p, (int)blockIdx.x, TM, n_tiles, mid_round(WN));
+        if (!at.found) return;
+        e = at.e;
+        lo = at.lo;
+        hi = at.hi;
+        rel = at.rel;
+        rt = at.rt;
     } else {
         const GroupPlace all = find_place(p, -1, TM, n_tiles);
         zero_rest<EPI>(p, all.used);
@@ -453,7 +461,8 @@ static int launch_mid_mb(const GemmProblem &p, hipStream_t stream)
         attr_set.fetch_or(dev_bit, std::memory_order_release);
     }
     constexpr int tn_out = (EPI == EPI_DEQUANT_SWIGLU || EPI == EPI_SWIGLU) ? 32 * WN : 64 * WN;
-    const int64_t tiles = row_tiles_bound(p, 64 * MB) * ((p.n_out + tn_out - 1) / tn_out);
+    const int64_t col_tiles = (p.n_out + tn_out - 1) / tn_out;
+    const int64_t tiles = p.tail_cus ? std::min<int64_t>(TAIL_TILES, p.num_groups * (TAIL_ROWS / 64) * col_tiles) : row_tiles_bound(p, 64 * MB) * col_tiles;
     hipLaunchKernelGGL(kern, dim3((unsigned)mid_grid(tiles)), dim3(128 * WN), lds, stream, p);
     return launch_status("gemm_mid_kernel");
 }

@@ -80,7 +80,7 @@ const char *gemm_tile_unsupported(const GemmProblem &p, int kind, int epi)
 // each kernel has an estimate of its time,
 //     us = start + max(steps * max(step_alone, step_full * fill) + finish * fill, weights * per_mb),
 //     steps: 128-byte steps of K one wave walks, fill: tiles / CUs, weights: MB of right-hand operands,
-// and the smallest one wins (the 256 x 256 kernel unless another is estimated 8 % faster).  With one workgroup to a CU a last,
+// and the smallest one wins (the 256 x 256 kernel unless another is estimated 8 % faster; for it, grouped, with the second launch below).  With one workgroup to a CU a last,
 // partly empty round costs at least half a full one: fill counts as floor(fill) + 0.5 + 0.5 * the rest.  The constants are a fit of
 // this form to the times of all kernels on 1200 problems (dense and grouped, all kinds and layouts, 1 to 16384 rows, K and N from
 // 256 to 8192) in which the choices count, not the times, which are off by 11 to 17 % each: the choices are within 1.5 % of the
@@ -101,6 +101,25 @@ static const PathModel PATH_MODEL[NUM_PATHS] = {
     {STREAM_TM, STREAM_TN, 8, false, 3.7, 1.24, 1.92, 2.0, {0.21, 0.255, 0.46}},
 };
 
+// Whether a grouped problem on 256 x 256 tiles leaves the short row tiles of its last round to a second launch (gemm_tail.h; the device
+// decides which, if any).  Worth it behind one round of long tiles, which the second, mostly empty round would nearly double: MXFP8,
+// 16 groups of 3072 rows in all, K 7168, N 4096 (1.12 to 1.19 rounds) 156-177 -> 150-159 us, 8 of 4096, K 4096 (1.25) 87-91 -> 80-83.  Behind
+// two rounds, or with 2048 of K, the second launch's start and the weights it reads again cost what it saves (84 against 79-87 us; int8 at
+// 2.4 rounds 258 against 254), and SwiGLU weights stored [K, N] reach its narrow tiles in pieces of 32 bytes (int8 at 2.4 rounds 312 against 264).
+static bool may_have_tail(const GemmProblem &p, bool swiglu, double steps, double fill)
+{
+    return p.group_sizes != nullptr && p.num_groups > 1 && !p.tile_kernel_only && fill > 1.0 && fill <= 1.4 && steps >= 32 &&
+           (p.trans_b || (!swiglu && p.N < 1 << 21));
+}
+
+// Average number of tiles to a CU: a group's last row tile is half full on average; groups of a few rows have one tile each.
+static double fill_of(const GemmProblem &p, int tm, int tn_out, int cus)
+{
+    const double groups = std::min<int64_t>(p.num_groups, p.T);   // that can have rows
+    const double row_tiles = p.group_sizes ? std::max<double>(groups, (double)p.T / tm + 0.5 * groups) : (double)((p.T + tm - 1) / tm);
+    return row_tiles * ((p.n_out + tn_out - 1) / tn_out) / cus;
+}
+
 static GemmPath choose_path(const GemmProblem &p, int kind, int epi, int cus)
 {
     const int epb = kind == KIND_F4 ? 2 : 1;
@@ -116,12 +135,13 @@ static GemmPath choose_path(const GemmProblem &p, int kind, int epi, int cus)
     double best_us = 0.0;
     for (int i = 0; i < NUM_PATHS; i++) {
         const PathModel &m = PATH_MODEL[i];
-        // a group's last row tile is half full on average; groups of a few rows have one tile each
-        const double row_tiles = p.group_sizes ? std::max<double>(groups, (double)p.T / m.tm + 0.5 * groups) : (double)((p.T + m.tm - 1) / m.tm);
-        const int tn_out = swiglu ? m.tn / 2 : m.tn;
-        const double fill = row_tiles * ((p.n_out + tn_out - 1) / tn_out) / cus, whole = std::floor(fill);
-        const double rounds = m.rounds && fill > 1.0 && fill > whole ? whole + 0.5 + 0.5 * (fill - whole) : fill;
-        const double us = m.start + std::max(steps / m.waves_k * std::max(m.step_alone, m.step_full * rounds) + m.finish * fill, weights * m.per_mb[layout]);
+        const double fill = fill_of(p, m.tm, swiglu ? m.tn / 2 : m.tn, cus), whole = std::floor(fill);
+        double rounds = m.rounds && fill > 1.0 && fill > whole ? whole + 0.5 + 0.5 * (fill - whole) : fill;
+        // (groups: fill is an average, and a tile too many costs half a round: what that comes to over all fractions)
+        if (i == PATH_MID3 && p.group_sizes && fill > 1.0) rounds = fill + 0.25;
+        double us = m.start + std::max(steps / m.waves_k * std::max(m.step_alone, m.step_full * rounds) + m.finish * fill, weights * m.per_mb[layout]);
+        if (i == PATH_TILE && may_have_tail(p, swiglu, steps, fill))
+            us = std::min(us, m.start + std::max(steps * m.step_full + m.finish * fill, weights * m.per_mb[layout]) + 5.0 + 0.45 * steps);
         if (i == PATH_TILE) {
             best_us = 0.92 * us;
         } else if (us < best_us) {
@@ -139,6 +159,15 @@ static int launch_family(const GemmProblem &p, hipStream_t stream)
     CCH_HIP(hipGetDevice(&dev));
     CCH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     const GemmPath path = choose_path(p, KIND, EPI, cus);
+    constexpr bool SWIGLU = EPI == EPI_DEQUANT_SWIGLU || EPI == EPI_SWIGLU;
+    const int row_bytes = p.K / (KIND == KIND_F4 ? 2 : 1);
+    if (path == PATH_TILE && may_have_tail(p, SWIGLU, (row_bytes + BKB - 1) / BKB, fill_of(p, 256, SWIGLU ? 128 : 256, cus))) {
+        GemmProblem q = p;
+        q.tail_cus = cus;
+        const int rc = p.trans_b ? launch_tile_t<KIND, EPI, FMT, 1>(q, stream) : launch_tile_t<KIND, EPI, FMT, 0>(q, stream);
+        if (rc != CCH_OK) return rc;
+        return p.trans_b ? launch_mid_t<KIND, EPI, FMT, 1>(q, 64, 128, stream) : launch_mid_t<KIND, EPI, FMT, 0>(q, 64, 128, stream);
+    }
     switch (path) {
     case PATH_MID1:
     case PATH_MID2:

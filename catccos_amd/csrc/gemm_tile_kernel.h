@@ -62,7 +62,7 @@
 #pragma once
 #include <atomic>
 
-#include "gemm_device.h"
+#include "gemm_tail.h"
 
 namespace cch {
 
@@ -128,49 +128,32 @@ extern int (*g_prof_copy)(uint64_t *, int);
 #endif
 
 // The group table (row ranges and row-tile prefix sums, gemm_common.h) built by one wave (all 64 lanes of the
-// caller's first wave): lane l holds groups l, 64 + l, 128 + l, 192 + l.  The running row after group g is
-// min(T, sum of the non-negative sizes so far): once the rows are used up every later group is empty, before
-// that nothing is clipped (the reference's golden zero-pads the remainder,
-// examples/utils/gen_data_fp4_mx_alltoallv_gmm.py:788-790).
-__device__ inline void build_group_table_dpp(GroupTable &tab, const int32_t *group_sizes, int num_groups, int T)
+// caller's first wave).  Row tiles that the launch behind this one takes (gemm_tail.h) are left out of the prefix sums.
+template <bool SWIGLU>
+__device__ inline void build_group_table_dpp(GroupTable &tab, const GemmProblem &p)
 {
-    constexpr int NB = MAX_GROUPS / 64;
     const int lane = threadIdx.x & 63;
-    const int nb = (num_groups + 63) >> 6;   // batches of 64 groups in use (wave-uniform)
-    uint32_t sz[NB];
-#pragma unroll
-    for (int b = 0; b < NB; b++) {
-        const int g = b * 64 + lane;
-        sz[b] = 0;
-        if (b < nb && g < num_groups) sz[b] = group_sizes ? (uint32_t)min(max(group_sizes[g], 0), T) : (uint32_t)T;
-    }
-    uint32_t raw_before = 0;   // saturating sum of the sizes of the groups before this batch
+    const GroupRows rows = group_rows(p);
+    const uint32_t tail = p.tail_cus ? tail_key<SWIGLU>(p, rows) : 0u;
     int tile_before = 0;
 #pragma unroll
-    for (int b = 0; b < NB; b++) {
-        if (b < nb) {
+    for (int b = 0; b < GroupRows::NB; b++) {
+        if (b * 64 < p.num_groups) {
             const int g = b * 64 + lane;
-            const uint32_t incl = sat_add(raw_before, wave_scan_sat(sz[b]));
-            const int row_hi = (int)min(incl, (uint32_t)T);
-            // (the exclusive sum is the neighbour's inclusive one: incl - sz would be wrong once the sum has saturated)
-            const uint32_t prev = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x138, 0xF, 0xF, false);   // wave_shr:1
-            const int row_lo = lane == 0 ? (int)min(raw_before, (uint32_t)T) : (int)min(prev, (uint32_t)T);
-            const int tiles = (row_hi - row_lo + BM - 1) / BM;
+            const int tiles = (rows.hi[b] - rows.lo[b] + BM - 1) / BM - (in_tail(rows, b, tail) ? 1 : 0);
             const int tincl = (int)wave_scan_sat((uint32_t)tiles);
-            if (g < num_groups) {
-                tab.row_start[g] = row_lo;
+            if (g < p.num_groups) {
+                tab.row_start[g] = rows.lo[b];
                 tab.tile_start[g] = tile_before + tincl - tiles;
             }
-            raw_before = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
             tile_before += __builtin_amdgcn_readlane(tincl, 63);
         }
     }
     if (lane == 0) {
-        const int row = (int)min(raw_before, (uint32_t)T);
-        tab.row_start[num_groups] = row;   // pseudo group: rows that belong to no expert
-        tab.tile_start[num_groups] = tile_before;
-        tab.row_start[num_groups + 1] = T;
-        tab.tile_start[num_groups + 1] = tile_before + (T - row + BM - 1) / BM;
+        tab.row_start[p.num_groups] = rows.used;   // pseudo group: rows that belong to no expert
+        tab.tile_start[p.num_groups] = tile_before;
+        tab.row_start[p.num_groups + 1] = p.T;
+        tab.tile_start[p.num_groups + 1] = tile_before + (p.T - rows.used + BM - 1) / BM;
     }
 }
 
@@ -238,7 +221,7 @@ __global__ __launch_bounds__(TILE_THREADS) void gemm_tile_kernel(GemmProblem p)
             tab.tile_start[0] = 0; tab.tile_start[1] = tiles; tab.tile_start[2] = tiles;
         }
     } else if (threadIdx.x < 64) {
-        build_group_table_dpp(tab, p.group_sizes, p.num_groups, p.T);
+        build_group_table_dpp<SWIGLU>(tab, p);
     }
     __syncthreads();
 
