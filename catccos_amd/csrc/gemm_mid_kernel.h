@@ -37,7 +37,9 @@ __global__ __launch_bounds__(128 * WN, 2) void gemm_mid_kernel(GemmProblem p)
     constexpr bool DEQ = EPI == EPI_DEQUANT || EPI == EPI_DEQUANT_SWIGLU;
     constexpr int EPB = KT::ELEMS_PER_BYTE;
     constexpr int NW = 2 * WN, TM = 64 * MB, TN = 64 * WN;
-    constexpr int TN_OUT = SWIGLU ? TN / 2 : TN;   // SwiGLU: blocks of 32 gate columns and their 32 up columns alternate
+    constexpr int TN_OUT = SWIGLU ? TN / 2 : TN;   // SwiGLU: the tile's gate columns, then their up columns
+    // A wave's 32-column blocks of the panel start WC * wn columns in and lie JC apart (SwiGLU: one gate, one up).
+    constexpr int WC = SWIGLU ? 32 : 64, JC = SWIGLU ? TN / 2 : 32;
     constexpr int S = mid_stages(MB, WN);                  // stages of the ring
     constexpr int A_BYTES = TM * BKB, STAGE = mid_stage_bytes(MB, WN);
     constexpr int SC_OFF = S * STAGE, SC_BUF = (TM + TN) * 16;   // MX scales: buffers of 16 bytes per row and column
@@ -105,8 +107,10 @@ __global__ __launch_bounds__(128 * WN, 2) void gemm_mid_kernel(GemmProblem p)
     // which for an odd request is the even request's chunk ^ 4.
     const uint32_t kc0 = (uint32_t)(((lane & 7) ^ (lane >> 4)) << 4), kc1 = kc0 ^ 64u;   // (a wave's first row is a multiple of 16)
     const uint32_t a_lane = (uint32_t)(wave * NA * 8 + (lane >> 3)) * (uint32_t)pa;
-    // tile column c -> column of B: with SwiGLU blocks of 32 gate columns and their 32 up columns alternate
-    auto col_of = [&](int c) { return j0 + (SWIGLU ? ((c >> 5) & 1) * p.n_out + (c >> 6) * 32 + (c & 31) : c); };
+    // tile column c -> column of B.  SwiGLU: as long a piece of a row of [K, N] weights as there is on either side (64 or 128 bytes;
+    // with gate and up blocks of 32 alternating, MXFP8 3072 x 7168 x 4096 over 16 groups took 163 us on 128 x 256 tiles and 215 on
+    // 128 x 128, so 158 and 208; 384 rows on 64 x 128 tiles 129, so 125)
+    auto col_of = [&](int c) { return j0 + (SWIGLU ? c / JC * p.n_out + c % JC : c); };
     uint32_t b_lane, b_odd = 0;   // [K, N]: of the even and the odd requests
     if constexpr (TB) {
         b_lane = (uint32_t)(col_of(wave * NBQ * 8) + (lane >> 3)) * (uint32_t)lda;
@@ -207,18 +211,18 @@ __global__ __launch_bounds__(128 * WN, 2) void gemm_mid_kernel(GemmProblem p)
     for (int x = 0; x < 4; x++) {
         const uint32_t at = (uint32_t)r * BKB + ((((uint32_t)((x >> 1) * 4 + (x & 1) * 2 + g)) ^ swizzle_of_row(r)) << 4);
         fr_a[x] = lds_base + (uint32_t)(wm * 32 * MB) * BKB + at;
-        fr_b[x] = lds_base + (uint32_t)A_BYTES + (uint32_t)(wn * 64) * BKB + at;
+        fr_b[x] = lds_base + (uint32_t)A_BYTES + (uint32_t)(wn * WC) * BKB + at;
     }
     {
         const int q = lane >> 4, i = lane & 15;
-        // fp8 / int8: lane addresses K-row 16*(q/2) + i/2, chunk wn*4 + j*2 + (q & 1), half i & 1; FP4: K-row 32*(q/2) + i, chunk
-        // wn*2 + j, half q & 1 (the rows of the further reads are multiples of 8 or 16 away: the same row bits)
-        const int row = EPB == 2 ? 32 * (q >> 1) + i : 16 * (q >> 1) + (i >> 1), chunk = EPB == 2 ? wn * 2 : wn * 4 + (q & 1);
+        // (column blocks start at multiples of 32 columns) fp8 / int8: lane addresses K-row 16*(q/2) + i/2, chunk q & 1 of the block, half
+        // i & 1; FP4: K-row 32*(q/2) + i, half q & 1 (the rows of the further reads are multiples of 8 or 16 away: the same row bits)
+        const int row = EPB == 2 ? 32 * (q >> 1) + i : 16 * (q >> 1) + (i >> 1), chunk = wn * WC / (16 * EPB) + (EPB == 2 ? 0 : q & 1);
         const uint32_t at = (uint32_t)row * (CPR * 16u) + (uint32_t)(chunk ^ b_swizzle(row)) * 16u + (uint32_t)(EPB == 2 ? q & 1 : i & 1) * 8u;
 #pragma unroll
-        for (int j = 0; j < 2; j++) fbt[j] = lds_base + (uint32_t)A_BYTES + (at ^ ((uint32_t)j << (EPB == 2 ? 4 : 5)));
+        for (int j = 0; j < 2; j++) fbt[j] = lds_base + (uint32_t)A_BYTES + (at ^ (uint32_t)(j * (JC / EPB)));   // (that bit of the chunk is free)
     }
-    const uint32_t rd_sa = (uint32_t)(SC_OFF + (wm * 32 * MB + r) * 16), rd_sb = (uint32_t)(SC_OFF + TM * 16) + (TB ? (uint32_t)(wn * 64 + r) * 16u : (uint32_t)(wn * 64 + r) * 2u);
+    const uint32_t rd_sa = (uint32_t)(SC_OFF + (wm * 32 * MB + r) * 16), rd_sb = (uint32_t)(SC_OFF + TM * 16) + (uint32_t)(wn * WC + r) * (TB ? 16u : 2u);
     const uint32_t ph_a = UA ? ((uint32_t)(m0 + r) * (uint32_t)psa) & 3u : 0u;
     const uint32_t ph_b = UA ? ((uint32_t)(j0 + r) * (uint32_t)p.sld) & 3u : 0u;   // (the other terms are multiples of four rows)
     const int nblk = (p.K + 31) >> 5;
@@ -247,10 +251,10 @@ __global__ __launch_bounds__(128 * WN, 2) void gemm_mid_kernel(GemmProblem p)
 #pragma unroll
                 for (int j = 0; j < 2; j++) {
                     if constexpr (!TB) {
-                        const uint32_t at = rd_sb + buf + (uint32_t)((ws * NSP + d) * 4 * TN) + (uint32_t)(j * 64 + g);
+                        const uint32_t at = rd_sb + buf + (uint32_t)((ws * NSP + d) * 4 * TN) + (uint32_t)(j * JC * 2 + g);
                         sc[d][MB + j] = (uint32_t)smem[at] | (uint32_t)smem[at + 2u * TN] << 16;
                     } else {
-                        const uint32_t at = rd_sb + buf + (uint32_t)((ws * NSP + d) * 4) + j * 512u;
+                        const uint32_t at = rd_sb + buf + (uint32_t)((ws * NSP + d) * 4 + j * JC * 16);
                         if constexpr (UA) sc[d][MB + j] = (uint32_t)smem[at + ph_b + g] | (uint32_t)smem[at + ph_b + g + 2] << 16;
                         else sc[d][MB + j] = *reinterpret_cast<const uint32_t *>(smem + at);
                     }
@@ -268,7 +272,7 @@ __global__ __launch_bounds__(128 * WN, 2) void gemm_mid_kernel(GemmProblem p)
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             if constexpr (TB) {
-                const v4i l = lds_read16_abs(fr_b[2 * ks] + (uint32_t)(STG * STAGE + j * 4096)), h = lds_read16_abs(fr_b[2 * ks + 1] + (uint32_t)(STG * STAGE + j * 4096));
+                const v4i l = lds_read16_abs(fr_b[2 * ks] + (uint32_t)(STG * STAGE + j * JC * BKB)), h = lds_read16_abs(fr_b[2 * ks + 1] + (uint32_t)(STG * STAGE + j * JC * BKB));
                 fb[j][ks] = (v8i){l[0], l[1], l[2], l[3], h[0], h[1], h[2], h[3]};
             } else {
                 typedef __attribute__((address_space(3))) v2i *LdsV2;
