@@ -140,8 +140,11 @@ static GemmPath choose_path(const GemmProblem &p, int kind, int epi, int cus)
         // (groups: fill is an average, and a tile too many costs half a round: what that comes to over all fractions)
         if (i == PATH_MID3 && p.group_sizes && fill > 1.0) rounds = fill + 0.25;
         double us = m.start + std::max(steps / m.waves_k * std::max(m.step_alone, m.step_full * rounds) + m.finish * fill, weights * m.per_mb[layout]);
+        // (Every CU is busy then, and weights of either layout arrive at the better rate: 470 MB as [N, K] within the 120 us of one full
+        // round.  At the table's 0.30 such problems went to 128 x 256 tiles: 3072 rows over 16 groups, K 7168, N 4096, of 192 rows each
+        // 183 us, slightly skewed 193; now 138 and 152.)
         if (i == PATH_TILE && may_have_tail(p, swiglu, steps, fill))
-            us = std::min(us, m.start + std::max(steps * m.step_full + m.finish * fill, weights * m.per_mb[layout]) + 5.0 + 0.45 * steps);
+            us = std::min(us, m.start + std::max(steps * m.step_full + m.finish * fill, weights * 0.20) + 5.0 + 0.45 * steps);
         if (i == PATH_TILE) {
             best_us = 0.92 * us;
         } else if (us < best_us) {
