@@ -8,6 +8,7 @@ The entry points of a serving program's inner loop first offer the call to their
 takes plain contiguous GPU tensors of the right types and shapes and answers NotImplemented to everything else.
 """
 import importlib as _importlib
+import warnings as _warnings
 
 import torch
 
@@ -45,16 +46,22 @@ def _ptr(t):
 
 
 class _Direct:
-    """The native forms, loaded with the first call (like the library, whose absence is an error too)."""
+    """The native forms, loaded with the first call.  The module is built for one interpreter and one PyTorch; where it is missing
+    or does not load, a warning says so once and every call takes the general path, which needs the HIP library alone."""
 
     def __getattr__(self, name):
+        names = ("mx_quant", "dynamic_quant_i8", "moe_init_routing", "w8a8_matmul_dequant", "gmm_i8", "mx_matmul", "mx_grouped_matmul", "moe_ffn_mxfp8")
+        if name not in names:
+            raise AttributeError(name)
         try:
             mod = _importlib.import_module("._direct", __package__)
         except ImportError as e:
-            raise FileNotFoundError("catccos_amd/_direct.so is missing or does not load (build it with `python -m catccos_amd.build`): %s" % e) from e
-        for f in ("mx_quant", "dynamic_quant_i8", "moe_init_routing", "w8a8_matmul_dequant", "gmm_i8", "mx_matmul", "mx_grouped_matmul", "moe_ffn_mxfp8"):
-            setattr(self, f, getattr(mod, f))
-        return getattr(mod, name)
+            _warnings.warn("catccos_amd/_direct.so is missing or does not load, calls cost several times the host time "
+                           "(build it with `python -m catccos_amd.build`): %s" % e, RuntimeWarning, stacklevel=3)
+            mod = None
+        for f in names:
+            setattr(self, f, getattr(mod, f) if mod else lambda *a: NotImplemented)
+        return getattr(self, name)
 
 
 _direct = _Direct()

@@ -26,6 +26,32 @@ def test_host_tensors_and_odd_arguments_are_declined():
         cc.mx_quant(x)
 
 
+def _without_module(monkeypatch):
+    def fails(name, package=None):
+        raise ImportError("libtorch_python.so: cannot open shared object file")
+    monkeypatch.setattr(ops._importlib, "import_module", fails)
+    monkeypatch.setattr(ops, "_direct", ops._Direct())
+
+
+def test_host_tensors_are_refused_as_such_without_the_native_module(monkeypatch):
+    _without_module(monkeypatch)
+    with pytest.warns(RuntimeWarning, match="does not load"):
+        with pytest.raises(ValueError, match="GPU tensors only"):
+            cc.mx_quant(torch.zeros(2, 64, dtype=torch.bfloat16))
+
+
+@pytest.mark.gpu
+def test_calls_are_served_without_the_native_module(monkeypatch):
+    calls = _calls()
+    want = [_flat(f(*a, **kw)) for f, a, kw in calls]
+    _without_module(monkeypatch)
+    with pytest.warns(RuntimeWarning, match="does not load"):
+        got = [_flat(f(*a, **kw)) for f, a, kw in calls]
+    for w, g in zip(want, got):
+        for x, y in zip(w, g):
+            assert torch.equal(x.view(torch.uint8), y.view(torch.uint8))
+
+
 def _calls(dev="cuda"):
     g = torch.Generator(device=dev)
     g.manual_seed(1)
