@@ -15,6 +15,7 @@ extern std::atomic<int> g_route_three_launches;        // routing.hip
 static std::atomic<int> g_force_generic{0};
 static std::atomic<int> g_require_tiled{0};
 static std::atomic<int> g_tile_order{-1};   // -1: chosen per problem
+static std::atomic<int> g_kernel{-1};      // -1: chosen per problem
 static std::atomic<int> g_nt_out{-1};      // -1: chosen per problem
 static std::atomic<int> g_i8_fp16_step{0};
 
@@ -26,7 +27,7 @@ static int run(const GemmProblem &prob, int kind, int epi, hipStream_t stream)
     GemmProblem p = prob;
     const int order = g_tile_order.load();
     p.tile_order = order >= 0 ? order : 2;
-    p.tile_kernel_only = order >= 0;
+    p.kernel = order >= 0 ? (int)PATH_TILE : g_kernel.load();
     p.i8_fp16_step = g_i8_fp16_step.load() != 0;
     const int nto = g_nt_out.load();
     p.nt_out = nto >= 0 ? nto : (kind == KIND_F4);
@@ -81,6 +82,11 @@ int cch_set_option(const char *name, int value)
     }
     if (strcmp(name, "gemm_tile_order") == 0) {
         g_tile_order.store(value);
+        return CCH_OK;
+    }
+    if (strcmp(name, "gemm_kernel") == 0) {
+        CCH_REQUIRE(value >= -1 && value < NUM_PATHS, "cch_set_option: gemm_kernel %d outside -1..%d", value, NUM_PATHS - 1);
+        g_kernel.store(value);
         return CCH_OK;
     }
     if (strcmp(name, "routing_three_launches") == 0) {

@@ -15,6 +15,11 @@ enum GemmKind { KIND_I8 = 0, KIND_F8 = 1, KIND_F4 = 2 };
 // (include/catccos/epilogue/block/block_epilogue_regbase_swiglu.hpp:38-80)
 enum GemmEpilogue { EPI_PLAIN = 0, EPI_DEQUANT = 1, EPI_DEQUANT_SWIGLU = 2, EPI_SWIGLU = 3 };
 
+// The tiled MFMA kernels, numbered as the switch "gemm_kernel" names them: 256 x 256 tiles (gemm_tile_kernel.h), 64 x 128, 128 x 128 and
+// 128 x 256 tiles (gemm_mid_kernel.h), tiles of 32 x 64 whose 4 or 8 waves split K (gemm_stream_kernel.h), and 256 x 256 tiles with
+// a second launch of 64 x 128 ones for a grouped problem's last round (gemm_tail.h).
+enum GemmPath { PATH_TILE, PATH_MID1, PATH_MID2, PATH_MID3, PATH_STREAM4, PATH_STREAM8, NUM_KERNELS, PATH_TILE_TAIL = NUM_KERNELS, NUM_PATHS };
+
 constexpr int MAX_GROUPS = 256;
 constexpr int TAIL_TILES = 512;   // most tiles that the second launch of a grouped problem may have (gemm_tail.h): one round of its kernel
 
@@ -56,7 +61,7 @@ struct GemmProblem {
     int tail_cus;            // grouped problems, 256 x 256 kernel: CUs, if a second launch takes the last rows of some groups
                              // (gemm_tail.h); 0: it takes them all itself
     int nt_out;              // tiled kernels: output stores carry the non-temporal hint
-    int tile_kernel_only;    // an order of its tiles was asked for: the 256 x 256 kernel, whatever the size
+    int kernel;              // which kernel was asked for (GemmPath; tiled kernels only), -1: chosen per problem
     int tile_order;          // tiled kernels: 0 = row-major over (row tile, column tile); 1 = runs of consecutive tiles per XCD;
                              // 2 = a block of 4 row tiles x 8 column tiles per XCD where the shape allows (else 1 for groups, 0 without)
 };

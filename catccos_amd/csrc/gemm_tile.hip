@@ -85,14 +85,13 @@ const char *gemm_tile_unsupported(const GemmProblem &p, int kind, int epi)
 // this form to the times of all kernels on 1200 problems (dense and grouped, all kinds and layouts, 1 to 16384 rows, K and N from
 // 256 to 8192) in which the choices count, not the times, which are off by 11 to 17 % each: the choices are within 1.5 % of the
 // best ones in the geometric mean, and 1.83 times faster than the 256 x 256 kernel on all of them (dense 2.1, grouped 1.6).
-enum GemmPath { PATH_TILE, PATH_MID1, PATH_MID2, PATH_MID3, PATH_STREAM4, PATH_STREAM8, NUM_PATHS };
 struct PathModel {
     int tm, tn, waves_k;    // rows and columns of B per tile, waves that share a tile's K
     bool rounds;            // one workgroup per CU
     double start, step_alone, step_full, finish;
     double per_mb[3];       // B as [N, K], as [K, N], and as [K, N] with gate and up columns apart (narrower pieces of a row)
 };
-static const PathModel PATH_MODEL[NUM_PATHS] = {
+static const PathModel PATH_MODEL[NUM_KERNELS] = {
     {256, 256, 1, true, 9.7, 1.27, 1.66, 3.9, {0.30, 0.20, 0.21}},
     {64, 128, 1, false, 4.5, 0.37, 0.50, 1.55, {0.18, 0.22, 0.22}},
     {128, 128, 1, false, 5.75, 0.48, 0.65, 1.55, {0.19, 0.22, 0.27}},
@@ -108,7 +107,7 @@ static const PathModel PATH_MODEL[NUM_PATHS] = {
 // 2.4 rounds 258 against 254), and SwiGLU weights stored [K, N] reach its narrow tiles in pieces of 32 bytes (int8 at 2.4 rounds 312 against 264).
 static bool may_have_tail(const GemmProblem &p, bool swiglu, double steps, double fill)
 {
-    return p.group_sizes != nullptr && p.num_groups > 1 && !p.tile_kernel_only && fill > 1.0 && fill <= 1.4 && steps >= 32 &&
+    return p.group_sizes != nullptr && p.num_groups > 1 && fill > 1.0 && fill <= 1.4 && steps >= 32 &&
            (p.trans_b || (!swiglu && p.N < 1 << 21));
 }
 
@@ -120,20 +119,33 @@ static double fill_of(const GemmProblem &p, int tm, int tn_out, int cus)
     return row_tiles * ((p.n_out + tn_out - 1) / tn_out) / cus;
 }
 
+// Scale rows of A or B that can start 2 bytes past a dword: the mid-size kernels' UA form.
+static bool scales_off_dwords(const GemmProblem &p, int kind) { return kind != KIND_I8 && ((p.sld & 3) != 0 || (p.sa_pitch & 3) != 0); }
+
+// nullptr where kernel `path` can take a problem that gemm_tile_unsupported() has let pass.
+static const char *path_refuses(const GemmProblem &p, int kind, int path)
+{
+    if (path == PATH_TILE) return nullptr;
+    // the smaller kernels add up to 512 K-rows of a [K, N] operand to offsets below 2^31
+    if (!p.trans_b && p.N / (kind == KIND_F4 ? 2 : 1) >= 1 << 21) return "rows of a [K,N] operand of 2 MiB or more";
+    if (path == PATH_TILE_TAIL && p.group_sizes == nullptr) return "only grouped problems have a second launch";
+    if (path == PATH_MID3 && kind == KIND_F4 && scales_off_dwords(p, kind)) return "no LDS left for MXFP4 scale rows off 4-byte boundaries";
+    return nullptr;
+}
+
 static GemmPath choose_path(const GemmProblem &p, int kind, int epi, int cus)
 {
     const int epb = kind == KIND_F4 ? 2 : 1;
     const bool swiglu = epi == EPI_DEQUANT_SWIGLU || epi == EPI_SWIGLU;
-    if (p.tile_kernel_only) return PATH_TILE;
-    // the smaller kernels add up to 512 K-rows of a [K, N] operand to offsets below 2^31
-    if (!p.trans_b && p.N / epb >= 1 << 21) return PATH_TILE;
     const double steps = (p.K / epb + BKB - 1) / BKB;
     const double groups = std::min<int64_t>(p.num_groups, p.T);   // that can have rows
     const double weights = groups * (double)p.N * (p.K / epb) * 1e-6;
     const int layout = p.trans_b ? 0 : swiglu ? 2 : 1;
-    GemmPath best = PATH_TILE;
+    const bool tail = may_have_tail(p, swiglu, steps, fill_of(p, 256, swiglu ? 128 : 256, cus));
+    GemmPath best = tail ? PATH_TILE_TAIL : PATH_TILE;
+    if (path_refuses(p, kind, PATH_STREAM4)) return PATH_TILE;
     double best_us = 0.0;
-    for (int i = 0; i < NUM_PATHS; i++) {
+    for (int i = 0; i < NUM_KERNELS; i++) {
         const PathModel &m = PATH_MODEL[i];
         const double fill = fill_of(p, m.tm, swiglu ? m.tn / 2 : m.tn, cus), whole = std::floor(fill);
         double rounds = m.rounds && fill > 1.0 && fill > whole ? whole + 0.5 + 0.5 * (fill - whole) : fill;
@@ -143,7 +155,7 @@ static GemmPath choose_path(const GemmProblem &p, int kind, int epi, int cus)
         // (Every CU is busy then, and weights of either layout arrive at the better rate: 470 MB as [N, K] within the 120 us of one full
         // round.  At the table's 0.30 such problems went to 128 x 256 tiles: 3072 rows over 16 groups, K 7168, N 4096, of 192 rows each
         // 183 us, slightly skewed 193; now 138 and 152.)
-        if (i == PATH_TILE && may_have_tail(p, swiglu, steps, fill))
+        if (i == PATH_TILE && tail)
             us = std::min(us, m.start + std::max(steps * m.step_full + m.finish * fill, weights * 0.20) + 5.0 + 0.45 * steps);
         if (i == PATH_TILE) {
             best_us = 0.92 * us;
@@ -152,7 +164,7 @@ static GemmPath choose_path(const GemmProblem &p, int kind, int epi, int cus)
             best_us = us;
         }
     }
-    return best;
+    return path_refuses(p, kind, best) ? PATH_MID2 : best;   // (128 x 256 tiles: the other ones with 128 rows)
 }
 
 template <int KIND, int EPI, int FMT>
@@ -161,17 +173,19 @@ static int launch_family(const GemmProblem &p, hipStream_t stream)
     int dev = 0, cus = 0;
     CCH_HIP(hipGetDevice(&dev));
     CCH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const GemmPath path = choose_path(p, KIND, EPI, cus);
-    constexpr bool SWIGLU = EPI == EPI_DEQUANT_SWIGLU || EPI == EPI_SWIGLU;
-    const int row_bytes = p.K / (KIND == KIND_F4 ? 2 : 1);
-    if (path == PATH_TILE && may_have_tail(p, SWIGLU, (row_bytes + BKB - 1) / BKB, fill_of(p, 256, SWIGLU ? 128 : 256, cus))) {
+    if (p.kernel >= 0) {
+        const char *why = path_refuses(p, KIND, p.kernel);
+        if (why) return fail(CCH_ENOSUP, "gemm_kernel %d does not take this problem (T=%d N=%d K=%d trans_b=%d: %s)", p.kernel, p.T, p.N, p.K, p.trans_b, why);
+    }
+    const GemmPath path = p.kernel >= 0 ? (GemmPath)p.kernel : choose_path(p, KIND, EPI, cus);
+    switch (path) {
+    case PATH_TILE_TAIL: {
         GemmProblem q = p;
         q.tail_cus = cus;
         const int rc = p.trans_b ? launch_tile_t<KIND, EPI, FMT, 1>(q, stream) : launch_tile_t<KIND, EPI, FMT, 0>(q, stream);
         if (rc != CCH_OK) return rc;
         return p.trans_b ? launch_mid_t<KIND, EPI, FMT, 1>(q, 64, 128, stream) : launch_mid_t<KIND, EPI, FMT, 0>(q, 64, 128, stream);
     }
-    switch (path) {
     case PATH_MID1:
     case PATH_MID2:
     case PATH_MID3: {
@@ -201,3 +215,25 @@ int launch_gemm_tile(const GemmProblem &p, int kind, int epi, hipStream_t stream
 }
 
 }  // namespace cch
+
+extern "C" int cch_gemm_kernel_for(int fmt, int swiglu, int64_t num_experts, int64_t t, int64_t n, int64_t k, int trans_b, int cus)
+{
+    using namespace cch;
+    if (t < 1 || n < 1 || k < 1 || t >> 31 || n >> 31 || k >> 31 || num_experts < 0 || num_experts > MAX_GROUPS || cus < 1 || (swiglu && n % 2)) return -1;
+    static const int32_t some_sizes = 0;
+    alignas(16) static const uint8_t some_bytes[16] = {};
+    const int kind = fmt < 0 ? KIND_I8 : fmt == CCH_FMT_E2M1 ? KIND_F4 : KIND_F8, epi = kind == KIND_I8 ? (swiglu ? EPI_DEQUANT_SWIGLU : EPI_DEQUANT) : (swiglu ? EPI_SWIGLU : EPI_PLAIN);
+    GemmProblem p{};
+    p.a = p.b = p.sa = p.sb = some_bytes;
+    p.group_sizes = num_experts > 0 ? &some_sizes : nullptr;
+    p.num_groups = num_experts > 0 ? (int)num_experts : 1;
+    p.T = (int)t;
+    p.N = (int)n;
+    p.n_out = (int)(swiglu ? n / 2 : n);
+    p.K = (int)k;
+    p.trans_b = trans_b;
+    p.sld = kind == KIND_I8 ? 0 : (int)(2 * ((k + 63) / 64));
+    p.b_stride = n * k / (kind == KIND_F4 ? 2 : 1);
+    p.sb_stride = n * p.sld;
+    return gemm_tile_unsupported(p, kind, epi) ? -1 : (int)choose_path(p, kind, epi, cus);
+}

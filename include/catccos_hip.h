@@ -341,6 +341,8 @@ int cch_dyn_quant_i8_rows_smooth(const void *x, const int32_t *src_rows, const f
  * 4 row tiles x 8 column tiles of every round (where 8, 16, 32 or 64 column tiles and 256 workgroups
  * allow it; else 1 for grouped problems and 0 for dense ones), -1 (default) = 2; an order set here also keeps problems of every
  * size on those kernels (by default the ones too small for 256 x 256 tiles go to kernels with smaller tiles);
+ * "gemm_kernel" = 0..6 asks for one of the tiled MFMA kernels (CCH_GEMM_KERNEL_*) whatever the size, -1 (default) chooses per
+ * problem: a GEMM entry point returns CCH_ENOSUP where that kernel does not take the problem ("gemm_tile_order" goes first);
  * "i8_epilogue_fp16_step" = 1 makes the int8 epilogues (cch_gemm_i8_dequant*, cch_gmm_i8_dequant*, both kernel paths)
  * round acc * per_channel to IEEE half before the per-token factor, as the reference's device kernel does
  * (include/catccos/epilogue/block/block_epilogue_per_token_dequant_swiglu.hpp:348-361: the matrix unit's output stage
@@ -360,6 +362,20 @@ int cch_dyn_quant_i8_rows_smooth(const void *x, const int32_t *src_rows, const f
  * GEMM entry point empties the calling thread's message when it starts, so after CCH_OK the message is
  * either that note of this very call or empty. */
 int cch_set_option(const char *name, int value);
+
+/* Tiled MFMA kernels: persistent workgroups on 256 x 256 tiles; tiles of 64 x 128, 128 x 128 and 128 x 256; tiles of 32 x 64 whose
+ * 4 or 8 waves split K; 256 x 256 tiles whose mostly empty last round (grouped problems) is a second launch of 64 x 128 ones. */
+#define CCH_GEMM_KERNEL_256X256 0
+#define CCH_GEMM_KERNEL_64X128 1
+#define CCH_GEMM_KERNEL_128X128 2
+#define CCH_GEMM_KERNEL_128X256 3
+#define CCH_GEMM_KERNEL_STREAM4 4
+#define CCH_GEMM_KERNEL_STREAM8 5
+#define CCH_GEMM_KERNEL_256X256_TAIL 6
+/* The kernel that a GEMM entry point chooses for aligned operands on a GPU of `cus` CUs, or -1 (the generic kernels, or no
+ * problem at all).  fmt: CCH_FMT_E4M3, CCH_FMT_E5M2, CCH_FMT_E2M1, or -1 for int8; num_experts 0: a dense problem; n: columns of B
+ * (gate and up halves together).  Host code only, no GPU needed. */
+int cch_gemm_kernel_for(int fmt, int swiglu, int64_t num_experts, int64_t t, int64_t n, int64_t k, int trans_b, int cus);
 
 #ifdef __cplusplus
 }

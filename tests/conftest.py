@@ -12,6 +12,15 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu on the GPU box)")
 
 
+@pytest.fixture(params=[-1, 0], ids=["chosen", "256x256"])
+def kernel(request):
+    """The tiled GEMM kernel that a problem goes to by itself (at most tests' sizes one of the smaller tiles), and the 256 x 256 one."""
+    import catccos_amd as cc
+    cc.set_option("gemm_kernel", request.param)
+    yield request.param
+    cc.set_option("gemm_kernel", -1)
+
+
 def _has_gpu():
     try:
         import torch

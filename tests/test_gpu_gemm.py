@@ -68,10 +68,13 @@ def zipf_groups(rng, t, e, empty=True):
     return gs
 
 
-@pytest.fixture(params=[0, 1], ids=["tiled", "generic"])
+@pytest.fixture(params=[(0, -1), (0, 0), (1, -1)], ids=["tiled", "tiled-256x256", "generic"])
 def path(request):
-    cc.set_option("force_generic_gemm", request.param)
-    yield request.param
+    generic, kernel = request.param
+    cc.set_option("force_generic_gemm", generic)
+    cc.set_option("gemm_kernel", kernel)
+    yield generic
+    cc.set_option("gemm_kernel", -1)
     cc.set_option("force_generic_gemm", 0)
 
 
@@ -121,7 +124,7 @@ def test_gmm_swiglu(cfg, trans_b, path):
 
 @pytest.mark.parametrize("tiled", [True, False], ids=["tiled", "generic"])
 @pytest.mark.parametrize("trans_b", [0, 1])
-def test_int8_epilogues_with_the_reference_devices_fp16_step(tiled, trans_b):
+def test_int8_epilogues_with_the_reference_devices_fp16_step(tiled, trans_b, kernel):
     """`i8_epilogue_fp16_step`: acc * per_channel leaves the matrix stage as IEEE half and the per-token factor meets the
     widened half, as the reference's device kernel does it
     (include/catccos/epilogue/block/block_epilogue_per_token_dequant_swiglu.hpp:348-361; the golden generator's option,
@@ -207,7 +210,7 @@ def _reference_shapes(op, limit=4e10):
 
 
 @pytest.mark.parametrize("shape", _reference_shapes("ascend950_mxfp8_matmul_reduce_scatter"))
-def test_mx_gemm_reference_shape_list(shape):
+def test_mx_gemm_reference_shape_list(shape, kernel):
     """Every (M, K, N) of the reference's own list for the MXFP8 operator
     (examples/ascend950_mxfp8_matmul_reduce_scatter/scripts/test_shapes.csv, kept as the fixture
     golden/reference_shapes.json), in the layout its run uses (transB = 1)."""
@@ -222,7 +225,7 @@ def test_mx_gemm_reference_shape_list(shape):
 
 @pytest.mark.parametrize("op,fmt", [("ascend950_fp8_mx_grouped_matmul_alltoallv", "e4m3"), ("ascend950_fp4_mx_grouped_matmul_alltoallv", "e2m1"),
                                     ("ascend950_fp8_mx_alltoallv_grouped_matmul", "e4m3"), ("ascend950_fp4_mx_alltoallv_grouped_matmul", "e2m1")])
-def test_mx_gmm_reference_shape_lists(op, fmt):
+def test_mx_gmm_reference_shape_lists(op, fmt, kernel):
     """The grouped operators' own shapes (their scripts/test_shapes.csv), 8 experts as their run.sh defaults to."""
     for (m, k, n) in _reference_shapes(op):
         e = 8
@@ -237,7 +240,7 @@ def test_mx_gmm_reference_shape_lists(op, fmt):
         assert_close(got, want, (op, m, k, n))
 
 
-def test_mx_gemm_scale_extremes():
+def test_mx_gemm_scale_extremes(kernel):
     """Scale bytes far from 127 on both operands, incl. products that leave the fp32 normal range."""
     rng = np.random.default_rng(5)
     m, n, k = 64, 64, 256
@@ -285,7 +288,7 @@ def test_mx_gmm(fmt, cfg, trans_b, path):
 # layouts of B, empty and one-row groups.
 
 @pytest.fixture
-def tiled_only():
+def tiled_only(kernel):
     cc.set_option("force_generic_gemm", 0)
     cc.set_option("require_tiled_gemm", 1)
     yield
@@ -388,7 +391,7 @@ def test_mx_gmm_tiled(fmt, cfg, trans_b, tiled_only):
     assert_close(got, want, ("mx gmm tiled", fmt, cfg[:4], trans_b))
 
 
-def test_mx_gmm_mapped_fp16_is_the_rounded_accumulator():
+def test_mx_gmm_mapped_fp16_is_the_rounded_accumulator(kernel):
     """The half-precision output is the same fp32 result rounded to nearest even: on data whose
     results are exact in both types (small integers) the two outputs agree exactly, and on random
     data the fp16 output is closer to the oracle than bf16's 8 bits allow."""
@@ -425,7 +428,7 @@ def test_mx_gmm_mapped_fp16_is_the_rounded_accumulator():
 @pytest.mark.parametrize("fmt", ["e4m3", "e2m1"])
 @pytest.mark.parametrize("trans_b", [0, 1])
 @pytest.mark.parametrize("tiled", [True, False])
-def test_mx_gmm_mapped_rows(fmt, trans_b, tiled):
+def test_mx_gmm_mapped_rows(fmt, trans_b, tiled, kernel):
     """Down-projection form: result rows leave in send-buffer order (by destination rank, then
     expert); dropped rows and rows of no group are not written."""
     ranks, e, k, n = 3, 5, 1024, 416
@@ -481,7 +484,7 @@ def _both_paths(fn):
 
 
 @pytest.mark.parametrize("seed", range(96))
-def test_tiled_matches_generic_on_random_groups(seed):
+def test_tiled_matches_generic_on_random_groups(seed, kernel):
     """Random expert counts, group sizes (empty, one-row, many-tile groups, rows of no group), K-step
     counts, widths and both weight layouts: the tiled kernels against the one-thread-per-output
     kernels on the device.  Both accumulate the same products in fp32 (int32 for int8), so they may
@@ -522,7 +525,7 @@ def test_tiled_matches_generic_on_random_groups(seed):
 
 @pytest.mark.parametrize("trans_b", [0, 1])
 @pytest.mark.parametrize("tiled", [True, False])
-def test_gmm_i8_dequant_without_activation(trans_b, tiled):
+def test_gmm_i8_dequant_without_activation(trans_b, tiled, kernel):
     """Grouped int8 matmul + per-token x per-channel dequant: every group is the dense golden of its rows."""
     e, t, k, n = 5, 900, 512, 384
     rng = np.random.default_rng(31 + trans_b)
@@ -552,7 +555,7 @@ def test_gmm_i8_dequant_without_activation(trans_b, tiled):
 
 @pytest.mark.parametrize("fmt", ["e4m3", "e2m1"])
 @pytest.mark.parametrize("tiled", [True, False])
-def test_mx_gmm_half_output_without_a_row_map(fmt, tiled):
+def test_mx_gmm_half_output_without_a_row_map(fmt, tiled, kernel):
     """out_dtype float16 on the plain grouped matmul: same accumulators, rounded to half; rows of no
     group are zero-filled as in the bf16 call."""
     ofmt = orc.E4M3 if fmt == "e4m3" else orc.E2M1
@@ -691,7 +694,7 @@ def test_group_table_of_many_groups_covers_every_tile_once(e, t, seed):
 # ---------------------------------------------------------------- half-precision output
 
 @pytest.mark.parametrize("tiled", [True, False], ids=["tiled", "generic"])
-def test_fp16_output_of_the_int8_and_dense_mx_operators(tiled):
+def test_fp16_output_of_the_int8_and_dense_mx_operators(tiled, kernel):
     """IEEE half output (what the reference's int8 launchers write, tests/dynamic_tiling/impl/kernel_int8.cpp:16)
     is the same fp32 result rounded to half: within the gate against the oracle and closer to it than bf16's
     8 bits allow (the oracle's fp32 value against a correctly rounded half: at most 2^-11 apart, relative)."""
@@ -741,7 +744,7 @@ def test_fp16_output_of_the_int8_and_dense_mx_operators(tiled):
 
 @pytest.mark.parametrize("sizes,t", [([-5, 300, -1, 2 ** 30, 7], 500), ([2 ** 31 - 1, 2 ** 31 - 1, 5], 300), ([0, 0, 0], 64), ([100] * 200, 9000)],
                          ids=["negative-and-huge", "sum-overflows-int32", "all-empty", "200-groups-run-out-of-rows"])
-def test_group_sizes_are_clipped_the_same_way_on_both_paths(sizes, t):
+def test_group_sizes_are_clipped_the_same_way_on_both_paths(sizes, t, kernel):
     """Group sizes below zero count as empty and the groups stop where the rows do (the reference's golden pads the
     remainder with zeros, examples/utils/gen_data_fp4_mx_alltoallv_gmm.py:788-790): the tiled kernels (table built by
     one wave with two scans) and the generic ones (one thread's running sum) agree to the bit on which rows belong

@@ -32,7 +32,7 @@ def case(e, t, k, n, gs, seed):
 @pytest.mark.parametrize("cfg", [(4, 700, 512, 1088, [300, 0, 143, 250]),     # n/2 = 544: 17 blocks (odd: a padding byte), 7 rows of no group
                                  (3, 300, 256, 512, [1, 0, 299]),
                                  (6, 2000, 768, 2048, [700, 13, 0, 256, 900, 131])])
-def test_fused_bytes_equal_quantised_bf16_tiled(fmt, trans_b, cfg):
+def test_fused_bytes_equal_quantised_bf16_tiled(fmt, trans_b, cfg, kernel):
     e, t, k, n, gs = cfg
     x, w, pt, pc, gsd = case(e, t, k, n, gs, seed=t + k + trans_b)
     wd = torch.from_numpy(np.ascontiguousarray(w.transpose(0, 2, 1)) if trans_b else w).cuda()
@@ -115,7 +115,7 @@ def to_dev(x):
                                  (3, 300, 1216, 512, [1, 0, 299]),            # K tail, scale rows off 4-byte boundaries
                                  (5, 1500, 768, 2048, [700, 13, 0, 256, 531])])
 @pytest.mark.parametrize("tiled", [True, False], ids=["tiled", "generic"])
-def test_mx_gmm_swiglu_against_oracle_chain_and_fused_bytes(fmt, trans_b, cfg, tiled):
+def test_mx_gmm_swiglu_against_oracle_chain_and_fused_bytes(fmt, trans_b, cfg, tiled, kernel):
     """bf16 result against the oracle chain (grouped MX GEMM -> bf16 -> SwiGLU of the bf16 tile), then the
     fused MX-quantised activation byte for byte against the oracle's row quantiser of that bf16 result."""
     e, t, k, n, gs = cfg
@@ -153,7 +153,7 @@ def test_mx_gmm_swiglu_against_oracle_chain_and_fused_bytes(fmt, trans_b, cfg, t
 
 
 @pytest.mark.parametrize("tiled", [True, False], ids=["tiled", "generic"])
-def test_edge_cases_of_the_fused_outputs(tiled):
+def test_edge_cases_of_the_fused_outputs(tiled, kernel):
     """All groups empty (every row is a row of no group: zero codes, scale bytes 127), group sizes that run past
     the rows (clipped, as the GEMMs do), one row, and no rows at all."""
     e, k, n = 3, 256, 512
