@@ -21,7 +21,7 @@ enum GemmEpilogue { EPI_PLAIN = 0, EPI_DEQUANT = 1, EPI_DEQUANT_SWIGLU = 2, EPI_
 enum GemmPath { PATH_TILE, PATH_MID1, PATH_MID2, PATH_MID3, PATH_STREAM4, PATH_STREAM8, NUM_KERNELS, PATH_TILE_TAIL = NUM_KERNELS, NUM_PATHS };
 
 constexpr int MAX_GROUPS = 256;
-constexpr int TAIL_TILES = 512;   // most tiles that the second launch of a grouped problem may have (gemm_tail.h): one round of its kernel
+constexpr int TAIL_TILES = 256;   // most tiles that the second launch of a grouped problem may have (gemm_tail.h): one to a CU
 
 // One (dense or grouped) problem: out[T, n_out] = epilogue(A[T,K] x B_e[K,N]).
 struct GemmProblem {

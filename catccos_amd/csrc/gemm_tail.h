@@ -6,8 +6,10 @@
 // few rows it has.  So where the row tiles that make up the last round can all be short ones, the launch leaves them out and a
 // second one of 64 x 128 tiles (gemm_mid_kernel.h, the same sums in the same order) computes those rows.
 // Both launches work out which rows these are, from the group sizes that only the device has: the smallest remainders (rows of a
-// group modulo 256, ties by group) that empty the last round, each at most TAIL_ROWS and all of them together at most one round of
-// the second kernel.
+// group modulo 256, ties by group) that empty the last round, each at most TAIL_ROWS and all of them together at most one tile of the
+// second kernel to a CU.  With two to a CU its steps take longer than the round it replaces: of 132 measured problems (1 to 2
+// rounds, 16 to 64 steps of K) whose second launch had 257 to 512 tiles 110 were slower with it, by 10 % on average and up to 36 %; of
+// 155 with at most 256 tiles 36 were slower and 85 faster, by 3 % on average and up to 19 %.
 #pragma once
 #include "gemm_device.h"
 

@@ -7,6 +7,7 @@
 #include "gemm_common.h"
 #include "gemm_mid.h"
 #include "gemm_stream.h"
+#include "gemm_tail.h"
 #include "gemm_tile_shape.h"
 
 namespace cch {
@@ -104,7 +105,9 @@ static const PathModel PATH_MODEL[NUM_KERNELS] = {
 // decides which, if any).  Worth it behind one round of long tiles, which the second, mostly empty round would nearly double: MXFP8,
 // 16 groups of 3072 rows in all, K 7168, N 4096 (1.12 to 1.19 rounds) 156-177 -> 150-159 us, 8 of 4096, K 4096 (1.25) 87-91 -> 80-83.  Behind
 // two rounds, or with 2048 of K, the second launch's start and the weights it reads again cost what it saves (84 against 79-87 us; int8 at
-// 2.4 rounds 258 against 254), and SwiGLU weights stored [K, N] reach its narrow tiles in pieces of 32 bytes (int8 at 2.4 rounds 312 against 264).
+// 2.4 rounds 258 against 254).  SwiGLU weights stored [K, N] reach its narrow tiles in pieces of 64 bytes: of the measured problems in this
+// window that have a second launch, 10 of those were 7 % slower with it on average, 20 with plain [K, N] weights 4 % faster, 23 with [N, K]
+// ones 3 % and 15 with [N, K] SwiGLU ones 11 %.
 static bool may_have_tail(const GemmProblem &p, bool swiglu, double steps, double fill)
 {
     return p.group_sizes != nullptr && p.num_groups > 1 && fill > 1.0 && fill <= 1.4 && steps >= 32 &&
@@ -215,6 +218,38 @@ int launch_gemm_tile(const GemmProblem &p, int kind, int epi, hipStream_t stream
 }
 
 }  // namespace cch
+
+namespace cch {
+// What the second launch of a grouped problem takes (gemm_tail.h), as both launches work it out: one wave.
+template <bool SWIGLU>
+__global__ __launch_bounds__(64) void tail_rows_kernel(GemmProblem p, int32_t *__restrict__ taken)
+{
+    const GroupRows rows = group_rows(p);
+    const uint32_t key = tail_key<SWIGLU>(p, rows);
+#pragma unroll
+    for (int b = 0; b < GroupRows::NB; b++) {
+        const int g = b * 64 + (int)threadIdx.x;
+        if (g < p.num_groups) taken[g] = in_tail(rows, b, key) ? (rows.hi[b] - rows.lo[b]) & (BM - 1) : 0;
+    }
+}
+}  // namespace cch
+
+extern "C" int cch_gemm_tail_rows(const int32_t *group_sizes, int64_t num_experts, int64_t t, int64_t n, int swiglu, int cus, int32_t *taken, void *stream)
+{
+    using namespace cch;
+    clear_error();
+    CCH_REQUIRE(num_experts >= 1 && num_experts <= MAX_GROUPS, "cch_gemm_tail_rows: num_experts=%lld outside 1..%d", (long long)num_experts, MAX_GROUPS);
+    CCH_REQUIRE(t >= 0 && !(t >> 31) && n >= 1 && !(n >> 31) && cus >= 1 && !(swiglu && n % 2), "cch_gemm_tail_rows: bad shape");
+    CCH_REQUIRE(group_sizes && taken, "cch_gemm_tail_rows: null pointer");
+    GemmProblem p{};
+    p.group_sizes = group_sizes;
+    p.num_groups = (int)num_experts;
+    p.T = (int)t;
+    p.n_out = (int)(swiglu ? n / 2 : n);
+    p.tail_cus = cus;
+    hipLaunchKernelGGL(swiglu ? tail_rows_kernel<true> : tail_rows_kernel<false>, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream), p, taken);
+    return launch_status("tail_rows_kernel");
+}
 
 extern "C" int cch_gemm_kernel_for(int fmt, int swiglu, int64_t num_experts, int64_t t, int64_t n, int64_t k, int trans_b, int cus)
 {

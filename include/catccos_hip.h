@@ -376,6 +376,10 @@ int cch_set_option(const char *name, int value);
  * problem at all).  fmt: CCH_FMT_E4M3, CCH_FMT_E5M2, CCH_FMT_E2M1, or -1 for int8; num_experts 0: a dense problem; n: columns of B
  * (gate and up halves together).  Host code only, no GPU needed. */
 int cch_gemm_kernel_for(int fmt, int swiglu, int64_t num_experts, int64_t t, int64_t n, int64_t k, int trans_b, int cus);
+/* For tests: how many rows of each group (int32 [num_experts], device memory) the second launch of CCH_GEMM_KERNEL_256X256_TAIL
+ * takes for these group sizes: the device code of both launches, run once. */
+int cch_gemm_tail_rows(const int32_t *group_sizes, int64_t num_experts, int64_t t, int64_t n, int swiglu, int cus, int32_t *taken,
+                       void *stream);
 
 #ifdef __cplusplus
 }

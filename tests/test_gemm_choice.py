@@ -43,3 +43,10 @@ def test_the_switch_names_a_kernel():
         assert "gemm_kernel" in L.cch_last_error().decode()
     for v in (*range(7), -1):
         assert L.cch_set_option(b"gemm_kernel", v) == _abi.OK
+
+
+def test_a_last_round_of_short_tiles_is_a_second_launch():
+    for fmt, swiglu, trans_b in ((E4M3, 0, 0), (E4M3, 0, 1), (E4M3, 1, 1), (I8, 0, 1), (I8, 1, 1)):
+        assert chosen(fmt, swiglu, 16, 3072, 4096, 7168, trans_b) == TAIL     # 1.2 rounds of 256 x 256 tiles
+        assert chosen(fmt, swiglu, 16, 8192, 4096, 7168, trans_b) == TILE     # 2.5
+    assert chosen(E4M3, 1, 16, 3072, 4096, 7168, 0) != TAIL                   # [K, N] gate and up columns
