@@ -79,33 +79,39 @@ const char *gemm_tile_unsupported(const GemmProblem &p, int kind, int epi)
 // The 256 x 256 tiles have the fewest bytes through L2 and LDS per product, and one persistent workgroup per CU; the smaller
 // tiles of the others fill more CUs, in shorter steps.  What decides is how many tiles there are to a CU and how long K is, so
 // each kernel has an estimate of its time,
-//     us = start + max(steps * max(step_alone, step_full * rounds) + finish * fill, weights * per_mb),
+//     us = start + max(steps * max(step_alone, step_full * fill) + finish * fill, weights * per_mb),
 //     steps: 128-byte steps of K one wave walks, fill: tiles / CUs, weights: MB of right-hand operands,
-// and the smallest one wins (the 256 x 256 kernel unless another is estimated 3 % faster).  Rounds are the fill, except where one workgroup
-// walks its tiles with the CU to itself: a last, partly empty round then costs at least half a full one.
-// The sizes of groups are not known here.  They are taken for alike (spread as far as a random routing spreads them) and for skewed (any
-// size up to twice the average), and the estimate is the mean of the two: 140 rows of each of 16 experts are one row tile of 256 if alike
-// and 1.1 if skewed, and 64 of 128 rows are one or two of 64 x 128 tiles.
-// The constants are a fit of this form, by the choices it leads to and not by the times (which are off by 10 to 20 % each), to 5400 times
-// of every kernel on 3000 problems: dense and grouped, alike to Zipf-sized groups, all kinds and layouts, 1 to 32768 rows, K and N from 512
-// to 8192, weights from HBM (dense ones also from the caches).  On 1900 others the choices are within 2.4 % of the best ones in the
-// geometric mean (dense 0.9, grouped 2.5), take 0.72 of the 256 x 256 kernel's time (dense 0.46, grouped 0.76), and are more than 10 % slower
-// than that kernel on 10.  (Before, with one estimate for average groups, constants common to all kinds and a rate of weights that changed
-// from 1 to 1.4 rounds: 2.7 % and 0.72, and 21 of them more than 10 % slower.)
+// and the smallest one wins (the 256 x 256 kernel unless another is estimated 8 % faster).  With one workgroup to a CU a last,
+// partly empty round costs at least half a full one: fill counts as floor(fill) + 0.5 + 0.5 * the rest.  The constants are fits of this form by
+// the choices they lead to, not by the times, which are off by 10 to 20 % each: the table's first to 1200 problems (dense and grouped, all kinds
+// and layouts), GROUPED_TILE to 6100 groupings of 3800 others.
+// The sizes of groups are not known here: fill counts average groups, whose last row tile is half full.  With [N, K] weights, which come to
+// the 256 x 256 kernel at a rate that depends on the CUs at work, that was not enough for its time, which goes up in whole rounds:
+// 128 rows of each of 16 experts are one row tile each if the groups are alike and 1.1 if they are skewed, and with 16 column tiles that is one round of
+// the chip or the start of another.  There its estimate is the mean of one for groups alike (spread as far as a random routing spreads them)
+// and one for skewed groups (any size up to twice the average), each over the row tiles more or less that so many groups come to.
+// On 1300 problems that nothing was fitted to (times of every kernel in profiles/gemm_kernel_times.csv, 1900 groupings) the choices are within
+// 2.6 % of the best kernel in the geometric mean (dense 1.6, grouped 2.7), take 0.72 of the 256 x 256 kernel's time (dense 0.46, grouped 0.76) and
+// are more than 10 % slower than that kernel on 18 groupings; with one estimate for average groups and a rate of weights that changed where a second launch
+// is tried on 21, and on 170 of 2500 groupings with [N, K] weights and many near whole rounds, now 79.  Of 2374 products of perf/cases.py's ranges 5 got
+// slower by more than 3 % and 3 faster.  (The same form for [K, N] weights too, or all constants fitted anew, per operand kind, gained more near whole rounds
+// and lost elsewhere: 18 and 51 of the 2374 slower by more than 3 %.)
 struct PathModel {
     int tm, tn, waves_k;    // rows and columns of B per tile, waves that share a tile's K
     bool rounds;            // a CU runs one workgroup at a time, and tiles long enough for that to count
-    double start, step_alone[3], step_full[3], finish[3][2];   // per kind (int8, FP8, FP4), finish also without and with SwiGLU
+    double start, step_alone, step_full, finish;
     double per_mb[3];       // B as [N, K], as [K, N], and as [K, N] with gate and up columns apart (narrower pieces of a row)
 };
 static const PathModel PATH_MODEL[NUM_KERNELS] = {
-    {256, 256, 1, true, 9.61, {1.3, 1.22, 1.2}, {1.4, 1.36, 1.47}, {{3.19, 3.29}, {4.18, 5.01}, {3.02, 4.97}}, {0.272, 0.172, 0.183}},
-    {64, 128, 1, false, 3.46, {0.494, 0.474, 0.512}, {0.592, 0.652, 0.656}, {{1.5, 1.56}, {1.17, 1.1}, {1.33, 1.46}}, {0.161, 0.201, 0.233}},
-    {128, 128, 1, false, 5.01, {0.611, 0.67, 0.65}, {0.737, 0.785, 0.75}, {{2.33, 2.58}, {1.12, 1.16}, {1.51, 1.44}}, {0.21, 0.243, 0.292}},
-    {128, 256, 1, true, 4.14, {0.836, 0.885, 0.837}, {1.12, 1.18, 1.08}, {{6.85, 6.23}, {6.84, 5.15}, {6.66, 5.52}}, {0.276, 0.25, 0.169}},
-    {STREAM_TM, STREAM_TN, 4, false, 1.68, {1.28, 1.76, 1.78}, {1.34, 1.56, 1.89}, {{0.662, 1.19}, {0.792, 1.08}, {1.21, 1.89}}, {0.302, 0.352, 0.43}},
-    {STREAM_TM, STREAM_TN, 8, false, 3.0, {1.11, 1.41, 1.36}, {2.52, 2.86, 3.41}, {{2.38, 2.08}, {1.79, 2.02}, {2.61, 2.29}}, {0.215, 0.26, 0.654}},
+    {256, 256, 1, true, 9.7, 1.27, 1.66, 3.9, {0.30, 0.20, 0.21}},
+    {64, 128, 1, false, 4.5, 0.37, 0.50, 1.55, {0.18, 0.22, 0.22}},
+    {128, 128, 1, false, 5.75, 0.48, 0.65, 1.55, {0.19, 0.22, 0.27}},
+    {128, 256, 1, true, 5.6, 0.69, 1.07, 4.9, {0.20, 0.22, 0.205}},
+    {STREAM_TM, STREAM_TN, 4, false, 3.35, 0.95, 1.09, 1.05, {0.245, 0.29, 0.30}},
+    {STREAM_TM, STREAM_TN, 8, false, 3.7, 1.24, 1.92, 2.0, {0.21, 0.255, 0.46}},
 };
+// The 256 x 256 kernel on grouped problems with [N, K] weights: every round started costs a whole `finish`.
+static const PathModel GROUPED_TILE = {256, 256, 1, true, 9.93, 1.22, 1.36, 4.34, {0.233, 0.0, 0.0}};
 
 // Average of the row tiles of a group whose size lies anywhere in [lo, hi] rows, tiles of tm rows; a group has at least one.
 static double row_tiles_of(double lo, double hi, int tm)
@@ -115,6 +121,24 @@ static double row_tiles_of(double lo, double hi, int tm)
         return n * (n + 1) / 2 + (x - n) * (n + 1);
     };
     return std::max(1.0, (sum(hi / tm) - sum(lo / tm)) * tm / (hi - lo));
+}
+
+// us of the 256 x 256 kernel on a grouped problem with [N, K] weights.
+static double grouped_tile_us(const GemmProblem &p, double steps, double weights, int tn_out, int cus)
+{
+    const PathModel &m = GROUPED_TILE;
+    const double groups = std::min<int64_t>(p.num_groups, p.T), average = p.T / groups, spread = 1.73 * std::sqrt(average);
+    const double per_row_tile = (double)((p.n_out + tn_out - 1) / tn_out) / cus, more_or_less = 0.5 * std::sqrt(groups);
+    const double row_tiles[2] = {groups * row_tiles_of(std::max(0.0, average - spread), average + spread, m.tm),
+                                 groups * row_tiles_of(0.0, 2 * average, m.tm)};
+    double us = 0.0;
+    for (double tiles : row_tiles)
+        for (int d = -7; d <= 7; d += 2) {
+            const double fill = std::max(tiles + d / 8.0 * more_or_less, groups) * per_row_tile, whole = std::floor(fill), rest = fill - whole;
+            const double rounds = fill > 1.0 && rest > 0.0 ? whole + 0.5 + 0.5 * rest : fill, started = fill > 1.0 ? std::ceil(fill) : fill;
+            us += m.start + std::max(steps * std::max(m.step_alone, m.step_full * rounds) + m.finish * started, weights * m.per_mb[0]);
+        }
+    return us / 16;
 }
 
 // Whether a grouped problem on 256 x 256 tiles leaves the short row tiles of its last round to a second launch (gemm_tail.h; the device
@@ -130,7 +154,7 @@ static bool may_have_tail(const GemmProblem &p, bool swiglu, double steps, doubl
            (p.trans_b || (!swiglu && p.N < 1 << 21));
 }
 
-// Tiles to a CU where the groups' last row tiles are half full on average; groups of a few rows have one tile each.
+// Average number of tiles to a CU: a group's last row tile is half full on average; groups of a few rows have one tile each.
 static double fill_of(const GemmProblem &p, int tm, int tn_out, int cus)
 {
     const double groups = std::min<int64_t>(p.num_groups, p.T);   // that can have rows
@@ -158,34 +182,25 @@ static GemmPath choose_path(const GemmProblem &p, int kind, int epi, int cus)
     const bool swiglu = epi == EPI_DEQUANT_SWIGLU || epi == EPI_SWIGLU;
     const double steps = (p.K / epb + BKB - 1) / BKB;
     const double groups = std::min<int64_t>(p.num_groups, p.T);   // that can have rows
-    const double weights = groups * (double)p.N * (p.K / epb) * 1e-6, average = p.T / groups, spread = 1.73 * std::sqrt(average);
+    const double weights = groups * (double)p.N * (p.K / epb) * 1e-6;
     const int layout = p.trans_b ? 0 : swiglu ? 2 : 1;
-    GemmPath best = may_have_tail(p, swiglu, steps, fill_of(p, 256, swiglu ? 128 : 256, cus)) ? PATH_TILE_TAIL : PATH_TILE;
+    const bool tail = may_have_tail(p, swiglu, steps, fill_of(p, 256, swiglu ? 128 : 256, cus));
+    GemmPath best = tail ? PATH_TILE_TAIL : PATH_TILE;
     if (path_refuses(p, kind, PATH_STREAM4)) return PATH_TILE;
     double best_us = 0.0;
     for (int i = 0; i < NUM_KERNELS; i++) {
         const PathModel &m = PATH_MODEL[i];
-        const int tn_out = swiglu ? m.tn / 2 : m.tn;
-        const double per_row_tile = (double)((p.n_out + tn_out - 1) / tn_out) / cus;
-        auto us_of = [&](double fill, double rounds) {
-            return m.start + std::max(steps / m.waves_k * std::max(m.step_alone[kind], m.step_full[kind] * rounds) + m.finish[kind][swiglu] * fill,
-                                      weights * m.per_mb[layout]);
-        };
-        auto alike = [&](double fill) {
-            const double whole = std::floor(fill);
-            return us_of(fill, m.rounds && fill > 1.0 && fill > whole ? whole + 0.5 + 0.5 * (fill - whole) : fill);
-        };
-        // (anywhere between two whole rounds: what half a round comes to over all of them, from three quarters of the first on)
-        auto skewed = [&](double fill) { return us_of(fill, m.rounds ? fill + std::min(0.25, std::max(0.0, fill - 0.75)) : fill); };
-        double us;
-        if (p.group_sizes) {
-            us = 0.5 * (alike(groups * row_tiles_of(std::max(0.0, average - spread), average + spread, m.tm) * per_row_tile) +
-                        skewed(groups * row_tiles_of(0.0, 2 * average, m.tm) * per_row_tile));
-        } else {
-            us = alike((double)((p.T + m.tm - 1) / m.tm) * per_row_tile);
-        }
+        const double fill = fill_of(p, m.tm, swiglu ? m.tn / 2 : m.tn, cus), whole = std::floor(fill);
+        double rounds = m.rounds && fill > 1.0 && fill > whole ? whole + 0.5 + 0.5 * (fill - whole) : fill;
+        // (groups: fill is an average, and a tile too many costs half a round: what that comes to over all fractions)
+        if (i == PATH_MID3 && p.group_sizes && fill > 1.0) rounds = fill + 0.25;
+        double us = m.start + std::max(steps / m.waves_k * std::max(m.step_alone, m.step_full * rounds) + m.finish * fill, weights * m.per_mb[layout]);
+        if (i == PATH_TILE && p.group_sizes && p.trans_b) us = grouped_tile_us(p, steps, weights, swiglu ? 128 : 256, cus);
+        // (with [K, N] weights the second launch is priced by itself)
+        else if (i == PATH_TILE && tail)
+            us = std::min(us, m.start + std::max(steps * m.step_full + m.finish * fill, weights * m.per_mb[layout]) + 5.0 + 0.45 * steps);
         if (i == PATH_TILE) {
-            best_us = 0.97 * us;
+            best_us = 0.92 * us;
         } else if (us < best_us) {
             best = (GemmPath)i;
             best_us = us;
