@@ -21,7 +21,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int DQ_THREADS = 256;   // 4 rows per workgroup
-constexpr int DQ_FEW_ROWS = 256;  // rows that get a workgroup (of up to eight waves) each
+constexpr int DQ_FEW_ROWS = 256;  // up to so many rows are shared by up to eight waves each
 constexpr int DQ_MAX_CHUNKS = 32; // 32 x 512 columns held in registers, by up to four waves
 
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v)
@@ -210,7 +210,8 @@ static int launch_dq(const void *x, const int32_t *src, const float *smooth, con
     // pieces of work measured fastest (5.8 TB/s at K = 7168 against 5.4 with two waves per row
     // and 5.0 with one)
     // Few rows (a decode step): up to DQ_FEW_ROWS of them are on the chip at a time whatever the split, so the
-    // time is one wave's chain of instructions, and a row is shared by as many waves as it has chunks.
+    // time is one wave's chain of instructions.  A row of one chunk (512 columns) is one wave's, four rows to a workgroup; of two to
+    // four chunks four waves', of five to eight eight waves', one chunk each; of nine to sixteen eight waves', two chunks each.
     // Measured (two and four waves of four chunks -> this): 64 x 4096 4.3 -> 3.2 us, 96 x 2048 4.0 -> 3.1, 64 x 7168 4.2 -> 3.6,
     // 256 x 4096 4.4 -> 3.4, 256 x 8192 4.9 -> 4.3; from 512 rows on the split below is as fast or faster.
     if (t <= DQ_FEW_ROWS && chunks <= 16) {

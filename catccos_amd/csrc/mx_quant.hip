@@ -462,7 +462,8 @@ static int launch_scatter(const void *x, const int32_t *dst_idx, void *packed, i
     const int64_t wpr = (nblk * 4 + 63) / 64;
     // Only the loads ask for alignment.  Packed rows are a multiple of 8 bytes for every fourth multiple of 64 columns only, and
     // with byte stores for the others 4096 x 6784 to two rows each took 58.7 us (now 24.7), 512 x 1984 to four 9.1 (5.5), 2 x 7040
-    // to two 5.6 (3.5).
+    // to two 5.6 (3.5).  (The stores are without the non-temporal hint, also where rows are aligned: 4096 x 6912 to two 27.9 us, with it
+    // 29.8, 16384 x 2816 to four 77.3 against 84.9, 512 x 6912 to six 9.5 against 10.1, FP4 likewise, none slower.)
     const bool vec = (k % 8 == 0) && aligned(x, 16);
     int dev = 0, cus = 0;
     CCH_HIP(hipGetDevice(&dev));

@@ -207,7 +207,7 @@ int cch_mx_gmm_swiglu_mx(const void *a, const void *sa, const void *b, const voi
  * stage's buffer goes into the up projection as it is, as the reference's GMM1 reads its packed
  * operand (PackedMxTileCopyTlaToUB, examples/ascend950_dispatch_ffn_combine/
  * ascend950_dispatch_ffn_combine_device.h:118-122).  The tiled kernels take rows of a multiple of 4
- * bytes (every K that is a multiple of 64). */
+ * bytes (every K that is a multiple of 128); those of an odd multiple of 64 go to the generic kernel. */
 int cch_mx_gmm_swiglu_mx_packed(const void *packed_a, const void *b, const void *sb, const int32_t *group_sizes, void *payload,
                                 void *scales, int64_t num_experts, int64_t t, int64_t n, int64_t k, int fmt, int trans_b, int out_fmt,
                                 void *stream);
@@ -342,7 +342,10 @@ int cch_dyn_quant_i8_rows_smooth(const void *x, const int32_t *src_rows, const f
  * allow it; else 1 for grouped problems and 0 for dense ones), -1 (default) = 2; an order set here also keeps problems of every
  * size on those kernels (by default the ones too small for 256 x 256 tiles go to kernels with smaller tiles);
  * "gemm_kernel" = 0..6 asks for one of the tiled MFMA kernels (CCH_GEMM_KERNEL_*) whatever the size, -1 (default) chooses per
- * problem: a GEMM entry point returns CCH_ENOSUP where that kernel does not take the problem ("gemm_tile_order" goes first);
+ * problem: a GEMM entry point returns CCH_ENOSUP where that kernel does not take the problem ("gemm_tile_order" goes first).
+ * Kernels 0, 1, 2, 3 and 6 add up K in the same order and give the same bits; 4 and 5, which problems of few rows go to, add up K
+ * in 4 or 8 parts, also in fp32, which now and then moves the rounding of an MX result.  So by default the last bit of an MX
+ * result can depend on how many rows the call has; 0 makes it independent of that (int8 sums are exact on all of them);
  * "i8_epilogue_fp16_step" = 1 makes the int8 epilogues (cch_gemm_i8_dequant*, cch_gmm_i8_dequant*, both kernel paths)
  * round acc * per_channel to IEEE half before the per-token factor, as the reference's device kernel does
  * (include/catccos/epilogue/block/block_epilogue_per_token_dequant_swiglu.hpp:348-361: the matrix unit's output stage
