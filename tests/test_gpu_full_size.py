@@ -2,7 +2,8 @@
 cache-blocked routine (the gate of the small-shape tests; the routine is pinned bit for bit to the row-at-a-time
 golden and does a configuration in a second or two on the box's cores), plus a property that holds at any size and
 needs no oracle - an exact power-of-two scaling (bf16 rounding commutes with a factor of two) or the equality
-of the grouped result with per-expert dense calls (same accumulation order along K for every element).
+of the grouped result with per-expert dense calls (same accumulation order along K for every element; the MX calls ask for the
+256 x 256 kernel there, since calls of few rows split K by default).
 Inputs are drawn on the GPU and quantised by the library's own quantisers, which have bit-exact parity
 tests of their own."""
 import numpy as np
@@ -116,13 +117,20 @@ def test_cfg5_mx_grouped_16384_tokens_32_experts(fmt, ofmt):
     out = cc.mx_grouped_matmul(a, sa, b, sb, gs, fmt, 0)
     gold = orc.mx_gmm(a.cpu().numpy(), sa.cpu().numpy(), b.cpu().numpy(), sb.cpu().numpy(), n, k, ofmt, 0, group_sizes=gs_h, blocked=True)
     close(out.float().cpu().numpy(), gold, fmt + ", every row")
-    # per-expert dense calls equal the grouped result bit for bit; empty groups contribute nothing
+    # per-expert dense calls on the same kernel equal the grouped result bit for bit; on the kernel of their own choice their sums may be
+    # in another order, which moves a bf16 rounding now and then; empty groups contribute nothing
     r0 = 0
     for g in range(e):
         sz = int(gs_h[g])
         if sz:
-            one = cc.mx_matmul(a[r0:r0 + sz], sa[r0:r0 + sz], b[g], sb[g], fmt, 0)
-            assert torch.equal(one, out[r0:r0 + sz]), g
+            one = cc.mx_matmul(a[r0:r0 + sz], sa[r0:r0 + sz], b[g], sb[g], fmt, 0).float()
+            cc.set_option("gemm_kernel", 0)
+            same = cc.mx_matmul(a[r0:r0 + sz], sa[r0:r0 + sz], b[g], sb[g], fmt, 0)
+            cc.set_option("gemm_kernel", -1)
+            assert torch.equal(same, out[r0:r0 + sz]), g
+            differ = one != same.float()
+            assert float(differ.float().mean()) <= 1e-2, g
+            assert bool(((one - same.float()).abs() <= 2.0 ** -7 * same.float().abs() + 2.0 ** -20 * same.float().abs().max())[differ].all()), g
         r0 += sz
     assert r0 == t
     # the result does not depend on the launch: forty more, queued back to back (as the bench queues them), equal the first to
