@@ -198,20 +198,21 @@ __global__ __launch_bounds__(QUANT_THREADS) void mx_quant_rows_kernel(
     }
 }
 
-// Fast path of the row quantiser: round to nearest even with the hardware conversions, K a
-// multiple of 1024 (so that wave-steps pair up inside a row and none is partial) and 16-byte
-// aligned buffers.  No per-lane bounds checks; a wave owns pairs of adjacent wave-steps
-// (1024 elements of one row), keeps the next pair's loads in flight while it converts the
-// current one, stores 16 (FP8) or 8 (FP4) payload bytes per lane and writes the 32 scale bytes
-// of the pair as dwords gathered with row shifts.
-// SCATTER: as in mx_quant_rows_kernel, the row goes to rows dst_idx[r*topk + 0 .. topk-1]; `sld`
-// is then the distance between scale rows of the packed output.
+// Fast path of the row quantiser: round to nearest even with the hardware conversions, K a multiple of 64 and 16-byte
+// aligned buffers.  Rows of whole pairs of MX blocks lie back to back, payload and scales alike, so the tensor is one run of
+// elements: a wave owns 1024 consecutive ones (wherever rows begin), keeps its next 1024 in flight while it converts the current ones,
+// stores 16 (FP8) or 8 (FP4) payload bytes per lane and writes the 32 scale bytes as dwords gathered with row shifts.
+// Only the last piece of the run can be partial; nothing else is checked per lane.
+// (Bound by HBM where large, by a launch and one load's latency where small.  K no multiple of 1024 took the general kernel before.)
+// SCATTER (K a multiple of 1024): row r goes to rows dst_idx[r*topk + 0 .. topk-1]; a piece is then 1024 elements of one row, `ppr` of
+// them a row, and `sld` the distance between scale rows of the packed output.
 // HALF: the input is IEEE half instead of bf16 (same layout, same stores; the shared exponent comes
 // from the block maximum widened to fp32 and the codes from the packed-half conversions).
+// `npairs` counts pieces; the last one holds `rest` elements (a multiple of 64; 1024: none is partial).
 template <int FMT, bool SCATTER = false, bool HALF = false>
 __global__ __launch_bounds__(QUANT_THREADS) void mx_quant_rows_fast_kernel(
-    const uint16_t *__restrict__ x, uint8_t *__restrict__ payload, uint8_t *__restrict__ scales, int K, int sld, int pld,
-    int ppr, int npairs, const int32_t *__restrict__ dst_idx = nullptr, int topk = 1, int out_rows = 0x7FFFFFFF)
+    const uint16_t *__restrict__ x, uint8_t *__restrict__ payload, uint8_t *__restrict__ scales, int npairs, int rest, int K = 0, int sld = 0,
+    int pld = 0, int ppr = 1, const int32_t *__restrict__ dst_idx = nullptr, int topk = 1, int out_rows = 0x7FFFFFFF)
 {
     constexpr bool FP4 = is_fp4_v<FMT>;
     const int lane = threadIdx.x & 63;
@@ -222,9 +223,16 @@ __global__ __launch_bounds__(QUANT_THREADS) void mx_quant_rows_fast_kernel(
     struct Dest {
         int row[SCATTER ? QUANT_MAX_TOPK : 1];
     };
+    auto partial = [&](int p) { return !SCATTER && p == npairs - 1 && rest < 1024; };   // wave-uniform
     auto fetch = [&](int p, u32x4 (&v)[2], Dest &d) {
-        const int r = p / ppr, c = p - r * ppr;  // row, pair within the row (wave-uniform)
+        const int r = SCATTER ? p / ppr : 0, c = SCATTER ? p - r * ppr : p;  // row, piece of it (wave-uniform)
         const uint16_t *src = x + (size_t)r * K + (size_t)c * 1024 + lane * 8;
+        if (partial(p)) {
+            v[0] = v[1] = (u32x4){0, 0, 0, 0};
+            if (lane * 8 < rest) v[0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src));
+            if (512 + lane * 8 < rest) v[1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + 512));
+            return;
+        }
         v[0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src));
         v[1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + 512));
         if constexpr (SCATTER) {
@@ -236,7 +244,7 @@ __global__ __launch_bounds__(QUANT_THREADS) void mx_quant_rows_fast_kernel(
         }
     };
     auto convert = [&](int p, const u32x4 (&v)[2], const Dest &d) {
-        const int r0 = p / ppr, c = p - r0 * ppr;
+        const int c = SCATTER ? p % ppr : 0;
         uint32_t q[2][2], sdw[2];
 #pragma unroll
         for (int h = 0; h < 2; h++) {
@@ -264,13 +272,28 @@ __global__ __launch_bounds__(QUANT_THREADS) void mx_quant_rows_fast_kernel(
         const uint32_t send0 = odd_lane ? q[0][0] : q[1][0], send1 = odd_lane ? q[0][1] : q[1][1];
         const uint32_t recv0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)send0, 0xB1, 0xF, 0xF, true);
         const uint32_t recv1 = FP4 ? 0u : (uint32_t)__builtin_amdgcn_update_dpp(0, (int)send1, 0xB1, 0xF, 0xF, true);
-        // element offset inside the row of the first value this lane stores
+        // element offset inside the row (the run's piece) of the first value this lane stores
         const int k = c * 1024 + (odd_lane ? 512 + (lane - 1) * 8 : lane * 8);
+        const int have = partial(p) ? rest : 1024;   // elements of the piece
 #pragma unroll
         for (int t = 0; t < (SCATTER ? QUANT_MAX_TOPK : 1); t++) {
-            const int r = SCATTER ? d.row[t] : r0;
+            const int r = SCATTER ? d.row[t] : 0;
             if (r < 0) continue;  // wave-uniform
-            uint8_t *dst = payload + (size_t)r * pld + (FP4 ? (k >> 1) : k);
+            uint8_t *dst = payload + (SCATTER ? (size_t)r * pld : (size_t)p * (FP4 ? 512 : 1024)) + (FP4 ? (k >> 1) : k);
+            if (!SCATTER && have < 1024) {
+                // the end of the run: 16 elements per lane, scales in pairs of blocks
+                if (k < have) {
+                    if (FP4) *reinterpret_cast<u32x2 *>(dst) = odd_lane ? (u32x2){recv0, q[1][0]} : (u32x2){q[0][0], recv0};
+                    else *reinterpret_cast<u32x4 *>(dst) = odd_lane ? (u32x4){recv0, recv1, q[1][0], q[1][1]} : (u32x4){q[0][0], q[0][1], recv0, recv1};
+                }
+                if ((lane & 15) == 0) {
+                    uint16_t *sp = reinterpret_cast<uint16_t *>(scales + (size_t)p * 32 + (lane >> 4) * 4);
+#pragma unroll
+                    for (int i = 0; i < 4; i++)   // two halves of step 0's dword, two of step 1's, 64 elements each
+                        if ((i >> 1) * 512 + (lane >> 4) * 128 + (i & 1) * 64 < have) sp[(i >> 1) * 8 + (i & 1)] = (uint16_t)(sdw[i >> 1] >> ((i & 1) * 16));
+                }
+                continue;
+            }
             if (FP4) {
                 const u32x2 o = odd_lane ? (u32x2){recv0, q[1][0]} : (u32x2){q[0][0], recv0};
                 __builtin_nontemporal_store(o, reinterpret_cast<u32x2 *>(dst));
@@ -279,7 +302,7 @@ __global__ __launch_bounds__(QUANT_THREADS) void mx_quant_rows_fast_kernel(
                 __builtin_nontemporal_store(o, reinterpret_cast<u32x4 *>(dst));
             }
             if ((lane & 15) == 0) {
-                uint32_t *sp = reinterpret_cast<uint32_t *>(scales + (size_t)r * sld + c * 32 + (lane >> 4) * 4);
+                uint32_t *sp = reinterpret_cast<uint32_t *>(scales + (SCATTER ? (size_t)r * sld + c * 32 : (size_t)p * 32) + (lane >> 4) * 4);
                 sp[0] = sdw[0];
                 sp[4] = sdw[1];
             }
@@ -303,29 +326,27 @@ __global__ __launch_bounds__(QUANT_THREADS) void mx_quant_rows_fast_kernel(
     }
 }
 
-// Fast form for IEEE half input (round to nearest even): returns 1 when the shape or the alignment
-// is not the fast kernel's, so that the caller takes its general kernel.
-template <int FMT>
-static int launch_rows_fast_half(const void *x, void *payload, void *scales, int64_t m, int64_t k, hipStream_t stream)
+// The fast kernel's launch: returns 1 when the shape or the alignment is not its own, so that the caller takes its general kernel.
+template <int FMT, bool HALF>
+static int launch_rows_fast(const void *x, void *payload, void *scales, int64_t m, int64_t k, hipStream_t stream)
 {
-    if (!(k % 1024 == 0 && aligned(x, 16) && aligned(payload, 16) && aligned(scales, 4) && m * (k / 1024) < ((int64_t)1 << 30))) return 1;
-    const int64_t nblk = k / 32, sld = 2 * ((nblk + 1) / 2), pld = is_fp4_v<FMT> ? k / 2 : k;
+    const int64_t npairs = (m * k + 1023) / 1024;
+    if (!(k % 64 == 0 && aligned(x, 16) && aligned(payload, 16) && aligned(scales, 4) && npairs < ((int64_t)1 << 30))) return 1;
     int dev = 0, cus = 0;
     CCH_HIP(hipGetDevice(&dev));
     CCH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const int64_t npairs = m * (k / 1024);
     const unsigned grid = (unsigned)std::min<int64_t>((npairs + QUANT_THREADS / 64 - 1) / (QUANT_THREADS / 64), (int64_t)cus * QUANT_BLOCKS_PER_CU);
-    hipLaunchKernelGGL((mx_quant_rows_fast_kernel<FMT, false, true>), dim3(grid), dim3(QUANT_THREADS), 0, stream,
-                       static_cast<const uint16_t *>(x), static_cast<uint8_t *>(payload), static_cast<uint8_t *>(scales), (int)k, (int)sld,
-                       (int)pld, (int)(k / 1024), (int)npairs);
-    return launch_status("mx_quant_rows_fast_kernel (half input)");
+    hipLaunchKernelGGL((mx_quant_rows_fast_kernel<FMT, false, HALF>), dim3(grid), dim3(QUANT_THREADS), 0, stream,
+                       static_cast<const uint16_t *>(x), static_cast<uint8_t *>(payload), static_cast<uint8_t *>(scales), (int)npairs,
+                       (int)(m * k - (npairs - 1) * 1024));
+    return launch_status("mx_quant_rows_fast_kernel");
 }
 
 int mx_quant_rows_fast_half(const void *x, void *payload, void *scales, int64_t m, int64_t k, int fmt, hipStream_t stream)
 {
-    if (fmt == CCH_FMT_E4M3) return launch_rows_fast_half<CCH_FMT_E4M3>(x, payload, scales, m, k, stream);
-    if (fmt == CCH_FMT_E5M2) return launch_rows_fast_half<CCH_FMT_E5M2>(x, payload, scales, m, k, stream);
-    if (fmt == CCH_FMT_E2M1) return launch_rows_fast_half<CCH_FMT_E2M1>(x, payload, scales, m, k, stream);
+    if (fmt == CCH_FMT_E4M3) return launch_rows_fast<CCH_FMT_E4M3, true>(x, payload, scales, m, k, stream);
+    if (fmt == CCH_FMT_E5M2) return launch_rows_fast<CCH_FMT_E5M2, true>(x, payload, scales, m, k, stream);
+    if (fmt == CCH_FMT_E2M1) return launch_rows_fast<CCH_FMT_E2M1, true>(x, payload, scales, m, k, stream);
     return 1;
 }
 
@@ -341,14 +362,9 @@ static int launch_rows(const void *x, void *payload, void *scales, int64_t m, in
     CCH_HIP(hipGetDevice(&dev));
     CCH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     const int64_t max_blocks = (int64_t)cus * QUANT_BLOCKS_PER_CU;
-    if constexpr (HWCVT)
-    if (k % 1024 == 0 && aligned(x, 16) && aligned(payload, 16) && aligned(scales, 4) && m * (k / 1024) < ((int64_t)1 << 30)) {
-        const int64_t npairs = m * (k / 1024);
-        const unsigned grid = (unsigned)std::min<int64_t>((npairs + QUANT_THREADS / 64 - 1) / (QUANT_THREADS / 64), max_blocks);
-        hipLaunchKernelGGL((mx_quant_rows_fast_kernel<FMT>), dim3(grid), dim3(QUANT_THREADS), 0, stream,
-                           static_cast<const uint16_t *>(x), static_cast<uint8_t *>(payload), static_cast<uint8_t *>(scales),
-                           (int)k, (int)sld, (int)pld, (int)(k / 1024), (int)npairs);
-        return launch_status("mx_quant_rows_fast_kernel");
+    if constexpr (HWCVT) {
+        const int rc = launch_rows_fast<FMT, false>(x, payload, scales, m, k, stream);
+        if (rc != 1) return rc;
     }
     const int64_t rows_per_launch = std::max<int64_t>(1, (int64_t)(1 << 30) / wpr);
     for (int64_t r0 = 0; r0 < m; r0 += rows_per_launch) {
@@ -476,8 +492,8 @@ static int launch_scatter(const void *x, const int32_t *dst_idx, void *packed, i
         const int64_t npairs = tokens * (k / 1024);
         const unsigned grid = (unsigned)std::min<int64_t>((npairs + QUANT_THREADS / 64 - 1) / (QUANT_THREADS / 64), max_blocks);
         hipLaunchKernelGGL((mx_quant_rows_fast_kernel<FMT, true>), dim3(grid), dim3(QUANT_THREADS), 0, stream,
-                           static_cast<const uint16_t *>(x), out, out + pbytes, (int)k, (int)row_bytes, (int)row_bytes,
-                           (int)(k / 1024), (int)npairs, dst_idx, topk, out_rows);
+                           static_cast<const uint16_t *>(x), out, out + pbytes, (int)npairs, 1024, (int)k, (int)row_bytes, (int)row_bytes,
+                           (int)(k / 1024), dst_idx, topk, out_rows);
         return launch_status("mx_quant_rows_fast_kernel (scatter)");
     }
     const int64_t rows_per_launch = std::max<int64_t>(1, (int64_t)(1 << 30) / wpr);

@@ -155,3 +155,26 @@ def test_quant_b_bit_exact(ofmt, gfmt, trans_b, rounding):
     po, so = orc.mx_quant_b(b, ofmt, rounding, trans_b)
     assert np.array_equal(s.cpu().numpy(), so)
     assert np.array_equal(p.cpu().numpy(), po)
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("fmt", ["e4m3", "e5m2", "e2m1"])
+@pytest.mark.parametrize("m,k", [(1, 64), (1, 960), (3, 64), (1, 1024), (1, 1088), (2, 1984), (5, 192), (7, 2112), (333, 1984), (64, 7104)])
+def test_rows_as_one_run(m, k, fmt, half):
+    """K a multiple of 64 alone: pieces of 1024 elements start and end inside rows, the last one is partial (or just not); bytes are the
+    oracle's and nothing behind the two outputs is written."""
+    x = cfg1_input(m, k, seed=m + k)
+    code = {"e4m3": orc.E4M3, "e5m2": orc.E5M2, "e2m1": orc.E2M1}[fmt]
+    if half:
+        x = orc.bf16_to_f32(x).astype(np.float16).view(np.uint16)
+        po, so = orc.mx_quant_rows_f16(x, code, orc.RNE)
+    else:
+        po, so = orc.mx_quant_rows(x, code, orc.RNE)
+    payload = torch.full((po.size + 256,), 0xA5, dtype=torch.uint8, device="cuda")
+    scales = torch.full((so.size + 256,), 0xA5, dtype=torch.uint8, device="cuda")
+    xd = torch.from_numpy(x.view(np.int16)).cuda()
+    fn = _abi.lib().cch_mx_quant_rows_f16 if half else _abi.lib().cch_mx_quant_rows
+    _abi.check(fn(xd.data_ptr(), payload.data_ptr(), scales.data_ptr(), m, k, dict(FMTS)[code], 0, torch.cuda.current_stream().cuda_stream))
+    p, s = payload.cpu().numpy(), scales.cpu().numpy()
+    assert np.array_equal(s[:so.size].reshape(so.shape), so) and (s[so.size:] == 0xA5).all()
+    assert np.array_equal(p[:po.size].reshape(po.shape), po) and (p[po.size:] == 0xA5).all()
