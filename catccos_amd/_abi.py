@@ -56,11 +56,13 @@ PROTOTYPES = {
     "cch_mx_gemm": [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _I, _P],
     "cch_mx_gmm": [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I, _I, _P],
     "cch_mx_gmm_mapped": [_P, _P, _P, _P, _P, _P, _P, _I64, _I, _I64, _I64, _I64, _I64, _I, _I, _P],
+    "cch_moe_ffn_mxfp8_workspace_bytes": [_I64, _I64, _I, _I64, _I64],
+    "cch_moe_ffn_mxfp8": [_P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I, _I64, _I64, _I, _P, _I64, _P],
     "cch_set_option": [c.c_char_p, _I],
     "cch_gemm_tail_rows": [_P, _I64, _I64, _I64, _I, _I, _P, _P],
     "cch_gemm_kernel_for": [_I, _I, _I64, _I64, _I64, _I64, _I, _I],
 }
-_RESTYPE = {"cch_last_error": c.c_char_p, "cch_moe_init_routing_workspace_bytes": _I64}
+_RESTYPE = {"cch_last_error": c.c_char_p, "cch_moe_init_routing_workspace_bytes": _I64, "cch_moe_ffn_mxfp8_workspace_bytes": _I64}
 
 _lib = None
 

@@ -49,6 +49,9 @@ static int run(const GemmProblem &prob, int kind, int epi, hipStream_t stream)
     return launch_gemm_naive(p, kind, epi, stream);
 }
 
+int mx_gmm_swiglu_mx_rows(const void *packed_a, int64_t row_pitch, const void *b, const void *sb, const int32_t *group_sizes, void *payload, void *scales,
+                          int64_t num_experts, int64_t t, int64_t n, int64_t k, int fmt, int trans_b, int out_fmt, void *stream);
+
 static int check_shape(const char *who, int64_t t, int64_t n, int64_t k)
 {
     CCH_REQUIRE(t >= 0 && n >= 0 && k >= 0, "%s: negative shape", who);
@@ -321,6 +324,14 @@ int cch_mx_gmm_swiglu_mx_packed(const void *packed_a, const void *b, const void 
                                 void *scales, int64_t num_experts, int64_t t, int64_t n, int64_t k, int fmt, int trans_b, int out_fmt,
                                 void *stream)
 {
+    return cch::mx_gmm_swiglu_mx_rows(packed_a, 0, b, sb, group_sizes, payload, scales, num_experts, t, n, k, fmt, trans_b, out_fmt, stream);
+}
+}  // extern "C"
+
+// The same with packed rows `row_pitch` bytes apart (0: back to back; otherwise no less than a row).
+int cch::mx_gmm_swiglu_mx_rows(const void *packed_a, int64_t row_pitch, const void *b, const void *sb, const int32_t *group_sizes, void *payload, void *scales,
+                               int64_t num_experts, int64_t t, int64_t n, int64_t k, int fmt, int trans_b, int out_fmt, void *stream)
+{
     GemmProblem p{};
     int kind = 0;
     CCH_REQUIRE(out_fmt == CCH_FMT_E4M3 || out_fmt == CCH_FMT_E5M2 || out_fmt == CCH_FMT_E2M1,
@@ -335,8 +346,7 @@ int cch_mx_gmm_swiglu_mx_packed(const void *packed_a, const void *b, const void 
     int rc = mx_problem("cch_mx_gmm_swiglu_mx_packed", p, rows, rows ? rows + payload_bytes : nullptr, b, sb, group_sizes, payload, num_experts, t, n,
                         k, fmt, trans_b, &kind);
     if (rc) return rc;
-    p.a_pitch = row_bytes;
-    p.sa_pitch = row_bytes;
+    p.a_pitch = p.sa_pitch = row_pitch ? row_pitch : row_bytes;
     p.n_out = (int)(n / 2);
     p.out_scales = static_cast<uint8_t *>(scales);
     p.mx_out = 1;
@@ -344,6 +354,8 @@ int cch_mx_gmm_swiglu_mx_packed(const void *packed_a, const void *b, const void 
     p.mx_out_sld = (int)(2 * ((p.n_out + 63) / 64));
     return run(p, kind, EPI_SWIGLU, static_cast<hipStream_t>(stream));
 }
+
+extern "C" {
 
 int cch_mx_gmm_mapped(const void *a, const void *sa, const void *b, const void *sb, const int32_t *group_sizes,
                       const int32_t *out_row_map, void *out, int64_t out_rows, int out_dtype, int64_t num_experts, int64_t t,

@@ -200,41 +200,33 @@ __global__ __launch_bounds__(QUANT_THREADS) void mx_quant_rows_kernel(
 
 // Fast path of the row quantiser: round to nearest even with the hardware conversions, K a multiple of 64 and 16-byte
 // aligned buffers.  Rows of whole pairs of MX blocks lie back to back, payload and scales alike, so the tensor is one run of
-// elements: a wave owns 1024 consecutive ones (wherever rows begin), keeps its next 1024 in flight while it converts the current ones,
+// elements: a wave owns pieces of 1024 consecutive ones (wherever rows begin), keeps its next piece in flight while it converts the current one,
 // stores 16 (FP8) or 8 (FP4) payload bytes per lane and writes the 32 scale bytes as dwords gathered with row shifts.
 // Only the last piece of the run can be partial; nothing else is checked per lane.
-// (Bound by HBM where large, by a launch and one load's latency where small.  K no multiple of 1024 took the general kernel before.)
-// SCATTER (K a multiple of 1024): row r goes to rows dst_idx[r*topk + 0 .. topk-1]; a piece is then 1024 elements of one row, `ppr` of
-// them a row, and `sld` the distance between scale rows of the packed output.
+// Bound by HBM where large (4096 x 7168: 5.9 TB/s), by a launch and one load's latency where small.  Against the general kernel, which K no
+// multiple of 1024 took before: 4096 x 6784 17.7 -> 14.9 us, 8192 x 1984 10.9 -> 9.3, 16384 x 1984 to FP4 18.0 -> 14.7, 8192 x 7104 from half
+// 36.9 -> 30.9, 2048 x 3008 5.1 -> 4.0, 64 x 1984 3.0 -> 2.4.
+// SCATTER: row r goes to rows dst_idx[r*topk + 0 .. topk-1], `pitch` bytes apart (a multiple of 16); a row is then `ppr` pieces of its
+// own.  `rest` is what the last piece of the run (SCATTER: of each row) holds, a multiple of 64.
 // HALF: the input is IEEE half instead of bf16 (same layout, same stores; the shared exponent comes
 // from the block maximum widened to fp32 and the codes from the packed-half conversions).
-// `npairs` counts pieces; the last one holds `rest` elements (a multiple of 64; 1024: none is partial).
 template <int FMT, bool SCATTER = false, bool HALF = false>
 __global__ __launch_bounds__(QUANT_THREADS) void mx_quant_rows_fast_kernel(
-    const uint16_t *__restrict__ x, uint8_t *__restrict__ payload, uint8_t *__restrict__ scales, int npairs, int rest, int K = 0, int sld = 0,
-    int pld = 0, int ppr = 1, const int32_t *__restrict__ dst_idx = nullptr, int topk = 1, int out_rows = 0x7FFFFFFF)
+    const uint16_t *__restrict__ x, uint8_t *__restrict__ payload, uint8_t *__restrict__ scales, int npairs, int rest, int K = 0, int pitch = 0,
+    int ppr = 1, const int32_t *__restrict__ dst_idx = nullptr, int topk = 1, int out_rows = 0x7FFFFFFF)
 {
     constexpr bool FP4 = is_fp4_v<FMT>;
-    const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (QUANT_THREADS / 64) + (threadIdx.x >> 6)));
     const int stride = (int)gridDim.x * (QUANT_THREADS / 64);
-    const bool odd_lane = lane & 1;
 
     struct Dest {
         int row[SCATTER ? QUANT_MAX_TOPK : 1];
     };
-    auto partial = [&](int p) { return !SCATTER && p == npairs - 1 && rest < 1024; };   // wave-uniform
+    // (all wave-uniform)
+    auto have = [&](int p) { return (SCATTER ? p % ppr == ppr - 1 : p == npairs - 1) ? rest : 1024; };
     auto fetch = [&](int p, u32x4 (&v)[2], Dest &d) {
-        const int r = SCATTER ? p / ppr : 0, c = SCATTER ? p - r * ppr : p;  // row, piece of it (wave-uniform)
-        const uint16_t *src = x + (size_t)r * K + (size_t)c * 1024 + lane * 8;
-        if (partial(p)) {
-            v[0] = v[1] = (u32x4){0, 0, 0, 0};
-            if (lane * 8 < rest) v[0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src));
-            if (512 + lane * 8 < rest) v[1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + 512));
-            return;
-        }
-        v[0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src));
-        v[1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + 512));
+        const int r = SCATTER ? p / ppr : 0, c = SCATTER ? p - r * ppr : p;  // row, piece of it
+        load_piece(x + (size_t)r * K + (size_t)c * 1024, have(p), v);
         if constexpr (SCATTER) {
 #pragma unroll
             for (int t = 0; t < QUANT_MAX_TOPK; t++) {
@@ -244,68 +236,17 @@ __global__ __launch_bounds__(QUANT_THREADS) void mx_quant_rows_fast_kernel(
         }
     };
     auto convert = [&](int p, const u32x4 (&v)[2], const Dest &d) {
-        const int c = SCATTER ? p % ppr : 0;
         uint32_t q[2][2], sdw[2];
+        quant_piece<FMT, HALF>(v, q, sdw);
+        const PieceOut o = piece_out<FMT>(q, sdw);
+        const int n = have(p);
+        if constexpr (SCATTER) {
+            const int c = p % ppr;
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const uint32_t w[4] = {v[h][0], v[h][1], v[h][2], v[h][3]};
-            const uint32_t amax_bits = block_amax_bits(w);   // |half| patterns order like |bf16| patterns
-            int e;
-            bool is_nan;
-            uint32_t sbyte;
-            if constexpr (HALF) {
-                is_nan = amax_bits >= 0x7C00u;   // Inf or NaN in the block
-                sbyte = shared_exp_byte_f32<FMT>(half_bits_to_f32(amax_bits), is_nan, e);
-                quant8_f16_hw<FMT>(w, e, q[h]);
-                if (is_nan) q[h][0] = q[h][1] = FP4 ? 0x77777777u : 0x7F7F7F7Fu;
-            } else {
-                sbyte = shared_exp_byte<FMT>(amax_bits, e, is_nan);
-                quant8_hw<FMT>(w, e, is_nan, q[h]);
-            }
-            // lanes 4j hold block j's scale byte: gather 4 of them into lanes 0, 16, 32, 48
-            const uint32_t b1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)sbyte, 0x104, 0xF, 0xF, true);  // row_shl:4
-            const uint32_t b2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)sbyte, 0x108, 0xF, 0xF, true);  // row_shl:8
-            const uint32_t b3 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)sbyte, 0x10C, 0xF, 0xF, true);  // row_shl:12
-            sdw[h] = sbyte | (b1 << 8) | (b2 << 16) | (b3 << 24);
-        }
-        // Neighbouring lanes swap: even lanes take both halves of step 0, odd lanes of step 1.
-        const uint32_t send0 = odd_lane ? q[0][0] : q[1][0], send1 = odd_lane ? q[0][1] : q[1][1];
-        const uint32_t recv0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)send0, 0xB1, 0xF, 0xF, true);
-        const uint32_t recv1 = FP4 ? 0u : (uint32_t)__builtin_amdgcn_update_dpp(0, (int)send1, 0xB1, 0xF, 0xF, true);
-        // element offset inside the row (the run's piece) of the first value this lane stores
-        const int k = c * 1024 + (odd_lane ? 512 + (lane - 1) * 8 : lane * 8);
-        const int have = partial(p) ? rest : 1024;   // elements of the piece
-#pragma unroll
-        for (int t = 0; t < (SCATTER ? QUANT_MAX_TOPK : 1); t++) {
-            const int r = SCATTER ? d.row[t] : 0;
-            if (r < 0) continue;  // wave-uniform
-            uint8_t *dst = payload + (SCATTER ? (size_t)r * pld : (size_t)p * (FP4 ? 512 : 1024)) + (FP4 ? (k >> 1) : k);
-            if (!SCATTER && have < 1024) {
-                // the end of the run: 16 elements per lane, scales in pairs of blocks
-                if (k < have) {
-                    if (FP4) *reinterpret_cast<u32x2 *>(dst) = odd_lane ? (u32x2){recv0, q[1][0]} : (u32x2){q[0][0], recv0};
-                    else *reinterpret_cast<u32x4 *>(dst) = odd_lane ? (u32x4){recv0, recv1, q[1][0], q[1][1]} : (u32x4){q[0][0], q[0][1], recv0, recv1};
-                }
-                if ((lane & 15) == 0) {
-                    uint16_t *sp = reinterpret_cast<uint16_t *>(scales + (size_t)p * 32 + (lane >> 4) * 4);
-#pragma unroll
-                    for (int i = 0; i < 4; i++)   // two halves of step 0's dword, two of step 1's, 64 elements each
-                        if ((i >> 1) * 512 + (lane >> 4) * 128 + (i & 1) * 64 < have) sp[(i >> 1) * 8 + (i & 1)] = (uint16_t)(sdw[i >> 1] >> ((i & 1) * 16));
-                }
-                continue;
-            }
-            if (FP4) {
-                const u32x2 o = odd_lane ? (u32x2){recv0, q[1][0]} : (u32x2){q[0][0], recv0};
-                __builtin_nontemporal_store(o, reinterpret_cast<u32x2 *>(dst));
-            } else {
-                const u32x4 o = odd_lane ? (u32x4){recv0, recv1, q[1][0], q[1][1]} : (u32x4){q[0][0], q[0][1], recv0, recv1};
-                __builtin_nontemporal_store(o, reinterpret_cast<u32x4 *>(dst));
-            }
-            if ((lane & 15) == 0) {
-                uint32_t *sp = reinterpret_cast<uint32_t *>(scales + (SCATTER ? (size_t)r * sld + c * 32 : (size_t)p * 32) + (lane >> 4) * 4);
-                sp[0] = sdw[0];
-                sp[4] = sdw[1];
-            }
+            for (int t = 0; t < QUANT_MAX_TOPK; t++)
+                if (d.row[t] >= 0) store_piece<FMT, true>(o, n, payload + (size_t)d.row[t] * pitch + c * (FP4 ? 512 : 1024), scales + (size_t)d.row[t] * pitch + c * 32);
+        } else {
+            store_piece<FMT, true>(o, n, payload + (size_t)p * (FP4 ? 512 : 1024), scales + (size_t)p * 32);
         }
     };
 
@@ -466,15 +407,14 @@ static int launch_b(const void *b, void *payload, void *scales, int64_t k, int64
     return launch_status("mx_quant_b_kernel");
 }
 
-// Quantise-once, scatter-to-top-K launch: packed output rows of `row_bytes` = payload bytes +
-// padded scale bytes.
+// Quantise-once, scatter-to-top-K launch: packed output rows of payload bytes + padded scale bytes, `row_bytes` apart.
 template <int FMT, int RND, bool HWCVT>
-static int launch_scatter(const void *x, const int32_t *dst_idx, void *packed, int64_t tokens, int64_t k, int topk,
+static int launch_scatter(const void *x, const int32_t *dst_idx, void *packed, int64_t row_bytes, int64_t tokens, int64_t k, int topk,
                           int out_rows, hipStream_t stream)
 {
     const bool fp4 = is_fp4_v<FMT>;
     const int64_t nblk = (k + 31) / 32, sld = 2 * ((nblk + 1) / 2), pbytes = fp4 ? (k + 1) / 2 : k;
-    const int64_t row_bytes = pbytes + sld;
+    if (row_bytes == 0) row_bytes = pbytes + sld;
     const int64_t wpr = (nblk * 4 + 63) / 64;
     // Only the loads ask for alignment.  Packed rows are a multiple of 8 bytes for every fourth multiple of 64 columns only, and
     // with byte stores for the others 4096 x 6784 to two rows each took 58.7 us (now 24.7), 512 x 1984 to four 9.1 (5.5), 2 x 7040
@@ -487,13 +427,12 @@ static int launch_scatter(const void *x, const int32_t *dst_idx, void *packed, i
     const int64_t max_blocks = (int64_t)cus * QUANT_BLOCKS_PER_CU;
     uint8_t *out = static_cast<uint8_t *>(packed);
     if constexpr (HWCVT)
-    if (k % 1024 == 0 && aligned(x, 16) && aligned(packed, 16) && row_bytes % 16 == 0 &&
-        tokens * (k / 1024) < ((int64_t)1 << 30)) {
-        const int64_t npairs = tokens * (k / 1024);
+    if (k % 64 == 0 && aligned(x, 16) && aligned(packed, 16) && row_bytes % 16 == 0 && tokens * ((k + 1023) / 1024) < ((int64_t)1 << 30)) {
+        const int64_t ppr = (k + 1023) / 1024, npairs = tokens * ppr;
         const unsigned grid = (unsigned)std::min<int64_t>((npairs + QUANT_THREADS / 64 - 1) / (QUANT_THREADS / 64), max_blocks);
         hipLaunchKernelGGL((mx_quant_rows_fast_kernel<FMT, true>), dim3(grid), dim3(QUANT_THREADS), 0, stream,
-                           static_cast<const uint16_t *>(x), out, out + pbytes, (int)npairs, 1024, (int)k, (int)row_bytes, (int)row_bytes,
-                           (int)(k / 1024), dst_idx, topk, out_rows);
+                           static_cast<const uint16_t *>(x), out, out + pbytes, (int)npairs, (int)(k - (ppr - 1) * 1024), (int)k, (int)row_bytes,
+                           (int)ppr, dst_idx, topk, out_rows);
         return launch_status("mx_quant_rows_fast_kernel (scatter)");
     }
     const int64_t rows_per_launch = std::max<int64_t>(1, (int64_t)(1 << 30) / wpr);
@@ -529,6 +468,9 @@ bool quant_set_option(const char *name, int value)
     return true;
 }
 
+int quant_scatter(const void *x, const int32_t *expanded_row_idx, void *packed_out, int64_t out_rows, int64_t row_pitch, int64_t tokens, int64_t k, int top_k,
+                  int fmt, int rounding, void *stream);
+
 }  // namespace cch
 
 extern "C" int cch_mx_quant_scatter_packed(const void *x, const int32_t *expanded_row_idx, void *packed_out, int64_t tokens,
@@ -540,7 +482,13 @@ extern "C" int cch_mx_quant_scatter_packed(const void *x, const int32_t *expande
 extern "C" int cch_mx_quant_scatter_packed_rows(const void *x, const int32_t *expanded_row_idx, void *packed_out, int64_t out_rows,
                                                 int64_t tokens, int64_t k, int top_k, int fmt, int rounding, void *stream)
 {
-    using namespace cch;
+    return cch::quant_scatter(x, expanded_row_idx, packed_out, out_rows, 0, tokens, k, top_k, fmt, rounding, stream);
+}
+
+// The same with rows `row_pitch` bytes apart (0: back to back; otherwise no less than a row).
+int cch::quant_scatter(const void *x, const int32_t *expanded_row_idx, void *packed_out, int64_t out_rows, int64_t row_pitch, int64_t tokens, int64_t k,
+                       int top_k, int fmt, int rounding, void *stream)
+{
     CCH_REQUIRE(out_rows >= 0, "cch_mx_quant_scatter_packed: out_rows=%lld", (long long)out_rows);
     const int orows = (int)std::min<int64_t>(out_rows, 0x7FFFFFFF);
     CCH_REQUIRE(tokens >= 0 && k >= 0, "cch_mx_quant_scatter_packed: negative shape tokens=%lld k=%lld", (long long)tokens,
@@ -555,17 +503,17 @@ extern "C" int cch_mx_quant_scatter_packed_rows(const void *x, const int32_t *ex
     const bool lut = rounding == CCH_ROUND_LUT;
     switch (fmt) {
         case CCH_FMT_E4M3:
-            return lut ? launch_scatter<CCH_FMT_E4M3, CCH_ROUND_LUT, false>(x, expanded_row_idx, packed_out, tokens, k, top_k, orows, s)
-                       : launch_scatter<CCH_FMT_E4M3, CCH_ROUND_RNE, true>(x, expanded_row_idx, packed_out, tokens, k, top_k, orows, s);
+            return lut ? launch_scatter<CCH_FMT_E4M3, CCH_ROUND_LUT, false>(x, expanded_row_idx, packed_out, row_pitch, tokens, k, top_k, orows, s)
+                       : launch_scatter<CCH_FMT_E4M3, CCH_ROUND_RNE, true>(x, expanded_row_idx, packed_out, row_pitch, tokens, k, top_k, orows, s);
         case CCH_FMT_E5M2:
-            return lut ? launch_scatter<CCH_FMT_E5M2, CCH_ROUND_LUT, false>(x, expanded_row_idx, packed_out, tokens, k, top_k, orows, s)
-                       : launch_scatter<CCH_FMT_E5M2, CCH_ROUND_RNE, true>(x, expanded_row_idx, packed_out, tokens, k, top_k, orows, s);
+            return lut ? launch_scatter<CCH_FMT_E5M2, CCH_ROUND_LUT, false>(x, expanded_row_idx, packed_out, row_pitch, tokens, k, top_k, orows, s)
+                       : launch_scatter<CCH_FMT_E5M2, CCH_ROUND_RNE, true>(x, expanded_row_idx, packed_out, row_pitch, tokens, k, top_k, orows, s);
         case CCH_FMT_E2M1:
-            return lut ? launch_scatter<CCH_FMT_E2M1, CCH_ROUND_LUT, false>(x, expanded_row_idx, packed_out, tokens, k, top_k, orows, s)
-                       : launch_scatter<CCH_FMT_E2M1, CCH_ROUND_RNE, true>(x, expanded_row_idx, packed_out, tokens, k, top_k, orows, s);
+            return lut ? launch_scatter<CCH_FMT_E2M1, CCH_ROUND_LUT, false>(x, expanded_row_idx, packed_out, row_pitch, tokens, k, top_k, orows, s)
+                       : launch_scatter<CCH_FMT_E2M1, CCH_ROUND_RNE, true>(x, expanded_row_idx, packed_out, row_pitch, tokens, k, top_k, orows, s);
         case CCH_FMT_E1M2:  // no hardware conversion for this format: integer encoder for both rules
-            return lut ? launch_scatter<CCH_FMT_E1M2, CCH_ROUND_LUT, false>(x, expanded_row_idx, packed_out, tokens, k, top_k, orows, s)
-                       : launch_scatter<CCH_FMT_E1M2, CCH_ROUND_RNE, false>(x, expanded_row_idx, packed_out, tokens, k, top_k, orows, s);
+            return lut ? launch_scatter<CCH_FMT_E1M2, CCH_ROUND_LUT, false>(x, expanded_row_idx, packed_out, row_pitch, tokens, k, top_k, orows, s)
+                       : launch_scatter<CCH_FMT_E1M2, CCH_ROUND_RNE, false>(x, expanded_row_idx, packed_out, row_pitch, tokens, k, top_k, orows, s);
         default:
             return fail(CCH_EINVAL, "cch_mx_quant_scatter_packed: unknown format %d", fmt);
     }

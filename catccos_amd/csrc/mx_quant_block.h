@@ -182,4 +182,105 @@ __device__ __forceinline__ void quant8_f16_hw(const uint32_t (&w)[4], int e, uin
     }
 }
 
+// ---- pieces of 1024 elements, as the streaming quantiser kernels take them: lane l holds elements 8l .. 8l+7 of either half
+
+// Codes q and scale bytes of a piece; lanes 0, 16, 32 and 48 hold four blocks' scale bytes of either half in sdw.
+template <int FMT, bool HALF>
+__device__ __forceinline__ void quant_piece(const u32x4 (&v)[2], uint32_t (&q)[2][2], uint32_t (&sdw)[2])
+{
+    constexpr bool FP4 = is_fp4_v<FMT>;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const uint32_t w[4] = {v[h][0], v[h][1], v[h][2], v[h][3]};
+        const uint32_t amax_bits = block_amax_bits(w);   // |half| patterns order like |bf16| patterns
+        int e;
+        bool is_nan;
+        uint32_t sbyte;
+        if constexpr (HALF) {
+            is_nan = amax_bits >= 0x7C00u;   // Inf or NaN in the block
+            sbyte = shared_exp_byte_f32<FMT>(half_bits_to_f32(amax_bits), is_nan, e);
+            quant8_f16_hw<FMT>(w, e, q[h]);
+            if (is_nan) q[h][0] = q[h][1] = FP4 ? 0x77777777u : 0x7F7F7F7Fu;
+        } else {
+            sbyte = shared_exp_byte<FMT>(amax_bits, e, is_nan);
+            quant8_hw<FMT>(w, e, is_nan, q[h]);
+        }
+        // lanes 4j hold block j's scale byte: gather 4 of them into lanes 0, 16, 32, 48
+        const uint32_t b1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)sbyte, 0x104, 0xF, 0xF, true);  // row_shl:4
+        const uint32_t b2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)sbyte, 0x108, 0xF, 0xF, true);  // row_shl:8
+        const uint32_t b3 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)sbyte, 0x10C, 0xF, 0xF, true);  // row_shl:12
+        sdw[h] = sbyte | (b1 << 8) | (b2 << 16) | (b3 << 24);
+    }
+}
+
+// What a lane stores of a piece: neighbouring lanes have swapped halves, even lanes hold 16 elements of the first half, odd lanes of the second.
+struct PieceOut {
+    u32x4 codes;      // (FP4: the first two)
+    uint32_t sdw[2];
+    int k;            // element of the piece that the lane's codes start at
+};
+template <int FMT>
+__device__ __forceinline__ PieceOut piece_out(const uint32_t (&q)[2][2], const uint32_t (&sdw)[2])
+{
+    constexpr bool FP4 = is_fp4_v<FMT>;
+    const int lane = threadIdx.x & 63;
+    const bool odd_lane = lane & 1;
+    const uint32_t send0 = odd_lane ? q[0][0] : q[1][0], send1 = odd_lane ? q[0][1] : q[1][1];
+    const uint32_t recv0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)send0, 0xB1, 0xF, 0xF, true);
+    const uint32_t recv1 = FP4 ? 0u : (uint32_t)__builtin_amdgcn_update_dpp(0, (int)send1, 0xB1, 0xF, 0xF, true);
+    PieceOut o;
+    if (FP4) o.codes = odd_lane ? (u32x4){recv0, q[1][0], 0, 0} : (u32x4){q[0][0], recv0, 0, 0};
+    else o.codes = odd_lane ? (u32x4){recv0, recv1, q[1][0], q[1][1]} : (u32x4){q[0][0], q[0][1], recv0, recv1};
+    o.sdw[0] = sdw[0];
+    o.sdw[1] = sdw[1];
+    o.k = odd_lane ? 512 + (lane - 1) * 8 : lane * 8;
+    return o;
+}
+
+// Stores a piece of `have` elements (1024, or fewer at the end of a row: a multiple of 64) whose codes start at `payload` (16-byte aligned)
+// and whose scales at `scales` (4-byte aligned, a partial piece's in pairs); NT: the codes with the non-temporal hint.
+template <int FMT, bool NT>
+__device__ __forceinline__ void store_piece(const PieceOut &o, int have, uint8_t *__restrict__ payload, uint8_t *__restrict__ scales)
+{
+    constexpr bool FP4 = is_fp4_v<FMT>;
+    const int lane = threadIdx.x & 63;
+    if (o.k < have) {
+        if (FP4) {
+            u32x2 *dst = reinterpret_cast<u32x2 *>(payload + (o.k >> 1));
+            if (NT) __builtin_nontemporal_store((u32x2){o.codes[0], o.codes[1]}, dst);
+            else *dst = (u32x2){o.codes[0], o.codes[1]};
+        } else {
+            u32x4 *dst = reinterpret_cast<u32x4 *>(payload + o.k);
+            if (NT) __builtin_nontemporal_store(o.codes, dst);
+            else *dst = o.codes;
+        }
+    }
+    if ((lane & 15) == 0) {
+        uint8_t *sp = scales + (lane >> 4) * 4;
+        if (have == 1024) {
+            reinterpret_cast<uint32_t *>(sp)[0] = o.sdw[0];
+            reinterpret_cast<uint32_t *>(sp)[4] = o.sdw[1];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++)   // two halves of the first dword, two of the second, 64 elements each
+                if ((i >> 1) * 512 + (lane >> 4) * 128 + (i & 1) * 64 < have)
+                    reinterpret_cast<uint16_t *>(sp)[(i >> 1) * 8 + (i & 1)] = (uint16_t)(o.sdw[i >> 1] >> ((i & 1) * 16));
+        }
+    }
+}
+
+// Loads a piece of `have` elements from `src` (16-byte aligned); what lies past it counts as zeros.
+__device__ __forceinline__ void load_piece(const uint16_t *__restrict__ src, int have, u32x4 (&v)[2])
+{
+    const int k = (threadIdx.x & 63) * 8;
+    if (have == 1024) {   // wave-uniform
+        v[0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + k));
+        v[1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + k + 512));
+    } else {
+        v[0] = v[1] = (u32x4){0, 0, 0, 0};
+        if (k < have) v[0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + k));
+        if (k + 512 < have) v[1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(src + k + 512));
+    }
+}
+
 }  // namespace cch

@@ -283,39 +283,19 @@ PyObject *MoeFfnMxfp8(PyObject *, PyObject *const *v, Py_ssize_t nv)
         !Plain(v[4], at::kByte, -1) || !Plain(v[5], at::kByte, 3) || !Plain(v[6], at::kByte, -1) || !Flag(v[7], trans_b))
         return Decline();
     const at::Tensor &x = T(v[0]), &idx = T(v[1]), &probs = T(v[2]), &w1 = T(v[3]), &sw1 = T(v[4]), &w2 = T(v[5]), &sw2 = T(v[6]);
-    const int64_t m = x.size(0), k = x.size(1), top_k = idx.size(1), rows = m * top_k, e = w1.size(0), n = w1.size(trans_b ? 1 : 2), h = n / 2;
-    if (idx.size(0) != m || probs.sizes() != idx.sizes() || w1.size(trans_b ? 2 : 1) != k || n % 2 || h == 0 || w2.size(0) != e ||
+    const int64_t m = x.size(0), k = x.size(1), top_k = idx.size(1), e = w1.size(0), n = w1.size(trans_b ? 1 : 2), h = n / 2;
+    if (idx.size(0) != m || probs.sizes() != idx.sizes() || top_k > 8 || w1.size(trans_b ? 2 : 1) != k || n % 2 || h == 0 || w2.size(0) != e ||
         w2.size(trans_b ? 2 : 1) != h || w2.size(trans_b ? 1 : 2) != k || sw1.numel() != e * ScaleCols(k) * n || sw2.numel() != e * ScaleCols(h) * k)
         return Decline();
     at::Tensor out;
     int rc;
     {
         pybind11::gil_scoped_release nogil;
-        const int64_t route_bytes = std::max<int64_t>(cch_moe_init_routing_workspace_bytes(rows, (int)e), 4);
-        // pieces of the intermediate buffer, each on a boundary that every kernel is content with
-        int64_t end = 0;
-        auto piece = [&](int64_t bytes) {
-            const int64_t at = end;
-            end += (bytes + 511) & ~(int64_t)511;
-            return at;
-        };
-        const int64_t at_d2s = piece(rows * 4), at_s2d = piece(rows * 4), at_cnt = piece(e * 4), at_route = piece(route_bytes),
-                      at_packed = piece(rows * (k + ScaleCols(k))), at_act = piece(rows * h), at_scales = piece(rows * ScaleCols(h)), at_y = piece(rows * k * 2);
-        const at::Tensor mid = New(x, {end}, at::kByte);
+        const int64_t bytes = cch_moe_ffn_mxfp8_workspace_bytes(m, k, (int)top_k, e, n);
+        const at::Tensor ws = New(x, {bytes}, at::kByte);
         out = New(x, {m, k}, at::kBFloat16);
-        uint8_t *p = static_cast<uint8_t *>(mid.data_ptr());
-        int32_t *s2d = reinterpret_cast<int32_t *>(p + at_s2d), *cnt = reinterpret_cast<int32_t *>(p + at_cnt);
-        void *stream = Stream();
-        rc = cch_moe_init_routing(static_cast<const int32_t *>(idx.data_ptr()), rows, (int)e, reinterpret_cast<int32_t *>(p + at_d2s), s2d, cnt, 0, p + at_route,
-                                  route_bytes, stream);
-        if (rc == CCH_OK) rc = cch_mx_quant_scatter_packed_rows(x.data_ptr(), s2d, p + at_packed, rows, m, k, (int)top_k, CCH_FMT_E4M3, CCH_ROUND_RNE, stream);
-        if (rc == CCH_OK)
-            rc = cch_mx_gmm_swiglu_mx_packed(p + at_packed, w1.data_ptr(), sw1.data_ptr(), cnt, p + at_act, p + at_scales, e, rows, n, k, CCH_FMT_E4M3, trans_b,
-                                             CCH_FMT_E4M3, stream);
-        if (rc == CCH_OK)
-            rc = cch_mx_gmm(p + at_act, p + at_scales, w2.data_ptr(), sw2.data_ptr(), cnt, p + at_y, e, rows, k, h, CCH_FMT_E4M3, trans_b, stream);
-        if (rc == CCH_OK)
-            rc = cch_moe_token_unpermute(p + at_y, s2d, static_cast<const float *>(probs.data_ptr()), out.data_ptr(), rows, m, k, (int)top_k, stream);
+        rc = cch_moe_ffn_mxfp8(x.data_ptr(), static_cast<const int32_t *>(idx.data_ptr()), static_cast<const float *>(probs.data_ptr()), w1.data_ptr(),
+                               sw1.data_ptr(), w2.data_ptr(), sw2.data_ptr(), out.data_ptr(), m, k, (int)top_k, e, n, trans_b, ws.data_ptr(), bytes, Stream());
     }
     return rc == CCH_OK ? THPVariable_Wrap(out) : Decline();
     END_HANDLE_TH_ERRORS

@@ -323,33 +323,18 @@ at::Tensor MoeFfnMxfp8(const at::Tensor &x_in, const at::Tensor &expert_idx_in, 
     c10::DeviceGuard guard(x_in.device());
     const at::Tensor x = x_in.contiguous(), idx = expert_idx_in.contiguous(), probs = probs_in.contiguous();
     const at::Tensor w1 = w1_in.contiguous(), sw1 = sw1_in.contiguous(), w2 = w2_in.contiguous(), sw2 = sw2_in.contiguous();
-    const int64_t m = x.size(0), k = x.size(1), top_k = idx.size(1), rows = m * top_k, e = w1.size(0);
+    const int64_t m = x.size(0), k = x.size(1), top_k = idx.size(1), e = w1.size(0);
     const int64_t n = trans_b ? w1.size(1) : w1.size(2), h = n / 2;
     TORCH_CHECK((trans_b ? w1.size(2) : w1.size(1)) == k && n % 2 == 0, "w1 must be [E, k, n] (trans_b: [E, n, k]) with n even");
     TORCH_CHECK((trans_b ? w2.size(2) : w2.size(1)) == h && (trans_b ? w2.size(1) : w2.size(2)) == k, "w2 must be [E, n/2, k] (trans_b: [E, k, n/2])");
     TORCH_CHECK(sw1.numel() == e * ScaleCols(k) * n && sw2.numel() == e * ScaleCols(h) * k, "scale tensors do not match the weights");
-    void *stream = StreamOf(x);
-    const auto i32 = x.options().dtype(at::kInt);
-    at::Tensor d2s = at::empty({rows}, i32), s2d = at::empty({rows}, i32), cnt = at::empty({e}, i32);
-    const int64_t ws_bytes = std::max<int64_t>(cch_moe_init_routing_workspace_bytes(rows, (int)e), 4);
-    at::Tensor ws = Bytes(x, {ws_bytes});
-    Check(cch_moe_init_routing(idx.data_ptr<int32_t>(), rows, (int)e, d2s.data_ptr<int32_t>(), s2d.data_ptr<int32_t>(), cnt.data_ptr<int32_t>(), 0,
-                               ws.data_ptr(), ws_bytes, stream),
-          "moe_ffn_mxfp8 (routing)");
-    at::Tensor packed = Bytes(x, {rows, k + ScaleCols(k)});
-    Check(cch_mx_quant_scatter_packed_rows(x.data_ptr(), s2d.data_ptr<int32_t>(), packed.data_ptr(), rows, m, k, (int)top_k, CCH_FMT_E4M3, CCH_ROUND_RNE, stream),
-          "moe_ffn_mxfp8 (dispatch)");
-    at::Tensor act = Bytes(x, {rows, h}), act_scales = Bytes(x, {rows, ScaleCols(h)});
-    Check(cch_mx_gmm_swiglu_mx_packed(packed.data_ptr(), w1.data_ptr(), sw1.data_ptr(), cnt.data_ptr<int32_t>(), act.data_ptr(), act_scales.data_ptr(), e, rows,
-                                      n, k, CCH_FMT_E4M3, (int)trans_b, CCH_FMT_E4M3, stream),
-          "moe_ffn_mxfp8 (up projection)");
-    at::Tensor y = at::empty({rows, k}, x.options());
-    Check(cch_mx_gmm(act.data_ptr(), act_scales.data_ptr(), w2.data_ptr(), sw2.data_ptr(), cnt.data_ptr<int32_t>(), y.data_ptr(), e, rows, k, h, CCH_FMT_E4M3,
-                     (int)trans_b, stream),
-          "moe_ffn_mxfp8 (down projection)");
+    TORCH_CHECK(top_k >= 1 && top_k <= 8, "top_k must be 1..8");
     at::Tensor out = at::empty({m, k}, x.options());
-    Check(cch_moe_token_unpermute(y.data_ptr(), s2d.data_ptr<int32_t>(), probs.data_ptr<float>(), out.data_ptr(), rows, m, k, (int)top_k, stream),
-          "moe_ffn_mxfp8 (combine)");
+    const int64_t ws_bytes = cch_moe_ffn_mxfp8_workspace_bytes(m, k, (int)top_k, e, n);
+    at::Tensor ws = Bytes(x, {ws_bytes});
+    Check(cch_moe_ffn_mxfp8(x.data_ptr(), idx.data_ptr<int32_t>(), probs.data_ptr<float>(), w1.data_ptr(), sw1.data_ptr(), w2.data_ptr(), sw2.data_ptr(),
+                            out.data_ptr(), m, k, (int)top_k, e, n, (int)trans_b, ws.data_ptr(), ws_bytes, StreamOf(x)),
+          "moe_ffn_mxfp8");
     return out;
 }
 

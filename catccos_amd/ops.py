@@ -492,7 +492,7 @@ def mx_grouped_matmul_mapped(a, sa, b, sb, group_sizes, out_row_map, out, fmt="e
 
 
 def moe_ffn_mxfp8(x, expert_idx, probs, w1, sw1, w2, sw2, trans_b=1):
-    """The MXFP8 MoE FFN of one rank that holds every expert, routing to combine, five launches on the current stream
+    """The MXFP8 MoE FFN of one rank that holds every expert, routing to combine, four or five launches on the current stream
     (the reference's Ascend950DispatchFFNCombine, examples/ascend950_dispatch_ffn_combine/ascend950_dispatch_ffn_combine_device.h:124-176):
     routing sort -> MXFP8 quantise-and-scatter -> GMM1 + SwiGLU + MXFP8 quantise -> GMM2 -> weighted un-permute.
 
@@ -509,12 +509,25 @@ def moe_ffn_mxfp8(x, expert_idx, probs, w1, sw1, w2, sw2, trans_b=1):
         raise ValueError("expert_idx and probs must be [m, top_k]")
     m, k = x.shape
     top_k, e = expert_idx.shape[1], w1.shape[0]
-    _, s2d, cnt = moe_init_routing(expert_idx, e)
-    packed = torch.empty((m * top_k, packed_row_bytes(k)), dtype=torch.uint8, device=x.device)
-    mx_quant_scatter_packed(x, s2d, packed, top_k)
-    act, act_scales = mx_grouped_matmul_swiglu_packed(packed, k, w1, sw1, cnt, "e4m3", trans_b, "e4m3")
-    y = mx_grouped_matmul(act, act_scales, w2, sw2, cnt, "e4m3", trans_b)
-    if y.shape[1] != k:
+    if not 1 <= top_k <= 8:
+        raise ValueError("top_k must be 1..8")
+    if expert_idx.dtype != torch.int32 or probs.dtype != torch.float32:
+        raise ValueError("expert_idx must be int32 and probs float32")
+    if w1.dim() != 3 or w2.dim() != 3 or any(w.dtype != torch.uint8 for w in (w1, sw1, w2, sw2)):
+        raise ValueError("w1, w2 must be 3-D uint8 tensors, sw1, sw2 uint8")
+    n = w1.shape[1] if trans_b else w1.shape[2]
+    if n % 2 or (w1.shape[2] if trans_b else w1.shape[1]) != k or sw1.numel() != e * scale_cols(k) * n:
+        raise ValueError("shape mismatch between x, w1 and sw1")
+    if w2.shape[0] != e or (w2.shape[2] if trans_b else w2.shape[1]) != n // 2:
+        raise ValueError("inner dimensions of the two projections differ")
+    if (w2.shape[1] if trans_b else w2.shape[2]) != k:
         raise ValueError("w2 must map back to the hidden size of x")
-    return moe_token_unpermute(y, s2d, probs, top_k)
-
+    if sw2.numel() != e * scale_cols(n // 2) * k:
+        raise ValueError("sw2 has %d entries, expected %d" % (sw2.numel(), e * scale_cols(n // 2) * k))
+    x, expert_idx, probs, w1, sw1, w2, sw2 = (v.contiguous() for v in (x, expert_idx, probs, w1, sw1, w2, sw2))
+    out = torch.empty((m, k), dtype=torch.bfloat16, device=x.device)
+    nbytes = _abi.lib().cch_moe_ffn_mxfp8_workspace_bytes(m, k, top_k, e, n)
+    ws = torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=x.device)
+    check(_abi.lib().cch_moe_ffn_mxfp8(_ptr(x), _ptr(expert_idx), _ptr(probs), _ptr(w1), _ptr(sw1), _ptr(w2), _ptr(sw2), _ptr(out), m, k, top_k, e, n,
+                                       int(trans_b), _ptr(ws), ws.numel(), _stream()))
+    return out

@@ -303,6 +303,24 @@ int cch_moe_init_routing(const int32_t *expert_idx, int64_t rows, int num_expert
 int cch_moe_init_routing_noalloc(const int32_t *expert_idx, int64_t rows, int num_experts, int32_t *dst_to_src,
                                  int32_t *src_to_dst, int32_t *expert_tokens, int cumsum, void *stream);
 
+/* ---- The MXFP8 MoE FFN of one rank that holds every expert, routing to combine ----
+ * Ascend950DispatchFFNCombine (examples/ascend950_dispatch_ffn_combine/
+ * ascend950_dispatch_ffn_combine_device.h:124-176) with the exchanges of one rank: the stages cch_moe_init_routing,
+ * cch_mx_quant_scatter_packed, cch_mx_gmm_swiglu_mx_packed, cch_mx_gmm and cch_moe_token_unpermute on one
+ * stream, four or five launches (up to 8192 routes the sort and the quantiser are one).
+ *   x           bf16 [m, k]; expert_idx int32 [m, top_k] (an entry outside [0, num_experts) is dropped)
+ *   probs       fp32 [m, top_k]; top_k 1..8
+ *   w1 / sw1    E4M3 payload and E8M0 scales of the up projections [num_experts] x [k, n] (gate columns first) in the
+ *               layout trans_b names, w2 / sw2 of the down projections [n/2, k]
+ *   out         bf16 [m, k]
+ *   workspace   device memory on a 512-byte boundary, at least cch_moe_ffn_mxfp8_workspace_bytes(...); nothing in it
+ *               has to be kept or cleared between calls, calls that overlap need one each */
+int64_t cch_moe_ffn_mxfp8_workspace_bytes(int64_t m, int64_t k, int top_k, int64_t num_experts, int64_t n);
+int cch_moe_ffn_mxfp8(const void *x, const int32_t *expert_idx, const float *probs, const void *w1, const void *sw1, const void *w2, const void *sw2,
+                      void *out, int64_t m, int64_t k, int top_k, int64_t num_experts, int64_t n, int trans_b, void *workspace, int64_t workspace_bytes,
+                      void *stream);
+
+
 /* ---- Per-token dynamic int8 quantisation with row gather (feeds config 4) ----
  * Replaces MoeV2GatherDynamicQuant (examples/aux_ops/moe_init_routing_quant_v2/
  * moe_v2_gather_dynamic_quant.h:117-150 Compute, :213-250 the gather loop).

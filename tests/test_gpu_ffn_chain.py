@@ -90,3 +90,42 @@ def test_ffn_chain_against_oracle_chain(cfg):
     got, want = out.float().cpu().numpy(), orc.bf16_to_f32(out_o)
     rms = np.sqrt(np.mean(want ** 2))
     assert np.sqrt(np.mean((got - want) ** 2)) <= 2e-2 * rms and np.abs(got - want).max() <= 0.12 * rms
+
+
+@pytest.mark.parametrize("m,k,n,e,topk,dropped", [
+    (1, 64, 128, 1, 1, False),         # one route, one piece of one pair of blocks
+    (37, 960, 256, 3, 2, True),        # K an odd multiple of 64, dropped entries of either sign
+    (129, 1984, 128, 8, 8, True),      # 1032 routes: two groups of keys per wave; eight tokens per workgroup
+    (300, 1088, 256, 256, 7, False),   # 2100 routes, as many experts as one workgroup sorts
+    (515, 512, 128, 5, 8, True),       # 4120 routes, sixteen tokens and all 128 route places of a workgroup
+    (1024, 64, 128, 4, 8, False),      # 8192 routes: the most that one workgroup sorts
+    (1025, 192, 128, 4, 8, True),      # one token more: the sort's own launches
+    (5, 17472, 128, 2, 2, False),      # 18 pieces a token, more than a workgroup's waves
+    (6, 512, 128, 257, 3, True),       # more experts than MAX: refused
+])
+def test_whole_ffn_is_its_stages(m, k, n, e, topk, dropped):
+    """moe_ffn_mxfp8 against its stages called one by one on rows that were gathered instead of scattered: the same bytes."""
+    g = torch.Generator(device="cuda").manual_seed(m + k + e)
+    x = (torch.randn(m, k, device="cuda", generator=g) * 2).bfloat16()
+    idx = torch.randint(-2 if dropped else 0, e + (3 if dropped else 0), (m, topk), device="cuda", generator=g, dtype=torch.int32)
+    probs = torch.rand(m, topk, device="cuda", generator=g)
+    w1 = [cc.mx_quant_b(torch.randn(k, n, device="cuda", generator=g).bfloat16() * k ** -0.5, trans_b=1) for _ in range(min(e, 8))]
+    w2 = [cc.mx_quant_b(torch.randn(n // 2, k, device="cuda", generator=g).bfloat16() * n ** -0.5, trans_b=1) for _ in range(min(e, 8))]
+    w1, sw1, w2, sw2 = (torch.stack([w[i % len(w)][h] for i in range(e)]) for w in (w1, w2) for h in (0, 1))
+    if e > 256:
+        with pytest.raises(cc.CatccosError, match="num_experts"):
+            cc.moe_ffn_mxfp8(x, idx, probs, w1, sw1, w2, sw2)
+        return
+    d2s, s2d, cnt = cc.moe_init_routing(idx, e)
+    a, sa = cc.mx_quant(x)
+    token = (d2s.clamp(min=0) // topk).long()
+    cc.set_option("require_tiled_gemm", 1)
+    try:
+        out = cc.moe_ffn_mxfp8(x, idx, probs, w1, sw1, w2, sw2)
+        act, act_scales = cc.mx_grouped_matmul_swiglu(a[token], sa[token], w1, sw1, cnt, "e4m3", 1, out_fmt="e4m3")
+        y = cc.mx_grouped_matmul(act, act_scales, w2, sw2, cnt, "e4m3", 1)
+    finally:
+        cc.set_option("require_tiled_gemm", 0)
+    want = cc.moe_token_unpermute(y, s2d, probs, topk)
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+    assert torch.isfinite(want.float()).all() and want.float().abs().max() > 0
