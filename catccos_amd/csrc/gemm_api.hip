@@ -16,6 +16,7 @@ static std::atomic<int> g_force_generic{0};
 static std::atomic<int> g_require_tiled{0};
 static std::atomic<int> g_tile_order{-1};   // -1: chosen per problem
 static std::atomic<int> g_kernel{-1};      // -1: chosen per problem
+static std::atomic<int> g_tiles_192{-1};   // -1: chosen per problem
 static std::atomic<int> g_nt_out{-1};      // -1: chosen per problem
 static std::atomic<int> g_i8_fp16_step{0};
 
@@ -28,6 +29,7 @@ static int run(const GemmProblem &prob, int kind, int epi, hipStream_t stream)
     const int order = g_tile_order.load();
     p.tile_order = order >= 0 ? order : 2;
     p.kernel = order >= 0 ? (int)PATH_TILE : g_kernel.load();
+    p.tiles_192 = g_tiles_192.load();
     p.i8_fp16_step = g_i8_fp16_step.load() != 0;
     const int nto = g_nt_out.load();
     p.nt_out = nto >= 0 ? nto : (kind == KIND_F4);
@@ -90,6 +92,11 @@ int cch_set_option(const char *name, int value)
     if (strcmp(name, "gemm_kernel") == 0) {
         CCH_REQUIRE(value >= -1 && value < NUM_PATHS, "cch_set_option: gemm_kernel %d outside -1..%d", value, NUM_PATHS - 1);
         g_kernel.store(value);
+        return CCH_OK;
+    }
+    if (strcmp(name, "gemm_192_tiles") == 0) {
+        CCH_REQUIRE(value >= -1 && value <= 1, "cch_set_option: gemm_192_tiles %d outside -1..1", value);
+        g_tiles_192.store(value);
         return CCH_OK;
     }
     if (strcmp(name, "routing_three_launches") == 0) {

@@ -62,6 +62,7 @@ struct GemmProblem {
                              // (gemm_tail.h); 0: it takes them all itself
     int nt_out;              // tiled kernels: output stores carry the non-temporal hint
     int kernel;              // which kernel was asked for (GemmPath; tiled kernels only), -1: chosen per problem
+    int tiles_192;           // 192 x 192 tiles: 0 never, 1 wherever there is such a kernel, -1 where they fill the chip (gemm_tile.hip)
     int tile_order;          // tiled kernels: 0 = row-major over (row tile, column tile); 1 = runs of consecutive tiles per XCD;
                              // 2 = a block of 4 row tiles x 8 column tiles per XCD where the shape allows (else 1 for groups, 0 without)
 };

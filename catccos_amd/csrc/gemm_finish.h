@@ -7,9 +7,9 @@
 namespace cch {
 
 // The raw sums v (and, with SwiGLU, those of the up columns) become the eight outputs: dequantisation, activation.  `ch` holds the
-// per-channel factors (SwiGLU: gate columns, then up columns), `tok` the row's per-token factor.
-template <int EPI>
-__device__ __forceinline__ void finish8(float (&v)[8], const float (&up)[8], const float *ch, float tok, bool fp16_step)
+// per-channel factors (SwiGLU: gate columns, then up columns), `tok` the row's per-token factor.  FP16_STEP: GemmProblem::i8_fp16_step.
+template <int EPI, bool FP16_STEP>
+__device__ __forceinline__ void finish8(float (&v)[8], const float (&up)[8], const float *ch, float tok)
 {
     constexpr bool SWIGLU = EPI == EPI_DEQUANT_SWIGLU || EPI == EPI_SWIGLU;
 #pragma unroll
@@ -19,7 +19,7 @@ __device__ __forceinline__ void finish8(float (&v)[8], const float (&up)[8], con
             if constexpr (EPI == EPI_DEQUANT_SWIGLU) {
                 gate *= ch[x];
                 u *= ch[8 + x];
-                if (fp16_step) {
+                if constexpr (FP16_STEP) {
                     // (two roundings, fp32 and then half: the compiler would otherwise fuse product and conversion)
                     asm volatile("" : "+v"(gate), "+v"(u));
                     gate = (float)(_Float16)gate;
@@ -33,7 +33,7 @@ __device__ __forceinline__ void finish8(float (&v)[8], const float (&up)[8], con
             }
             v[x] = gate * __builtin_amdgcn_rcpf(1.0f + __expf(-gate)) * u;
         } else if constexpr (EPI == EPI_DEQUANT) {
-            if (fp16_step) {
+            if constexpr (FP16_STEP) {
                 float prod = v[x] * ch[x];
                 asm volatile("" : "+v"(prod));
                 v[x] = (float)(_Float16)prod * tok;
@@ -46,14 +46,14 @@ __device__ __forceinline__ void finish8(float (&v)[8], const float (&up)[8], con
 
 // Stores the eight outputs at row `row` (of the whole output; `mapped` where a row map redirects it) and columns col .. col+7.
 // MX-quantised output: the four lanes of a quad hold one row's 32 columns, one MX block (all four must call).
-template <int EPI>
+template <int EPI, bool FP16>
 __device__ __forceinline__ void store8(const GemmProblem &p, const float (&v)[8], bool ok, int row, int mapped, int col)
 {
     constexpr bool SWIGLU = EPI == EPI_DEQUANT_SWIGLU || EPI == EPI_SWIGLU;
     uint32_t w[4];
 #pragma unroll
     for (int x = 0; x < 4; x++) {
-        if (p.out_fp16) w[x] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){v[2 * x], v[2 * x + 1]}, f16x2));
+        if constexpr (FP16) w[x] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){v[2 * x], v[2 * x + 1]}, f16x2));
         else w[x] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){v[2 * x], v[2 * x + 1]}, bf16x2));
     }
     if constexpr (SWIGLU) {
@@ -94,6 +94,31 @@ __device__ __forceinline__ void store8(const GemmProblem &p, const float (&v)[8]
         }
     }
     if (ok) *reinterpret_cast<v4u *>(p.out + out_row * p.n_out + col) = (v4u){w[0], w[1], w[2], w[3]};
+}
+
+// Calls f(FP16_STEP, FP16) with what the problem asks for: a branch around the items of a tile instead of twelve inside each (they were
+// a third of a small launch's epilogue).
+template <int EPI, class F>
+__device__ __forceinline__ void with_output_kind(const GemmProblem &p, F &&f)
+{
+    if constexpr (EPI == EPI_DEQUANT || EPI == EPI_DEQUANT_SWIGLU) {
+        if (p.i8_fp16_step) {
+            if (p.out_fp16) f(IC<1>{}, IC<1>{});
+            else f(IC<1>{}, IC<0>{});
+            return;
+        }
+    }
+    if (p.out_fp16) f(IC<0>{}, IC<1>{});
+    else f(IC<0>{}, IC<0>{});
+}
+
+// The arguments that a kernel needs at its start and those that its end needs lie in different lines of memory, and the compiler reads a line
+// where it first needs one: three round trips to a launch's arguments before the first request and another in front of the epilogue.  This
+// reads one word of every line at once; what is read later comes from the scalar cache.
+__device__ __forceinline__ void touch_arguments(const GemmProblem &p)
+{
+    static_assert(sizeof(GemmProblem) <= 256, "four lines");
+    asm volatile("" :: "s"((int)(uintptr_t)p.a), "s"((int)(uintptr_t)p.out_row_map), "s"(p.T), "s"(p.tile_order));
 }
 
 // Where a tile number lies among the groups of a problem.  Every wave finds it by itself from the prefix sums of the group

@@ -7,11 +7,12 @@
 
 namespace cch {
 
-// A tile has 64 * mb rows and 64 * wn columns of B (2 x wn waves).
-constexpr int mid_stage_bytes(int mb, int wn) { return (64 * mb + 64 * wn) * 128; }       // A and B panel of one step
-constexpr int mid_stages(int mb, int wn) { return mb == 2 && wn == 2 ? 2 : 3; }           // of the ring: what two workgroups per CU (wn = 4: one) leave room for
-constexpr int mid_round(int wn) { return wn == 4 ? 256 : 512; }                           // workgroups that run at a time
-constexpr int mid_run(int wn) { return wn == 4 ? 4 : 8; }                                 // column tiles per block of a group's tiles
+// A tile has 64 * mb rows and 32 * jb * wn columns of B (2 x wn waves of 32 * mb x 32 * jb outputs).
+constexpr int mid_cols(int wn, int jb) { return 32 * jb * wn; }
+constexpr int mid_stage_bytes(int mb, int wn, int jb) { return (64 * mb + mid_cols(wn, jb)) * 128; }   // A and B panel of one step
+constexpr int mid_stages(int mb, int wn) { return mb == 2 && wn == 2 ? 2 : 3; }           // of the ring: what two workgroups per CU (the wide tiles: one) leave room for
+constexpr int mid_round(int cols) { return cols > 128 ? 256 : 512; }                      // workgroups that run at a time
+constexpr int mid_run(int cols) { return cols > 128 ? 4 : 8; }                            // column tiles per block of a group's tiles
 // MX: K-steps whose scales one 16-byte fetch per row holds (rows that can start 2 bytes past a dword leave room for the shift),
 // and buffers of them: a group is requested S steps ahead, when the steps of the group it replaces must all have been read
 constexpr int mid_steps_per_scales(int kind, int ua) { return kind == KIND_I8 ? 1 : (ua ? 2 : 4) / (kind == KIND_F4 ? 2 : 1); }

@@ -39,6 +39,7 @@ __global__ __launch_bounds__(W * 64, W == 4 ? 3 : 2) void gemm_stream_kernel(Gem
     constexpr int NSP = MX ? EPB : 0;                            // scale registers per 32 rows or columns and chunk, two K64 blocks each
     constexpr int CBSZ = FMT == CCH_FMT_E2M1 ? 4 : (FMT == CCH_FMT_E5M2 ? 1 : 0);
 
+    touch_arguments(p);
     const int lane = threadIdx.x & 63;
     const int wave = uniform(threadIdx.x >> 6);
     const int r = lane & 31, g = lane >> 5;
@@ -325,17 +326,19 @@ __global__ __launch_bounds__(W * 64, W == 4 ? 3 : 2) void gemm_stream_kernel(Gem
             v[4 + x] = (float)s1[x];
         }
     };
+    with_output_kind<EPI>(p, [&](auto step_c, auto half_c) {
 #pragma unroll
-    for (int it = 0; it < NITEM; it++) {
-        const int item = (int)threadIdx.x + it * W * 64;
-        const int row = item / IPR, lcol = (item % IPR) * 8;
-        if (TM * IPR % (W * 64) != 0 && row >= TM) break;
-        float v[8], up[8] = {};
-        sum8(row, lcol, v);
-        if constexpr (SWIGLU) sum8(row, 32 + lcol, up);
-        finish8<EPI>(v, up, ch, tok[it], p.i8_fp16_step != 0);
-        store8<EPI>(p, v, row < rows && icol + 8 <= p.n_out, m0 + row, mapped[it], icol);
-    }
+        for (int it = 0; it < NITEM; it++) {
+            const int item = (int)threadIdx.x + it * W * 64;
+            const int row = item / IPR, lcol = (item % IPR) * 8;
+            if (TM * IPR % (W * 64) != 0 && row >= TM) break;
+            float v[8], up[8] = {};
+            sum8(row, lcol, v);
+            if constexpr (SWIGLU) sum8(row, 32 + lcol, up);
+            finish8<EPI, decltype(step_c)::value != 0>(v, up, ch, tok[it]);
+            store8<EPI, decltype(half_c)::value != 0>(p, v, row < rows && icol + 8 <= p.n_out, m0 + row, mapped[it], icol);
+        }
+    });
 }
 
 template <int KIND, int EPI, int FMT, int TB, int W>

@@ -209,6 +209,19 @@ static GemmPath choose_path(const GemmProblem &p, int kind, int epi, int cus)
     return path_refuses(p, kind, best) ? PATH_MID2 : best;   // (128 x 256 tiles: the other ones with 128 rows)
 }
 
+// Whether a problem runs on 192 x 192 tiles (gemm_mid_kernel.h; MX kinds, [N, K] weights, no activation), whatever choose_path says: where 128 x 128
+// tiles, two to a CU, make more than one round and 192 x 192 ones at most one.  Measured (us, best other kernel -> this): E4M3 3000 x 1984 x 3000
+// 32.9 -> 28.0, 5484 x 2560 x 1536 34.7 -> 29.9, 1335 x 1088 x 6856 25.9 -> 21.2, 1140 x 4352 x 7448 53 -> 44.5; E2M1 5466 x 5120 x 1528 40.6 -> 32.4.  Where 128 x 128 tiles
+// make one round those are as fast or faster (30 problems of 170 to 240 192 x 192 tiles: 0.85 to 1.02), with more than one round of 192 x 192 ones both are
+// (273 tiles: 22.9 against 15.5), and int8 gains 2 % at most.
+static bool takes_192(const GemmProblem &p, int kind, int epi, int cus)
+{
+    if (kind == KIND_I8 || epi != EPI_PLAIN || !p.trans_b || (kind == KIND_F4 && scales_off_dwords(p, kind))) return false;
+    if (p.tiles_192 >= 0) return p.tiles_192 != 0;
+    auto tiles = [&](int64_t side) { return (p.T + side - 1) / side * ((p.N + side - 1) / side); };
+    return p.kernel < 0 && p.group_sizes == nullptr && tiles(128) > 2 * cus && tiles(192) <= cus;
+}
+
 template <int KIND, int EPI, int FMT>
 static int launch_family(const GemmProblem &p, hipStream_t stream)
 {
@@ -219,6 +232,7 @@ static int launch_family(const GemmProblem &p, hipStream_t stream)
         const char *why = path_refuses(p, KIND, p.kernel);
         if (why) return fail(CCH_ENOSUP, "gemm_kernel %d does not take this problem (T=%d N=%d K=%d trans_b=%d: %s)", p.kernel, p.T, p.N, p.K, p.trans_b, why);
     }
+    if (takes_192(p, KIND, EPI, cus)) return launch_mid_t<KIND, EPI, FMT, 1>(p, 192, 192, stream);
     const GemmPath path = p.kernel >= 0 ? (GemmPath)p.kernel : choose_path(p, KIND, EPI, cus);
     switch (path) {
     case PATH_TILE_TAIL: {

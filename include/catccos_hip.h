@@ -364,6 +364,8 @@ int cch_dyn_quant_i8_rows_smooth(const void *x, const int32_t *src_rows, const f
  * Kernels 0, 1, 2, 3 and 6 add up K in the same order and give the same bits; 4 and 5, which problems of few rows go to, add up K
  * in 4 or 8 parts, also in fp32, which now and then moves the rounding of an MX result.  So by default the last bit of an MX
  * result can depend on how many rows the call has; 0 makes it independent of that (int8 sums are exact on all of them);
+ * "gemm_192_tiles" = 1 / 0 has MX products with [N,K] weights and no activation run on 192 x 192 tiles wherever there is such a kernel (in
+ * front of "gemm_kernel") or never, -1 (default) chooses per problem; the same bits as kernel 0;
  * "i8_epilogue_fp16_step" = 1 makes the int8 epilogues (cch_gemm_i8_dequant*, cch_gmm_i8_dequant*, both kernel paths)
  * round acc * per_channel to IEEE half before the per-token factor, as the reference's device kernel does
  * (include/catccos/epilogue/block/block_epilogue_per_token_dequant_swiglu.hpp:348-361: the matrix unit's output stage
