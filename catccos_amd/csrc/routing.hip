@@ -6,8 +6,9 @@
 // (examples/aux_ops/moe_init_routing_quant_v2/moe_init_routing_quant_v2.h:70-110: sort by expert,
 // MoeV2SrcToDstOp inverts the permutation, MoeV2ExpertTokenOut counts) and its CPU stand-in
 // (examples/utils/gen_data_moe.py:48-57: torch.argsort(stable=True) + bincount).  Keys are small
-// integers, so the sort is a counting sort in three launches: per-chunk histograms, one scan over
-// (expert, chunk), and a placement pass in which four waves walk their quarters of a chunk in order.
+// integers, so the sort is a counting sort: per-chunk histograms, and a placement pass in which four waves
+// walk their quarters of a chunk in order.  Between the two stands a scan over (expert, chunk), in a launch of its own where the
+// chunks are very many; otherwise every workgroup of the placement pass adds up what it needs.
 #include <algorithm>
 #include <atomic>
 
@@ -21,8 +22,9 @@ constexpr int ROUTE_MAX_EXPERTS = 1024;
 // cch_set_option("routing_three_launches", 1): the general path also where one workgroup would do (for tests)
 std::atomic<int> g_route_three_launches{0};
 
-// hist[e * nchunks + c] = rows of chunk c routed to expert e; dst_to_src of the chunk's positions
+// hist[e * nchunks + c] (BY_CHUNK: hist[c * experts + e]) = rows of chunk c routed to expert e; dst_to_src of the chunk's positions
 // is preset to -1 (positions past the routed rows keep it).
+template <bool BY_CHUNK>
 __global__ __launch_bounds__(256) void route_histogram_kernel(const int32_t *__restrict__ expert_idx, int rows, int experts,
                                                               int nchunks, int32_t *__restrict__ hist,
                                                               int32_t *__restrict__ dst_to_src)
@@ -40,7 +42,7 @@ __global__ __launch_bounds__(256) void route_histogram_kernel(const int32_t *__r
         }
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < experts; e += 256) hist[(size_t)e * nchunks + blockIdx.x] = h[e];
+    for (int e = threadIdx.x; e < experts; e += 256) hist[BY_CHUNK ? (size_t)blockIdx.x * experts + e : (size_t)e * nchunks + blockIdx.x] = h[e];
 }
 
 // In-place exclusive scan of hist in (expert, chunk) order: hist[e * nchunks + c] becomes the first
@@ -95,20 +97,43 @@ __global__ __launch_bounds__(1024) void route_scan_kernel(int32_t *__restrict__ 
 // chunk's scanned start) give its first position per expert, and a second walk over the same
 // rows hands the positions out in order.  A wave's LDS accesses execute in program order, so
 // "all lanes read the counter, then the first lane of each key moves it on" needs no barrier.
+//
+// SCANNED: hist holds first positions (route_scan_kernel).  Otherwise it holds the counts by chunk, and the workgroup sums each expert's
+// counts over all chunks and over the chunks before its own; workgroup 0 writes the tokens per expert.
 constexpr int ROUTE_WAVES = 4;
 constexpr int ROUTE_GROUPS = ROUTE_CHUNK / 64 / ROUTE_WAVES;   // groups of 64 rows per wave
+template <bool SCANNED>
 __global__ __launch_bounds__(64 * ROUTE_WAVES) void route_place_kernel(const int32_t *__restrict__ expert_idx, int rows, int experts,
-                                                                      int nchunks, int bits, const int32_t *__restrict__ starts,
+                                                                      int nchunks, int bits, const int32_t *__restrict__ hist,
                                                                       int32_t *__restrict__ dst_to_src,
-                                                                      int32_t *__restrict__ src_to_dst)
+                                                                      int32_t *__restrict__ src_to_dst,
+                                                                      int32_t *__restrict__ expert_tokens, int cumsum)
 {
-    __shared__ int32_t cnt[ROUTE_WAVES][ROUTE_MAX_EXPERTS];
+    constexpr int THREADS = 64 * ROUTE_WAVES, MAX_E = ROUTE_MAX_EXPERTS;
+    __shared__ int32_t cnt[ROUTE_WAVES][MAX_E];
+    __shared__ int32_t total[SCANNED ? 1 : MAX_E], before[SCANNED ? 1 : MAX_E], wave_total[ROUTE_WAVES];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int e = threadIdx.x; e < experts; e += 64 * ROUTE_WAVES) {
+    for (int e = threadIdx.x; e < (SCANNED ? experts : MAX_E); e += THREADS) {
 #pragma unroll
         for (int v = 0; v < ROUTE_WAVES; v++) cnt[v][e] = 0;
+        if constexpr (!SCANNED) total[e] = before[e] = 0;
     }
     __syncthreads();
+    if constexpr (!SCANNED) {
+        // thread t: expert t % span (and those THREADS further on), every parts-th chunk
+        const int span = min(1 << bits, THREADS), parts = THREADS / span, part = threadIdx.x / span;
+        for (int e = threadIdx.x % span; e < experts; e += span) {
+            int all = 0, mine = 0;
+#pragma unroll 8
+            for (int c = part; c < nchunks; c += parts) {
+                const int v = hist[(size_t)c * experts + e];
+                all += v;
+                mine += c < (int)blockIdx.x ? v : 0;
+            }
+            atomicAdd(&total[e], all);
+            atomicAdd(&before[e], mine);
+        }
+    }
     const int base = blockIdx.x * ROUTE_CHUNK + w * (ROUTE_GROUPS * 64);
     const uint64_t below = (1ull << lane) - 1ull;
     int key[ROUTE_GROUPS];
@@ -123,9 +148,34 @@ __global__ __launch_bounds__(64 * ROUTE_WAVES) void route_place_kernel(const int
         if (routed && (same[g] & below) == 0) cnt[w][e] += __popcll(same[g]);   // first lane of its key
     }
     __syncthreads();
+    if constexpr (!SCANNED) {
+        // thread t holds experts 4 t .. 4 t + 3: the totals before each of them, inside the wave and then over the waves
+        constexpr int PER = MAX_E / THREADS;
+        int sum = 0, own[PER];
+#pragma unroll
+        for (int i = 0; i < PER; i++) sum += own[i] = total[threadIdx.x * PER + i];
+        int incl = sum;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int up = __shfl_up(incl, off, 64);
+            if (lane >= off) incl += up;
+        }
+        if (lane == 63) wave_total[w] = incl;
+        __syncthreads();
+        int run = incl - sum;
+        for (int v = 0; v < w; v++) run += wave_total[v];
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            const int e = threadIdx.x * PER + i;
+            before[e] += run;
+            run += own[i];
+            if (blockIdx.x == 0 && e < experts) expert_tokens[e] = cumsum ? run : own[i];
+        }
+        __syncthreads();
+    }
     // counts -> first positions: the chunk's start per expert, then the waves in order
     for (int e = threadIdx.x; e < experts; e += 64 * ROUTE_WAVES) {
-        int run = starts[(size_t)e * nchunks + blockIdx.x];
+        int run = SCANNED ? hist[(size_t)e * nchunks + blockIdx.x] : before[e];
 #pragma unroll
         for (int v = 0; v < ROUTE_WAVES; v++) {
             const int c = cnt[v][e];
@@ -172,9 +222,13 @@ static int route_check(const char *who, const int32_t *expert_idx, int64_t rows,
     return CCH_OK;
 }
 
-// The three launches; hist holds nchunks * num_experts entries, every one of which the histogram
-// pass writes before the scan reads it (nothing has to start at zero).
-
+// hist holds nchunks * num_experts entries, every one of which the histogram pass writes before it is read (nothing has to start at zero).
+// Two launches or three: the placement's sums grow with chunks x chunks x experts, the scan's with chunks x experts on one CU.  Three -> two
+// (graph replays, us): 16384 routes over 16 experts 10.7 -> 7.5, 32768 over 256 26.7 -> 10.0, 131072 over 256 37.5 -> 15.1, 50000 over 1024
+// 75 -> 20, 1048576 (1024 chunks) over 16 24.7 -> 15.5, over 256 194 -> 83; but 4096 chunks over 16 67 -> 78.
+// (One workgroup against two launches: 4096 routes over 16 experts 5.1 and 7.3, over 256 6.5 and 9.0; 8192 over 8 7.4 and 7.2, over 16 7.9 and 7.4,
+// over 256 10.9 and 8.8.  Up to 8192 routes the workgroup stays: calls of that size leave the workspace alone, as their callers may rely on.)
+constexpr int64_t ROUTE_SUM_CHUNKS = 1024;
 static int route_launch(const int32_t *expert_idx, int64_t rows, int num_experts, int64_t nchunks, int32_t *dst_to_src,
                         int32_t *src_to_dst, int32_t *expert_tokens, int cumsum, int32_t *hist, hipStream_t s)
 {
@@ -186,13 +240,15 @@ static int route_launch(const int32_t *expert_idx, int64_t rows, int num_experts
                            expert_tokens, cumsum);
         return launch_status("route kernel");
     }
-    hipLaunchKernelGGL(route_histogram_kernel, dim3((unsigned)nchunks), dim3(256), 0, s, expert_idx, (int)rows, num_experts,
-                       (int)nchunks, hist, dst_to_src);
-    hipLaunchKernelGGL(route_scan_kernel, dim3(1), dim3(1024), 0, s, hist, num_experts, (int)nchunks, expert_tokens, cumsum);
     const int bits = route_key_bits(num_experts);
+    const bool sums = rows > 0 && nchunks <= ROUTE_SUM_CHUNKS && !g_route_three_launches.load(std::memory_order_relaxed);
+    hipLaunchKernelGGL(sums ? route_histogram_kernel<true> : route_histogram_kernel<false>, dim3((unsigned)nchunks), dim3(256), 0, s, expert_idx,
+                       (int)rows, num_experts, (int)nchunks, hist, dst_to_src);
+    if (!sums)
+        hipLaunchKernelGGL(route_scan_kernel, dim3(1), dim3(1024), 0, s, hist, num_experts, (int)nchunks, expert_tokens, cumsum);
     if (rows > 0)
-        hipLaunchKernelGGL(route_place_kernel, dim3((unsigned)nchunks), dim3(64 * ROUTE_WAVES), 0, s, expert_idx, (int)rows,
-                           num_experts, (int)nchunks, bits, hist, dst_to_src, src_to_dst);
+        hipLaunchKernelGGL(sums ? route_place_kernel<false> : route_place_kernel<true>, dim3((unsigned)nchunks), dim3(64 * ROUTE_WAVES), 0, s,
+                           expert_idx, (int)rows, num_experts, (int)nchunks, bits, hist, dst_to_src, src_to_dst, expert_tokens, cumsum);
     return launch_status("route kernels");
 }
 

@@ -64,6 +64,35 @@ def test_routing_one_workgroup_edges(rows, e):
             assert np.array_equal(a, w)
 
 
+@pytest.mark.parametrize("case", [(8193, 9), (8192, 1024), (20000, 1), (33000, 65), (33000, 255), (33000, 256), (33000, 257), (9000, 1023), (1024 * 1024, 3),
+                                  (1024 * 1024 + 1, 3)])
+def test_routing_two_launches(case):
+    """Without the scan's launch every workgroup of the placement pass sums the histograms itself, experts over 256 threads and chunks over what is
+    left: expert counts on either side of a power of two and of 256, the largest, and the last number of chunks before the scan has its own launch again.
+    The result is that of the three launches and the oracle's, for any workspace contents."""
+    rows, e = case
+    rng = np.random.default_rng(rows * 3 + e)
+    idx = rng.integers(-1, e + 1, rows).astype(np.int32)
+    idx[rng.integers(0, rows, 5)] = [2 ** 31 - 1, -2 ** 31, e, -1, 1 << e.bit_length()]
+    L, dev = cc._abi.lib(), torch.from_numpy(idx).cuda()
+    nbytes = L.cch_moe_init_routing_workspace_bytes(rows, e)
+    for cumsum in (0, 1):
+        want = orc.moe_init_routing(idx, e, bool(cumsum))
+        for three, fill in ((0, 0x7FFFFFFF), (0, -7), (1, 5)):
+            cc.set_option("routing_three_launches", three)
+            try:
+                d2s, s2d, cnt = (torch.full((n + 1,), -5, dtype=torch.int32, device="cuda") for n in (rows, rows, e))
+                ws = torch.full((nbytes // 4 + 1,), fill, dtype=torch.int32, device="cuda")
+                cc._abi.check(L.cch_moe_init_routing(dev.data_ptr(), rows, e, d2s.data_ptr(), s2d.data_ptr(), cnt.data_ptr(), cumsum, ws.data_ptr(), nbytes,
+                                                     torch.cuda.current_stream().cuda_stream))
+                torch.cuda.synchronize()
+            finally:
+                cc.set_option("routing_three_launches", 0)
+            for got, w in zip((d2s, s2d, cnt), want):
+                assert int(got[-1]) == -5 and np.array_equal(got[:-1].cpu().numpy(), w)
+            assert int(ws[-1]) == fill
+
+
 def test_routing_skewed_and_sorted_inputs():
     for idx in (np.zeros(5000, np.int32), np.arange(5000, dtype=np.int32) % 7, np.sort(np.arange(5000, dtype=np.int32) % 7)[::-1].copy()):
         d2s, s2d, cnt = cc.moe_init_routing(torch.from_numpy(idx).cuda(), 7)
