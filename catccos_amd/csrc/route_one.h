@@ -1,4 +1,5 @@
-// Routing sort in one workgroup, as a piece of a kernel: the sort's own launch (routing.hip) and the FFN's first one (moe_ffn.hip) run it.
+// Routing sort in one workgroup, as a piece of a kernel: the sort's own launch up to 1024 rows (routing.hip) and the FFN's first one up to
+// 8192 (moe_ffn.hip, beside the quantiser's workgroups) run it.
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -8,7 +8,7 @@
 // (examples/utils/gen_data_moe.py:48-57: torch.argsort(stable=True) + bincount).  Keys are small
 // integers, so the sort is a counting sort: per-chunk histograms, and a placement pass in which four waves
 // walk their quarters of a chunk in order.  Between the two stands a scan over (expert, chunk), in a launch of its own where the
-// chunks are very many; otherwise every workgroup of the placement pass adds up what it needs.
+// chunks are very many; otherwise every workgroup of the placement pass adds up what it needs.  Up to 32768 rows and 256 experts the sort is one launch.
 #include <algorithm>
 #include <atomic>
 
@@ -198,14 +198,90 @@ __global__ __launch_bounds__(64 * ROUTE_WAVES) void route_place_kernel(const int
     }
 }
 
-// Few rows and experts: the whole sort in one workgroup and one launch (route_one.h).
-template <int GROUPS>
+// Up to 1024 rows: the whole sort in one workgroup (route_one.h).
 __global__ __launch_bounds__(64 * ONE_WAVES) void route_one_workgroup_kernel(const int32_t *__restrict__ expert_idx, int rows, int experts,
                                                                             int bits, int32_t *__restrict__ dst_to_src,
                                                                             int32_t *__restrict__ src_to_dst,
                                                                             int32_t *__restrict__ expert_tokens, int cumsum)
 {
-    route_one_workgroup<GROUPS>(expert_idx, rows, experts, bits, dst_to_src, src_to_dst, expert_tokens, cumsum);
+    route_one_workgroup<1>(expert_idx, rows, experts, bits, dst_to_src, src_to_dst, expert_tokens, cumsum);
+}
+
+// 1025 to 32768 rows, of which every workgroup places 1024, still in one launch and without memory of its own: each counts all rows (their keys come
+// from the L2), for its expert totals and for the rows in front of its own, so no workgroup waits for another.  In one workgroup the sort is
+// bound by the ballots that find a row's rank, 40 cycles per key bit and 64 rows; here a workgroup ranks its own rows only and counts the rest with
+// LDS atomics.  Measured against one workgroup (graph replays, us, 16 / 256 experts): 2048 rows 3.8 / 4.5 -> 3.6 / 4.1, 4096 5.1 / 6.5 -> 3.8 / 4.4, 8192
+// 8.0 / 10.9 -> 4.2 / 5.0; against the two launches below: 8200 7.5 / 9.1 -> 4.8 / 5.5, 16384 7.5 / 9.2 -> 5.1 / 5.8, 32768 7.9 / 10.1 -> 6.7 / 7.5.  (All rows
+// counted by ballots: 8192 rows 6.5 / 9.1.)
+constexpr int GROUPS_MAX_ROWS = 32 * 64 * ONE_WAVES;   // 32768: the counts of two halves share a register
+template <int GROUPS>   // of 1024 rows, one to a workgroup
+__global__ __launch_bounds__(64 * ONE_WAVES) void route_groups_kernel(const int32_t *__restrict__ expert_idx, int rows, int experts, int bits,
+                                                                     int32_t *__restrict__ dst_to_src, int32_t *__restrict__ src_to_dst,
+                                                                     int32_t *__restrict__ expert_tokens, int cumsum)
+{
+    __shared__ int32_t own[ONE_WAVES][ONE_MAX_EXPERTS];   // rows of this workgroup by wave, then their first positions
+    // all rows of every sixteenth lane by expert; in the upper half those in front of this workgroup (31744 at most).  Lanes of one wave that hold
+    // one expert meet at four to an address, and a seventeenth counter keeps experts on different banks.
+    constexpr int COPIES = 16, PITCH = COPIES + 1;
+    __shared__ int32_t all[ONE_MAX_EXPERTS * PITCH];
+    __shared__ int32_t wave_total[ONE_MAX_EXPERTS / 64];
+    __shared__ int32_t first[ONE_MAX_EXPERTS];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, group = blockIdx.x;
+    const uint64_t below = (1ull << lane) - 1ull;
+    int key[GROUPS], my_key = -1;
+#pragma unroll
+    for (int g = 0; g < GROUPS; g++) {
+        const int r = g * 64 * ONE_WAVES + (int)threadIdx.x;
+        key[g] = r < rows ? expert_idx[r] : -1;
+    }
+    for (int e = lane; e < ONE_MAX_EXPERTS; e += 64) own[w][e] = 0;   // (the wave's own until the second barrier)
+    for (int i = threadIdx.x; i < experts * PITCH; i += 64 * ONE_WAVES) all[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < GROUPS; g++) {
+        const bool routed = key[g] >= 0 && key[g] < experts;
+        if (routed) atomicAdd(&all[key[g] * PITCH + lane % COPIES], g < group ? 0x10001 : 1);
+        if (g == group) my_key = routed ? key[g] : -1;
+    }
+    const uint64_t my_same = same_key_lanes(my_key, my_key >= 0, bits);
+    if (my_key >= 0 && (my_same & below) == 0) own[w][my_key] = __popcll(my_same);   // first lane of its key
+    __syncthreads();
+    // thread e: expert e's totals, scanned inside each wave, and the first positions of this workgroup's waves
+    int total = 0, incl = 0;
+    if (w < ONE_MAX_EXPERTS / 64) {
+        const int e = threadIdx.x;
+        int sum = 0;
+#pragma unroll
+        for (int v = 0; v < COPIES; v++) sum += e < experts ? all[e * PITCH + v] : 0;
+        total = sum & 0xFFFF;
+        int run = sum >> 16;
+#pragma unroll
+        for (int v = 0; v < ONE_WAVES; v++) {
+            const int c = own[v][e];
+            own[v][e] = run;
+            run += c;
+        }
+        incl = total;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int up = __shfl_up(incl, off, 64);
+            if (lane >= off) incl += up;
+        }
+        if (lane == 63) wave_total[w] = incl;
+        first[e] = incl - total;   // (within its 64 experts)
+    }
+    __syncthreads();
+    int upto[ONE_MAX_EXPERTS / 64 + 1] = {0};
+#pragma unroll
+    for (int v = 0; v < ONE_MAX_EXPERTS / 64; v++) upto[v + 1] = upto[v] + wave_total[v];
+    auto before = [&](int block) { return block == 0 ? upto[0] : block == 1 ? upto[1] : block == 2 ? upto[2] : upto[3]; };
+    if (group == 0 && (int)threadIdx.x < experts) expert_tokens[threadIdx.x] = cumsum ? before(w) + incl : total;
+    const int r = group * 64 * ONE_WAVES + (int)threadIdx.x;
+    if (r >= rows) return;
+    const int pos = my_key >= 0 ? before(my_key >> 6) + first[my_key] + own[w][my_key] + __popcll(my_same & below) : -1;
+    src_to_dst[r] = pos;
+    if (pos >= 0) dst_to_src[pos] = r;
+    if (r >= upto[ONE_MAX_EXPERTS / 64]) dst_to_src[r] = -1;   // (sorted positions past the routed rows hold no row)
 }
 
 // Checks shared by the two entry points; fills nchunks.
@@ -224,19 +300,17 @@ static int route_check(const char *who, const int32_t *expert_idx, int64_t rows,
 
 // hist holds nchunks * num_experts entries, every one of which the histogram pass writes before it is read (nothing has to start at zero).
 // Two launches or three: the placement's sums grow with chunks x chunks x experts, the scan's with chunks x experts on one CU.  Three -> two
-// (graph replays, us): 16384 routes over 16 experts 10.7 -> 7.5, 32768 over 256 26.7 -> 10.0, 131072 over 256 37.5 -> 15.1, 50000 over 1024
-// 75 -> 20, 1048576 (1024 chunks) over 16 24.7 -> 15.5, over 256 194 -> 83; but 4096 chunks over 16 67 -> 78.
-// (One workgroup against two launches: 4096 routes over 16 experts 5.1 and 7.3, over 256 6.5 and 9.0; 8192 over 8 7.4 and 7.2, over 16 7.9 and 7.4,
-// over 256 10.9 and 8.8.  Up to 8192 routes the workgroup stays: calls of that size leave the workspace alone, as their callers may rely on.)
+// (graph replays, us): 32768 routes over 256 experts 26.7 -> 10.0, 131072 over 256 37.5 -> 15.1, 50000 over 1024 75 -> 20, 1048576 (1024 chunks)
+// over 16 24.7 -> 15.5, over 256 194 -> 83; but 4096 chunks over 16 67 -> 78.
 constexpr int64_t ROUTE_SUM_CHUNKS = 1024;
 static int route_launch(const int32_t *expert_idx, int64_t rows, int num_experts, int64_t nchunks, int32_t *dst_to_src,
                         int32_t *src_to_dst, int32_t *expert_tokens, int cumsum, int32_t *hist, hipStream_t s)
 {
-    if (route_fits_one_workgroup(rows, num_experts) && !g_route_three_launches.load(std::memory_order_relaxed)) {
+    if (rows > 0 && rows <= GROUPS_MAX_ROWS && num_experts <= ONE_MAX_EXPERTS && !g_route_three_launches.load(std::memory_order_relaxed)) {
         const int bits = route_key_bits(num_experts), groups = (int)((rows + 64 * ONE_WAVES - 1) / (64 * ONE_WAVES));
-        auto kern = groups <= 1 ? route_one_workgroup_kernel<1> : groups <= 2 ? route_one_workgroup_kernel<2>
-                                                              : groups <= 4 ? route_one_workgroup_kernel<4> : route_one_workgroup_kernel<8>;
-        hipLaunchKernelGGL(kern, dim3(1), dim3(64 * ONE_WAVES), 0, s, expert_idx, (int)rows, num_experts, bits, dst_to_src, src_to_dst,
+        auto kern = groups <= 1 ? route_one_workgroup_kernel : groups <= 2 ? route_groups_kernel<2> : groups <= 4 ? route_groups_kernel<4>
+                          : groups <= 8 ? route_groups_kernel<8> : groups <= 16 ? route_groups_kernel<16> : route_groups_kernel<32>;
+        hipLaunchKernelGGL(kern, dim3((unsigned)groups), dim3(64 * ONE_WAVES), 0, s, expert_idx, (int)rows, num_experts, bits, dst_to_src, src_to_dst,
                            expert_tokens, cumsum);
         return launch_status("route kernel");
     }

@@ -281,7 +281,7 @@ int cch_moe_token_unpermute(const void *permuted_tokens, const int32_t *sorted_i
  *                  operator returns
  *   expert_tokens  int32 [num_experts]: entries per expert, or their running sum with cumsum != 0
  *   workspace      device memory of at least cch_moe_init_routing_workspace_bytes(rows, num_experts)
- * num_experts <= 1024.  Up to 8192 rows and 256 experts the sort is one launch of one workgroup (the
+ * num_experts <= 1024.  Up to 32768 rows and 256 experts the sort is one launch (the
  * workspace is then not touched), two or, from a million rows on, three launches otherwise; the results are the same integers. */
 int64_t cch_moe_init_routing_workspace_bytes(int64_t rows, int num_experts);
 int cch_moe_init_routing(const int32_t *expert_idx, int64_t rows, int num_experts, int32_t *dst_to_src, int32_t *src_to_dst,
@@ -298,7 +298,7 @@ int cch_moe_init_routing(const int32_t *expert_idx, int64_t rows, int num_expert
  *   sharing every call on a GPU uses that GPU's one array: calls that overlap on one GPU (two
  *           streams, two threads) race; calls in stream order do not.  Nothing in the array has to
  *           be cleared between calls (each call writes every entry it later reads).  Inputs that
- *           one workgroup sorts (up to 8192 rows and 256 experts) do not touch the array at all. */
+ *           are sorted in one launch (up to 32768 rows and 256 experts) do not touch the array at all. */
 #define CCH_ROUTING_NOALLOC_MAX_ENTRIES 262144
 int cch_moe_init_routing_noalloc(const int32_t *expert_idx, int64_t rows, int num_experts, int32_t *dst_to_src,
                                  int32_t *src_to_dst, int32_t *expert_tokens, int cumsum, void *stream);

@@ -64,7 +64,29 @@ def test_routing_one_workgroup_edges(rows, e):
             assert np.array_equal(a, w)
 
 
-@pytest.mark.parametrize("case", [(8193, 9), (8192, 1024), (20000, 1), (33000, 65), (33000, 255), (33000, 256), (33000, 257), (9000, 1023), (1024 * 1024, 3),
+@pytest.mark.parametrize("rows", [1025, 2047, 2049, 8193, 16384, 16385, 32767, 32768, 32769])
+@pytest.mark.parametrize("e", [1, 17, 256])
+def test_routing_groups_of_1024(rows, e):
+    """Every workgroup places 1024 rows and counts all others: the row counts on either side of each instantiation, all rows on one expert (the
+    largest counts, and every lane of a wave on the same one) and spread, with dropped routes; nothing is read from or left in the workspace."""
+    L = cc._abi.lib()
+    rng = np.random.default_rng(rows + e)
+    spread = rng.integers(-1, e + 1, rows).astype(np.int32)
+    spread[rng.integers(0, rows, 3)] = [2 ** 31 - 1, -2 ** 31, 256]
+    nbytes = L.cch_moe_init_routing_workspace_bytes(rows, e)
+    for idx in (spread, np.full(rows, e - 1, np.int32), np.full(rows, -1, np.int32)):
+        dev = torch.from_numpy(idx).cuda()
+        for cumsum in (0, 1):
+            d2s, s2d, cnt = (torch.full((n + 1,), -5, dtype=torch.int32, device="cuda") for n in (rows, rows, e))
+            ws = torch.full((nbytes // 4,), 99, dtype=torch.int32, device="cuda")
+            cc._abi.check(L.cch_moe_init_routing(dev.data_ptr(), rows, e, d2s.data_ptr(), s2d.data_ptr(), cnt.data_ptr(), cumsum, ws.data_ptr(), nbytes,
+                                                 torch.cuda.current_stream().cuda_stream))
+            for got, w in zip((d2s, s2d, cnt), orc.moe_init_routing(idx, e, bool(cumsum))):
+                assert int(got[-1]) == -5 and np.array_equal(got[:-1].cpu().numpy(), w)
+            assert rows > 32768 or bool((ws == 99).all())
+
+
+@pytest.mark.parametrize("case", [(1, 257), (8192, 1024), (33000, 1), (33000, 65), (33000, 255), (33000, 256), (33000, 257), (9000, 1023), (1024 * 1024, 3),
                                   (1024 * 1024 + 1, 3)])
 def test_routing_two_launches(case):
     """Without the scan's launch every workgroup of the placement pass sums the histograms itself, experts over 256 threads and chunks over what is
