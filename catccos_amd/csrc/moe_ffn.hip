@@ -12,6 +12,8 @@
 // for itself while its tokens are on their way from memory.  So the first workgroup sorts - for the stages behind - and the others count, quantise and scatter.
 // Whole calls, two launches -> one: 95 tokens to 6 of 8, K 512 26.9 -> 24.6 us, 2 to 6 of 8, K 1280 25.8 -> 23.0, 2000 to 4 of 32, K 1024 66.3 -> 62.4,
 // 512 to 6 of 16, K 7168 291.8 -> 287.5.  (Counting each route's predecessors one by one was slower from 96 routes a workgroup on: 38 us for the first.)
+// The routes are counted with LDS atomics; by ballots over the keys' bits the whole call took, from some thousand routes on, 1 to 4 % longer: 1000 tokens to
+// 8 of 64, K 2048 99.3 -> 96.9 us, 4000 to 2 of 8, K 512 35.0 -> 33.4, 2000 to 4 of 32, K 1024 59.6 -> 58.7; 512 to 6 of 16, K 7168 the same.
 #include <algorithm>
 #include <atomic>
 
@@ -45,6 +47,9 @@ __global__ __launch_bounds__(64 * FFN_WAVES) void moe_dispatch_kernel(const uint
         route_one_workgroup<GROUPS>(expert_idx, rows, experts, bits, dst_to_src, src_to_dst, expert_tokens, 0);
         return;
     }
+    // routes per expert, those of every sixteenth lane; in the upper half those before this workgroup's (8191 at most)
+    constexpr int COPIES = 16, PITCH = COPIES + 1;   // (17: experts on different banks)
+    __shared__ int32_t count[ONE_MAX_EXPERTS * PITCH];
     __shared__ int32_t total[ONE_MAX_EXPERTS], place_of[ONE_MAX_EXPERTS], place[FFN_MAX_ROUTES];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -72,21 +77,19 @@ __global__ __launch_bounds__(64 * FFN_WAVES) void moe_dispatch_kernel(const uint
     int own[2];
 #pragma unroll
     for (int h = 0; h < 2; h++) own[h] = h * 64 + lane < routes ? expert_idx[first + h * 64 + lane] : -1;
-    for (int e = threadIdx.x; e < ONE_MAX_EXPERTS; e += 64 * FFN_WAVES) total[e] = place_of[e] = 0;
+    for (int i = threadIdx.x; i < experts * PITCH; i += 64 * FFN_WAVES) count[i] = 0;
     __syncthreads();
-    // routes per expert, all of them and those before this workgroup's
     const uint64_t below = (1ull << lane) - 1ull;
 #pragma unroll
-    for (int u = 0; u < GROUPS; u++) {
-        const int i = (u * FFN_WAVES + wave) * 64;
-        if (i >= rows) break;   // (wave-uniform)
-        const bool routed = key[u] >= 0 && key[u] < experts;
-        const uint64_t same = same_key_lanes(key[u], routed, bits);
-        if (routed && (same & below) == 0) {
-            const int n = first - i;
-            atomicAdd(&total[key[u]], __builtin_popcountll(same));
-            if (n > 0) atomicAdd(&place_of[key[u]], __builtin_popcountll(n >= 64 ? same : same & ((1ull << n) - 1ull)));
-        }
+    for (int u = 0; u < GROUPS; u++)
+        if (key[u] >= 0 && key[u] < experts) atomicAdd(&count[key[u] * PITCH + lane % COPIES], (u * FFN_WAVES + wave) * 64 + lane < first ? 0x10001 : 1);
+    __syncthreads();
+    for (int e = threadIdx.x; e < ONE_MAX_EXPERTS; e += 64 * FFN_WAVES) {
+        int sum = 0;
+#pragma unroll
+        for (int i = 0; i < COPIES; i++) sum += e < experts ? count[e * PITCH + i] : 0;
+        total[e] = sum & 0xFFFF;
+        place_of[e] = sum >> 16;
     }
     __syncthreads();
     // the place of an expert's first route here: the routes of the experts before it, and its own of earlier workgroups
