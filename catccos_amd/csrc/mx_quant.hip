@@ -202,7 +202,9 @@ __global__ __launch_bounds__(QUANT_THREADS) void mx_quant_rows_kernel(
 // aligned buffers.  Rows of whole pairs of MX blocks lie back to back, payload and scales alike, so the tensor is one run of
 // elements: a wave owns pieces of 1024 consecutive ones (wherever rows begin), keeps its next piece in flight while it converts the current one,
 // stores 16 (FP8) or 8 (FP4) payload bytes per lane and writes the 32 scale bytes as dwords gathered with row shifts.
-// Only the last piece of the run can be partial; nothing else is checked per lane.
+// Only the last piece of the run can be partial; nothing else is checked per lane.  WHOLE: it is not (m * K, with SCATTER K, a multiple of 1024), and the
+// loop carries no second form of its loads and stores: E4M3 4096 x 7168 15.9 us with both forms in the loop, 15.8 without, FP4 4096 x 7168 14.0 and 13.6,
+// FP4 scattered to two rows 4096 x 5120 14.1 and 13.7, E4M3 scattered to one 4096 x 4096 11.3 and 10.9.
 // Bound by HBM where large (4096 x 7168: 5.9 TB/s), by a launch and one load's latency where small.  Against the general kernel, which K no
 // multiple of 1024 took before: 4096 x 6784 17.7 -> 14.9 us, 8192 x 1984 10.9 -> 9.3, 16384 x 1984 to FP4 18.0 -> 14.7, 8192 x 7104 from half
 // 36.9 -> 30.9, 2048 x 3008 5.1 -> 4.0, 64 x 1984 3.0 -> 2.4.
@@ -210,10 +212,10 @@ __global__ __launch_bounds__(QUANT_THREADS) void mx_quant_rows_kernel(
 // own.  `rest` is what the last piece of the run (SCATTER: of each row) holds, a multiple of 64.
 // HALF: the input is IEEE half instead of bf16 (same layout, same stores; the shared exponent comes
 // from the block maximum widened to fp32 and the codes from the packed-half conversions).
-template <int FMT, bool SCATTER = false, bool HALF = false>
+template <int FMT, bool WHOLE, bool SCATTER = false, bool HALF = false>
 __global__ __launch_bounds__(QUANT_THREADS) void mx_quant_rows_fast_kernel(
-    const uint16_t *__restrict__ x, uint8_t *__restrict__ payload, uint8_t *__restrict__ scales, int npairs, int rest, int K = 0, int pitch = 0,
-    int ppr = 1, const int32_t *__restrict__ dst_idx = nullptr, int topk = 1, int out_rows = 0x7FFFFFFF)
+    const uint16_t *__restrict__ x, uint8_t *__restrict__ payload, uint8_t *__restrict__ scales, int npairs, int rest, int K, int pitch,
+    int ppr, const int32_t *__restrict__ dst_idx, int topk, int out_rows)
 {
     constexpr bool FP4 = is_fp4_v<FMT>;
     const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (QUANT_THREADS / 64) + (threadIdx.x >> 6)));
@@ -223,7 +225,7 @@ __global__ __launch_bounds__(QUANT_THREADS) void mx_quant_rows_fast_kernel(
         int row[SCATTER ? QUANT_MAX_TOPK : 1];
     };
     // (all wave-uniform)
-    auto have = [&](int p) { return (SCATTER ? p % ppr == ppr - 1 : p == npairs - 1) ? rest : 1024; };
+    auto have = [&](int p) { return !WHOLE && (SCATTER ? p % ppr == ppr - 1 : p == npairs - 1) ? rest : 1024; };
     auto fetch = [&](int p, u32x4 (&v)[2], Dest &d) {
         const int r = SCATTER ? p / ppr : 0, c = SCATTER ? p - r * ppr : p;  // row, piece of it
         load_piece(x + (size_t)r * K + (size_t)c * 1024, have(p), v);
@@ -277,9 +279,10 @@ static int launch_rows_fast(const void *x, void *payload, void *scales, int64_t 
     CCH_HIP(hipGetDevice(&dev));
     CCH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     const unsigned grid = (unsigned)std::min<int64_t>((npairs + QUANT_THREADS / 64 - 1) / (QUANT_THREADS / 64), (int64_t)cus * QUANT_BLOCKS_PER_CU);
-    hipLaunchKernelGGL((mx_quant_rows_fast_kernel<FMT, false, HALF>), dim3(grid), dim3(QUANT_THREADS), 0, stream,
-                       static_cast<const uint16_t *>(x), static_cast<uint8_t *>(payload), static_cast<uint8_t *>(scales), (int)npairs,
-                       (int)(m * k - (npairs - 1) * 1024));
+    const int rest = (int)(m * k - (npairs - 1) * 1024);
+    auto kern = rest == 1024 ? mx_quant_rows_fast_kernel<FMT, true, false, HALF> : mx_quant_rows_fast_kernel<FMT, false, false, HALF>;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(QUANT_THREADS), 0, stream, static_cast<const uint16_t *>(x), static_cast<uint8_t *>(payload),
+                       static_cast<uint8_t *>(scales), (int)npairs, rest, 0, 0, 1, nullptr, 1, 0);
     return launch_status("mx_quant_rows_fast_kernel");
 }
 
@@ -430,7 +433,8 @@ static int launch_scatter(const void *x, const int32_t *dst_idx, void *packed, i
     if (k % 64 == 0 && aligned(x, 16) && aligned(packed, 16) && row_bytes % 16 == 0 && tokens * ((k + 1023) / 1024) < ((int64_t)1 << 30)) {
         const int64_t ppr = (k + 1023) / 1024, npairs = tokens * ppr;
         const unsigned grid = (unsigned)std::min<int64_t>((npairs + QUANT_THREADS / 64 - 1) / (QUANT_THREADS / 64), max_blocks);
-        hipLaunchKernelGGL((mx_quant_rows_fast_kernel<FMT, true>), dim3(grid), dim3(QUANT_THREADS), 0, stream,
+        auto kern = k % 1024 == 0 ? mx_quant_rows_fast_kernel<FMT, true, true> : mx_quant_rows_fast_kernel<FMT, false, true>;
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(QUANT_THREADS), 0, stream,
                            static_cast<const uint16_t *>(x), out, out + pbytes, (int)npairs, (int)(k - (ppr - 1) * 1024), (int)k, (int)row_bytes,
                            (int)ppr, dst_idx, topk, out_rows);
         return launch_status("mx_quant_rows_fast_kernel (scatter)");

@@ -157,7 +157,7 @@ extern "C" int cch_mx_quant_rows_f16(const void *x, void *payload, void *scales,
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool lut = rounding == CCH_ROUND_LUT;
     if (!lut) {
-        // whole 1024-element pieces per row and aligned buffers: the streaming form shared with the bf16 quantiser
+        // rows of whole pairs of blocks and aligned buffers: the streaming form shared with the bf16 quantiser
         const int rc = mx_quant_rows_fast_half(x, payload, scales, m, k, fmt, s);
         if (rc != 1) return rc;
     }

@@ -51,6 +51,14 @@ def test_scatter_byte_path_and_ragged_k(shape, fmt):
     run_case(tokens, k, topk, fmt, cc.ROUND_RNE, tokens * 3 + k)
 
 
+@pytest.mark.parametrize("fmt", ["e4m3", "e5m2", "e2m1"])
+@pytest.mark.parametrize("shape", [(13, 512, 3), (7, 1536, 2), (5, 2560, 8), (300, 4608, 1)])
+def test_scatter_rows_of_whole_and_partial_pieces(shape, fmt):
+    """Odd multiples of 512 columns: packed rows are whole 16-byte units and a row's last piece of 1024 elements is half full."""
+    tokens, k, topk = shape
+    run_case(tokens, k, topk, fmt, cc.ROUND_RNE, tokens * 7 + k)
+
+
 @pytest.mark.parametrize("fmt", ["e4m3", "e5m2", "e2m1", "e1m2"])
 def test_scatter_lut_rounding(fmt):
     run_case(40, 2048, 2, fmt, cc.ROUND_LUT, 5)
