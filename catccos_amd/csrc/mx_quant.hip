@@ -209,7 +209,11 @@ __global__ __launch_bounds__(QUANT_THREADS) void mx_quant_rows_kernel(
 // multiple of 1024 took before: 4096 x 6784 17.7 -> 14.9 us, 8192 x 1984 10.9 -> 9.3, 16384 x 1984 to FP4 18.0 -> 14.7, 8192 x 7104 from half
 // 36.9 -> 30.9, 2048 x 3008 5.1 -> 4.0, 64 x 1984 3.0 -> 2.4.
 // SCATTER: row r goes to rows dst_idx[r*topk + 0 .. topk-1], `pitch` bytes apart (a multiple of 16); a row is then `ppr` pieces of its
-// own.  `rest` is what the last piece of the run (SCATTER: of each row) holds, a multiple of 64.
+// own.  `rest` is what the last piece of the run (SCATTER: of each row) holds, a multiple of 64.  Rows of whole pieces are stored with the
+// non-temporal hint, others without.  What the hint is worth depends on what the caches still hold, from one size to the next (E4M3, us, hinted and plain:
+// whole 4096 x 7168 to two rows 24.4, 22.4, 8192 x 7168 to two 50.2, 53.2, to eight 141, 160; partial 4096 x 2560 to eight 28.3, 23.0, 16384 x 2560 to two
+// 38.4, 33.3, to four 61.6, 67.2): over 52 sizes of whole pieces the two are equal in the mean, over 28 of
+// partial ones the hint costs 3 %, and at three of them the general kernel, which stores without it, was ahead (4096 x 2560 to eight 27.0).
 // HALF: the input is IEEE half instead of bf16 (same layout, same stores; the shared exponent comes
 // from the block maximum widened to fp32 and the codes from the packed-half conversions).
 template <int FMT, bool WHOLE, bool SCATTER = false, bool HALF = false>
@@ -246,7 +250,7 @@ __global__ __launch_bounds__(QUANT_THREADS) void mx_quant_rows_fast_kernel(
             const int c = p % ppr;
 #pragma unroll
             for (int t = 0; t < QUANT_MAX_TOPK; t++)
-                if (d.row[t] >= 0) store_piece<FMT, true>(o, n, payload + (size_t)d.row[t] * pitch + c * (FP4 ? 512 : 1024), scales + (size_t)d.row[t] * pitch + c * 32);
+                if (d.row[t] >= 0) store_piece<FMT, WHOLE>(o, n, payload + (size_t)d.row[t] * pitch + c * (FP4 ? 512 : 1024), scales + (size_t)d.row[t] * pitch + c * 32);
         } else {
             store_piece<FMT, true>(o, n, payload + (size_t)p * (FP4 ? 512 : 1024), scales + (size_t)p * 32);
         }
@@ -421,16 +425,18 @@ static int launch_scatter(const void *x, const int32_t *dst_idx, void *packed, i
     const int64_t wpr = (nblk * 4 + 63) / 64;
     // Only the loads ask for alignment.  Packed rows are a multiple of 8 bytes for every fourth multiple of 64 columns only, and
     // with byte stores for the others 4096 x 6784 to two rows each took 58.7 us (now 24.7), 512 x 1984 to four 9.1 (5.5), 2 x 7040
-    // to two 5.6 (3.5).  (The stores are without the non-temporal hint, also where rows are aligned: 4096 x 6912 to two 27.9 us, with it
-    // 29.8, 16384 x 2816 to four 77.3 against 84.9, 512 x 6912 to six 9.5 against 10.1, FP4 likewise, none slower.)
+    // to two 5.6 (3.5).  (The general kernel's stores are without the non-temporal hint, also where rows are aligned: 4096 x 6912 to two 27.9 us,
+    // with it 29.8, 16384 x 2816 to four 77.3 against 84.9, 512 x 6912 to six 9.5 against 10.1, FP4 likewise, none slower.)
     const bool vec = (k % 8 == 0) && aligned(x, 16);
     int dev = 0, cus = 0;
     CCH_HIP(hipGetDevice(&dev));
     CCH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     const int64_t max_blocks = (int64_t)cus * QUANT_BLOCKS_PER_CU;
     uint8_t *out = static_cast<uint8_t *>(packed);
+    // (rows of at most half a piece would leave half of every wave idle: 16384 x 512 to two, four and eight rows 13.4, 17.5 and 24.2 us, 12.3, 16.7
+    // and 23.7 in the general kernel)
     if constexpr (HWCVT)
-    if (k % 64 == 0 && aligned(x, 16) && aligned(packed, 16) && row_bytes % 16 == 0 && tokens * ((k + 1023) / 1024) < ((int64_t)1 << 30)) {
+    if (k > 512 && k % 64 == 0 && aligned(x, 16) && aligned(packed, 16) && row_bytes % 16 == 0 && tokens * ((k + 1023) / 1024) < ((int64_t)1 << 30)) {
         const int64_t ppr = (k + 1023) / 1024, npairs = tokens * ppr;
         const unsigned grid = (unsigned)std::min<int64_t>((npairs + QUANT_THREADS / 64 - 1) / (QUANT_THREADS / 64), max_blocks);
         auto kern = k % 1024 == 0 ? mx_quant_rows_fast_kernel<FMT, true, true> : mx_quant_rows_fast_kernel<FMT, false, true>;
