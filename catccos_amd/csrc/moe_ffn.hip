@@ -9,18 +9,18 @@
 //
 // Up to 8192 routes the sort and the quantiser are one launch.  The quantiser needs where its tokens' routes go, which the sort
 // says at its end; but those places are two counts per expert, all routes and the routes of earlier tokens, which a workgroup takes
-// for itself while its tokens are on their way from memory.  So the first workgroup sorts - for the stages behind - and the others count, quantise and scatter.
-// Whole calls, two launches -> one: 95 tokens to 6 of 8, K 512 26.9 -> 24.6 us, 2 to 6 of 8, K 1280 25.8 -> 23.0, 2000 to 4 of 32, K 1024 66.3 -> 62.4,
-// 512 to 6 of 16, K 7168 291.8 -> 287.5.  (Counting each route's predecessors one by one was slower from 96 routes a workgroup on: 38 us for the first.)
-// The routes are counted with LDS atomics; by ballots over the keys' bits the whole call took, from some thousand routes on, 1 to 4 % longer: 1000 tokens to
-// 8 of 64, K 2048 99.3 -> 96.9 us, 4000 to 2 of 8, K 512 35.0 -> 33.4, 2000 to 4 of 32, K 1024 59.6 -> 58.7; 512 to 6 of 16, K 7168 the same.
+// for itself while its tokens are on their way from memory.  Together the workgroups have what the later stages ask of the sort: each
+// writes its routes' places, the first one the tokens per expert.  (With a workgroup of its own that sorted once more beside the others, as one CU can,
+// the launch waited for it, and its registers and LDS cost the others half of their places on a CU from 4097 routes on: 4096 tokens to 2 of 16, K 2048
+// 61.4 -> 54.4 us for the call without it, 8192 to 1 of 256, K 512 48.0 -> 41.4.)
+// The routes are counted with LDS atomics; by ballots over the keys' bits the whole call took, from some thousand routes on, 1 to 4 % longer.
 #include <algorithm>
 #include <atomic>
 
 #include "common.h"
 #include "mx_formats.h"
 #include "mx_quant_block.h"
-#include "route_one.h"
+#include "route_keys.h"
 
 namespace cch {
 
@@ -30,30 +30,26 @@ int quant_scatter(const void *x, const int32_t *expanded_row_idx, void *packed_o
 int mx_gmm_swiglu_mx_rows(const void *packed_a, int64_t row_pitch, const void *b, const void *sb, const int32_t *group_sizes, void *payload, void *scales,
                           int64_t num_experts, int64_t t, int64_t n, int64_t k, int fmt, int trans_b, int out_fmt, void *stream);
 
-constexpr int FFN_WAVES = ONE_WAVES;
+constexpr int FFN_WAVES = 16;
 constexpr int FFN_MAX_TOPK = 8;
-constexpr int FFN_MAX_ROUTES = FFN_WAVES * FFN_MAX_TOPK;   // of one workgroup's tokens
+constexpr int FFN_TOKENS_ROUTES = FFN_WAVES * FFN_MAX_TOPK;   // of one workgroup's tokens
+constexpr int FFN_MAX_GROUPS = 8, FFN_MAX_ROUTES = FFN_MAX_GROUPS * 64 * FFN_WAVES, FFN_MAX_EXPERTS = 256;   // of a call in one launch
 
-// Workgroup 0: the routing sort.  Every other one: `tpw` tokens, of `ppr` pieces of up to 1024 elements each (`rest` in a token's last), a wave
-// to a piece.  For the places of their routes the waves share the list of all routes, GROUPS x 64 entries each.
+// Every workgroup: `tpw` tokens, of `ppr` pieces of up to 1024 elements each (`rest` in a token's last), a wave to a piece.  For the places
+// of their routes the waves share the list of all routes, GROUPS x 64 entries each; the first workgroup also writes the tokens per expert.
 template <int GROUPS>
 __global__ __launch_bounds__(64 * FFN_WAVES) void moe_dispatch_kernel(const uint16_t *__restrict__ x, const int32_t *__restrict__ expert_idx, int tokens, int topk,
-                                                                     int experts, int bits, int32_t *__restrict__ dst_to_src, int32_t *__restrict__ src_to_dst,
-                                                                     int32_t *__restrict__ expert_tokens, uint8_t *__restrict__ packed, int K, int pitch, int ppr,
-                                                                     int rest, int tpw)
+                                                                     int experts, int bits, int32_t *__restrict__ src_to_dst, int32_t *__restrict__ expert_tokens,
+                                                                     uint8_t *__restrict__ packed, int K, int pitch, int ppr, int rest, int tpw)
 {
     const int rows = tokens * topk;
-    if (blockIdx.x == 0) {
-        route_one_workgroup<GROUPS>(expert_idx, rows, experts, bits, dst_to_src, src_to_dst, expert_tokens, 0);
-        return;
-    }
     // routes per expert, those of every sixteenth lane; in the upper half those before this workgroup's (8191 at most)
     constexpr int COPIES = 16, PITCH = COPIES + 1;   // (17: experts on different banks)
-    __shared__ int32_t count[ONE_MAX_EXPERTS * PITCH];
-    __shared__ int32_t total[ONE_MAX_EXPERTS], place_of[ONE_MAX_EXPERTS], place[FFN_MAX_ROUTES];
+    __shared__ int32_t count[FFN_MAX_EXPERTS * PITCH];
+    __shared__ int32_t total[FFN_MAX_EXPERTS], place_of[FFN_MAX_EXPERTS], place[FFN_TOKENS_ROUTES];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int t0 = ((int)blockIdx.x - 1) * tpw, mine = min(tpw, tokens - t0), routes = mine * topk, items = mine * ppr;
+    const int t0 = (int)blockIdx.x * tpw, mine = min(tpw, tokens - t0), routes = mine * topk, items = mine * ppr;
     auto item_of = [&](int i, int &t, int &have) {
         t = i / ppr;
         const int c = i - t * ppr;
@@ -84,21 +80,22 @@ __global__ __launch_bounds__(64 * FFN_WAVES) void moe_dispatch_kernel(const uint
     for (int u = 0; u < GROUPS; u++)
         if (key[u] >= 0 && key[u] < experts) atomicAdd(&count[key[u] * PITCH + lane % COPIES], (u * FFN_WAVES + wave) * 64 + lane < first ? 0x10001 : 1);
     __syncthreads();
-    for (int e = threadIdx.x; e < ONE_MAX_EXPERTS; e += 64 * FFN_WAVES) {
+    for (int e = threadIdx.x; e < FFN_MAX_EXPERTS; e += 64 * FFN_WAVES) {
         int sum = 0;
 #pragma unroll
         for (int i = 0; i < COPIES; i++) sum += e < experts ? count[e * PITCH + i] : 0;
         total[e] = sum & 0xFFFF;
         place_of[e] = sum >> 16;
+        if (blockIdx.x == 0 && e < experts) expert_tokens[e] = sum & 0xFFFF;
     }
     __syncthreads();
     // the place of an expert's first route here: the routes of the experts before it, and its own of earlier workgroups
     if (wave == 0) {
-        int sum = 0, part[ONE_MAX_EXPERTS / 64];
+        int sum = 0, part[FFN_MAX_EXPERTS / 64];
 #pragma unroll
-        for (int v = 0; v < ONE_MAX_EXPERTS / 64; v++) {
+        for (int v = 0; v < FFN_MAX_EXPERTS / 64; v++) {
             part[v] = sum;
-            sum += total[lane * (ONE_MAX_EXPERTS / 64) + v];
+            sum += total[lane * (FFN_MAX_EXPERTS / 64) + v];
         }
         int incl = sum;
 #pragma unroll
@@ -107,7 +104,7 @@ __global__ __launch_bounds__(64 * FFN_WAVES) void moe_dispatch_kernel(const uint
             if (lane >= off) incl += up;
         }
 #pragma unroll
-        for (int v = 0; v < ONE_MAX_EXPERTS / 64; v++) place_of[lane * (ONE_MAX_EXPERTS / 64) + v] += incl - sum + part[v];
+        for (int v = 0; v < FFN_MAX_EXPERTS / 64; v++) place_of[lane * (FFN_MAX_EXPERTS / 64) + v] += incl - sum + part[v];
         // (one wave's LDS accesses execute in program order)
 #pragma unroll
         for (int h = 0; h < 2; h++) {
@@ -118,6 +115,7 @@ __global__ __launch_bounds__(64 * FFN_WAVES) void moe_dispatch_kernel(const uint
             if (routed) at = place_of[own[h]] + __builtin_popcountll(same & below);
             if (routed && (same & below) == 0) place_of[own[h]] += __builtin_popcountll(same);
             place[h * 64 + lane] = at;
+            if (h * 64 + lane < routes) src_to_dst[first + h * 64 + lane] = at;
         }
     }
     __syncthreads();
@@ -148,17 +146,18 @@ static int64_t ffn_pitch(int64_t rows, int64_t k)
 static int ffn_dispatch(const void *x, const int32_t *expert_idx, int64_t m, int64_t k, int top_k, int experts, int32_t *dst_to_src, int32_t *src_to_dst,
                         int32_t *expert_tokens, void *packed, int64_t pitch, void *route_ws, int64_t route_bytes, void *stream)
 {
-    const int64_t rows = m * top_k;
-    if (!(route_fits_one_workgroup(rows, experts) && top_k <= FFN_MAX_TOPK && k % 64 == 0 && pitch % 16 == 0 && aligned(x, 16) && aligned(packed, 16)) ||
-        g_route_three_launches.load(std::memory_order_relaxed)) {
+    const int64_t rows = m * top_k, ppr = (k + 1023) / 1024, tpw = std::max<int64_t>(1, FFN_WAVES / ppr), workgroups = (m + tpw - 1) / tpw;
+    const bool one_launch = rows <= FFN_MAX_ROUTES && experts <= FFN_MAX_EXPERTS && top_k <= FFN_MAX_TOPK &&
+                            k % 64 == 0 && pitch % 16 == 0 && aligned(x, 16) && aligned(packed, 16) && !g_route_three_launches.load(std::memory_order_relaxed);
+    if (!one_launch) {
         const int rc = cch_moe_init_routing(expert_idx, rows, experts, dst_to_src, src_to_dst, expert_tokens, 0, route_ws, route_bytes, stream);
         return rc ? rc : quant_scatter(x, src_to_dst, packed, rows, pitch, m, k, top_k, CCH_FMT_E4M3, CCH_ROUND_RNE, stream);
     }
-    const int groups = (int)((rows + 64 * ONE_WAVES - 1) / (64 * ONE_WAVES)), ppr = (int)((k + 1023) / 1024), tpw = std::max(1, FFN_WAVES / ppr);
+    const int groups = (int)((rows + 64 * FFN_WAVES - 1) / (64 * FFN_WAVES));
     auto kern = groups <= 1 ? moe_dispatch_kernel<1> : groups <= 2 ? moe_dispatch_kernel<2> : groups <= 4 ? moe_dispatch_kernel<4> : moe_dispatch_kernel<8>;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(1 + (m + tpw - 1) / tpw)), dim3(64 * FFN_WAVES), 0, static_cast<hipStream_t>(stream),
-                       static_cast<const uint16_t *>(x), expert_idx, (int)m, top_k, experts, route_key_bits(experts), dst_to_src, src_to_dst, expert_tokens,
-                       static_cast<uint8_t *>(packed), (int)k, (int)pitch, ppr, (int)(k - (ppr - 1) * 1024), tpw);
+    hipLaunchKernelGGL(kern, dim3((unsigned)workgroups), dim3(64 * FFN_WAVES), 0, static_cast<hipStream_t>(stream),
+                       static_cast<const uint16_t *>(x), expert_idx, (int)m, top_k, experts, route_key_bits(experts), src_to_dst, expert_tokens,
+                       static_cast<uint8_t *>(packed), (int)k, (int)pitch, (int)ppr, (int)(k - (ppr - 1) * 1024), (int)tpw);
     return launch_status("moe_dispatch_kernel");
 }
 

@@ -13,7 +13,7 @@
 #include <atomic>
 
 #include "common.h"
-#include "route_one.h"
+#include "route_keys.h"
 
 namespace cch {
 
@@ -198,13 +198,64 @@ __global__ __launch_bounds__(64 * ROUTE_WAVES) void route_place_kernel(const int
     }
 }
 
-// Up to 1024 rows: the whole sort in one workgroup (route_one.h).
+// Up to 1024 rows (a decode step's routes): the whole sort in one workgroup.  Sixteen waves hold a row per lane, exactly like
+// the waves of the placement pass above; the per-wave counts per expert meet in LDS, thread e scans expert e's counts over the waves,
+// the experts' totals are scanned across the workgroup, and every lane finds its position.  No workspace.
+//
+// What counts here are chains of latencies and the stores' addresses: all keys are requested before anything is looked at, the totals are
+// scanned inside waves (three barriers in all, where a scan over LDS took sixteen), and dst_to_src is put together in LDS and leaves in
+// order (a wave's 64 scattered stores are 64 lines).  Measured (before -> now): 24 and 384 routes 3.2 -> 2.4 us, 1024 over 64 experts 3.9 -> 2.8.
+constexpr int ONE_WAVES = 16, ONE_MAX_EXPERTS = 256;
 __global__ __launch_bounds__(64 * ONE_WAVES) void route_one_workgroup_kernel(const int32_t *__restrict__ expert_idx, int rows, int experts,
                                                                             int bits, int32_t *__restrict__ dst_to_src,
                                                                             int32_t *__restrict__ src_to_dst,
                                                                             int32_t *__restrict__ expert_tokens, int cumsum)
 {
-    route_one_workgroup<1>(expert_idx, rows, experts, bits, dst_to_src, src_to_dst, expert_tokens, cumsum);
+    __shared__ int32_t cnt[ONE_WAVES][ONE_MAX_EXPERTS];
+    __shared__ int32_t sorted[ONE_WAVES * 64];
+    __shared__ int32_t wave_total[ONE_MAX_EXPERTS / 64];
+    __shared__ int32_t first[ONE_MAX_EXPERTS];   // sorted position of an expert's first row
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = threadIdx.x;
+    const uint64_t below = (1ull << lane) - 1ull;
+    int key = r < rows ? expert_idx[r] : -1;
+    // a wave's own counters: it alone touches them until the first barrier
+    for (int e = lane; e < ONE_MAX_EXPERTS; e += 64) cnt[w][e] = 0;
+    if (key >= experts) key = -1;
+    const uint64_t same = same_key_lanes(key, key >= 0, bits);
+    if (key >= 0 && (same & below) == 0) cnt[w][key] = __popcll(same);   // first lane of its key
+    __syncthreads();
+    // thread e: expert e's counts over the waves -> exclusive running sums; the totals scanned inside each wave
+    int total = 0, incl = 0;
+    if (w < ONE_MAX_EXPERTS / 64) {
+        const int e = threadIdx.x;
+#pragma unroll
+        for (int v = 0; v < ONE_WAVES; v++) {
+            const int c = cnt[v][e];
+            cnt[v][e] = total;
+            total += c;
+        }
+        incl = total;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int up = __shfl_up(incl, off, 64);
+            if (lane >= off) incl += up;
+        }
+        if (lane == 63) wave_total[w] = incl;
+        first[e] = incl - total;   // (within its 64 experts)
+    }
+    __syncthreads();
+    int upto[ONE_MAX_EXPERTS / 64 + 1] = {0};
+#pragma unroll
+    for (int v = 0; v < ONE_MAX_EXPERTS / 64; v++) upto[v + 1] = upto[v] + wave_total[v];
+    auto before = [&](int block) { return block == 0 ? upto[0] : block == 1 ? upto[1] : block == 2 ? upto[2] : upto[3]; };
+    if ((int)threadIdx.x < experts) expert_tokens[threadIdx.x] = cumsum ? before(w) + incl : total;
+    const int routed_rows = upto[ONE_MAX_EXPERTS / 64];
+    const int pos = key >= 0 ? before(key >> 6) + first[key] + cnt[w][key] + __popcll(same & below) : -1;
+    if (r < rows) src_to_dst[r] = pos;
+    if (pos >= 0) sorted[pos] = r;
+    __syncthreads();
+    // (sorted positions past the routed rows hold no row)
+    if (r < rows) dst_to_src[r] = r < routed_rows ? sorted[r] : -1;
 }
 
 // 1025 to 32768 rows, of which every workgroup places 1024, still in one launch and without memory of its own: each counts all rows (their keys come

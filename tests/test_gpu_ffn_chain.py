@@ -96,9 +96,9 @@ def test_ffn_chain_against_oracle_chain(cfg):
     (1, 64, 128, 1, 1, False),         # one route, one piece of one pair of blocks
     (37, 960, 256, 3, 2, True),        # K an odd multiple of 64, dropped entries of either sign
     (129, 1984, 128, 8, 8, True),      # 1032 routes: two groups of keys per wave; eight tokens per workgroup
-    (300, 1088, 256, 256, 7, False),   # 2100 routes, as many experts as one workgroup sorts
+    (300, 1088, 256, 256, 7, False),   # 2100 routes, as many experts as one launch takes
     (515, 512, 128, 5, 8, True),       # 4120 routes, sixteen tokens and all 128 route places of a workgroup
-    (1024, 64, 128, 4, 8, False),      # 8192 routes: the most that one workgroup sorts
+    (1024, 64, 128, 4, 8, False),      # 8192 routes: the most that one launch takes
     (1025, 192, 128, 4, 8, True),      # one token more: the sort's own launches
     (5, 17472, 128, 2, 2, False),      # 18 pieces a token, more than a workgroup's waves
     (6, 512, 128, 257, 3, True),       # more experts than MAX: refused
