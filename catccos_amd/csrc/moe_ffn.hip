@@ -7,13 +7,19 @@
 // multiple of 4 bytes where K is an odd multiple of 64, and then went to the one-thread-per-element GEMM (45 tokens to 6 of 16 experts, K 4160, N 512:
 // 6.2 ms for the call, now 0.037; 300 to 8 of 8, K 1984, N 1024: 12.2 ms, now 0.043).
 //
-// Up to 8192 routes the sort and the quantiser are one launch.  The quantiser needs where its tokens' routes go, which the sort
+// Where the routes are few enough the sort and the quantiser are one launch.  The quantiser needs where its tokens' routes go, which the sort
 // says at its end; but those places are two counts per expert, all routes and the routes of earlier tokens, which a workgroup takes
 // for itself while its tokens are on their way from memory.  Together the workgroups have what the later stages ask of the sort: each
 // writes its routes' places, the first one the tokens per expert.  (With a workgroup of its own that sorted once more beside the others, as one CU can,
 // the launch waited for it, and its registers and LDS cost the others half of their places on a CU from 4097 routes on: 4096 tokens to 2 of 16, K 2048
 // 61.4 -> 54.4 us for the call without it, 8192 to 1 of 256, K 512 48.0 -> 41.4.)
 // The routes are counted with LDS atomics; by ballots over the keys' bits the whole call took, from some thousand routes on, 1 to 4 % longer.
+//
+// The rule: up to FFN_MAX_COUNTED routes looked at by all workgroups together.  Each looks at all routes, and there are the more of them the longer
+// tokens are.  Whole calls, two launches -> one (us, n 256 or 512): 256 to 1 of 64, K 512 18.4 -> 17.2, 1500 to 2 of 64, K 2048 37.9 -> 36.2, 512 to 8 of 64,
+// K 7168 94.3 -> 92.5 (1.0 M looked at), 1024 to 8 of 64, K 8192 171 -> 167 (4.2 M), 2048 to 4 of 64, K 8192 178.7 -> 171.7, 2048 to 4 of 8, K 8192 173 -> 159 and
+// 4096 to 1 of 16, K 7168 103 -> 101 (8.4 M each); but 8192 to 1 of 16, K 4096 102 -> 106 (16.8 M), 8192 to 1 of 64, K 7168 192 -> 204 and 8192 to 1 of 64,
+// K 8192 211 -> 220 (33 M).
 #include <algorithm>
 #include <atomic>
 
@@ -34,6 +40,7 @@ constexpr int FFN_WAVES = 16;
 constexpr int FFN_MAX_TOPK = 8;
 constexpr int FFN_TOKENS_ROUTES = FFN_WAVES * FFN_MAX_TOPK;   // of one workgroup's tokens
 constexpr int FFN_MAX_GROUPS = 8, FFN_MAX_ROUTES = FFN_MAX_GROUPS * 64 * FFN_WAVES, FFN_MAX_EXPERTS = 256;   // of a call in one launch
+constexpr int64_t FFN_MAX_COUNTED = (int64_t)1 << 23;
 
 // Every workgroup: `tpw` tokens, of `ppr` pieces of up to 1024 elements each (`rest` in a token's last), a wave to a piece.  For the places
 // of their routes the waves share the list of all routes, GROUPS x 64 entries each; the first workgroup also writes the tokens per expert.
@@ -147,7 +154,7 @@ static int ffn_dispatch(const void *x, const int32_t *expert_idx, int64_t m, int
                         int32_t *expert_tokens, void *packed, int64_t pitch, void *route_ws, int64_t route_bytes, void *stream)
 {
     const int64_t rows = m * top_k, ppr = (k + 1023) / 1024, tpw = std::max<int64_t>(1, FFN_WAVES / ppr), workgroups = (m + tpw - 1) / tpw;
-    const bool one_launch = rows <= FFN_MAX_ROUTES && experts <= FFN_MAX_EXPERTS && top_k <= FFN_MAX_TOPK &&
+    const bool one_launch = rows <= FFN_MAX_ROUTES && workgroups * rows <= FFN_MAX_COUNTED && experts <= FFN_MAX_EXPERTS && top_k <= FFN_MAX_TOPK &&
                             k % 64 == 0 && pitch % 16 == 0 && aligned(x, 16) && aligned(packed, 16) && !g_route_three_launches.load(std::memory_order_relaxed);
     if (!one_launch) {
         const int rc = cch_moe_init_routing(expert_idx, rows, experts, dst_to_src, src_to_dst, expert_tokens, 0, route_ws, route_bytes, stream);

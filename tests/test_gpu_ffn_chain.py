@@ -100,6 +100,9 @@ def test_ffn_chain_against_oracle_chain(cfg):
     (515, 512, 128, 5, 8, True),       # 4120 routes, sixteen tokens and all 128 route places of a workgroup
     (1024, 64, 128, 4, 8, False),      # 8192 routes: the most that one launch takes
     (1025, 192, 128, 4, 8, True),      # one token more: the sort's own launches
+    (8192, 64, 128, 5, 1, True),       # 8192 routes to one expert each
+    (5016, 4160, 128, 5, 1, True),     # 1672 workgroups of three tokens of five pieces look at 5016 routes: 2^23 in all but for some
+    (5019, 4160, 128, 5, 1, True),     # and 1673 at 5019, more: two launches
     (5, 17472, 128, 2, 2, False),      # 18 pieces a token, more than a workgroup's waves
     (6, 512, 128, 257, 3, True),       # more experts than MAX: refused
 ])
