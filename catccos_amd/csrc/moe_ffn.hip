@@ -20,6 +20,10 @@
 // K 7168 94.3 -> 92.5 (1.0 M looked at), 1024 to 8 of 64, K 8192 171 -> 167 (4.2 M), 2048 to 4 of 64, K 8192 178.7 -> 171.7, 2048 to 4 of 8, K 8192 173 -> 159 and
 // 4096 to 1 of 16, K 7168 103 -> 101 (8.4 M each); but 8192 to 1 of 16, K 4096 102 -> 106 (16.8 M), 8192 to 1 of 64, K 7168 192 -> 204 and 8192 to 1 of 64,
 // K 8192 211 -> 220 (33 M).
+//
+// Packed rows are stored with the non-temporal hint where the weights are more than the caches hold (FFN_CACHED_WEIGHTS), as the quantiser's own launch
+// stores them: 3000 to 1 of 256, K 7168, n 256 302 us without, 288 with it, 512 to 6 of 16, K 7168, n 4096 225 and 215.  Where the weights stay in the caches
+// the rows had better do so too: 512 to 6 of 16, K 7168, n 512 70.5 without, 75 with it, 2048 to 1 of 64, K 7168, n 256 86.7 and 90.3.
 #include <algorithm>
 #include <atomic>
 
@@ -41,10 +45,11 @@ constexpr int FFN_MAX_TOPK = 8;
 constexpr int FFN_TOKENS_ROUTES = FFN_WAVES * FFN_MAX_TOPK;   // of one workgroup's tokens
 constexpr int FFN_MAX_GROUPS = 8, FFN_MAX_ROUTES = FFN_MAX_GROUPS * 64 * FFN_WAVES, FFN_MAX_EXPERTS = 256;   // of a call in one launch
 constexpr int64_t FFN_MAX_COUNTED = (int64_t)1 << 23;
+constexpr double FFN_CACHED_WEIGHTS = 256e6;
 
 // Every workgroup: `tpw` tokens, of `ppr` pieces of up to 1024 elements each (`rest` in a token's last), a wave to a piece.  For the places
 // of their routes the waves share the list of all routes, GROUPS x 64 entries each; the first workgroup also writes the tokens per expert.
-template <int GROUPS>
+template <int GROUPS, bool HINT>
 __global__ __launch_bounds__(64 * FFN_WAVES) void moe_dispatch_kernel(const uint16_t *__restrict__ x, const int32_t *__restrict__ expert_idx, int tokens, int topk,
                                                                      int experts, int bits, int32_t *__restrict__ src_to_dst, int32_t *__restrict__ expert_tokens,
                                                                      uint8_t *__restrict__ packed, int K, int pitch, int ppr, int rest, int tpw)
@@ -138,7 +143,7 @@ __global__ __launch_bounds__(64 * FFN_WAVES) void moe_dispatch_kernel(const uint
             const int at = __builtin_amdgcn_readfirstlane(place[t * topk + j]);
             if (at < 0) continue;
             uint8_t *row = packed + (size_t)at * pitch;
-            store_piece<CCH_FMT_E4M3, false>(o, have, row + c * 1024, row + K + c * 32);
+            store_piece<CCH_FMT_E4M3, HINT>(o, have, row + c * 1024, row + K + c * 32);
         }
     }
 }
@@ -151,7 +156,7 @@ static int64_t ffn_pitch(int64_t rows, int64_t k)
 }
 
 static int ffn_dispatch(const void *x, const int32_t *expert_idx, int64_t m, int64_t k, int top_k, int experts, int32_t *dst_to_src, int32_t *src_to_dst,
-                        int32_t *expert_tokens, void *packed, int64_t pitch, void *route_ws, int64_t route_bytes, void *stream)
+                        int32_t *expert_tokens, void *packed, int64_t pitch, int64_t n, void *route_ws, int64_t route_bytes, void *stream)
 {
     const int64_t rows = m * top_k, ppr = (k + 1023) / 1024, tpw = std::max<int64_t>(1, FFN_WAVES / ppr), workgroups = (m + tpw - 1) / tpw;
     const bool one_launch = rows <= FFN_MAX_ROUTES && workgroups * rows <= FFN_MAX_COUNTED && experts <= FFN_MAX_EXPERTS && top_k <= FFN_MAX_TOPK &&
@@ -161,7 +166,11 @@ static int ffn_dispatch(const void *x, const int32_t *expert_idx, int64_t m, int
         return rc ? rc : quant_scatter(x, src_to_dst, packed, rows, pitch, m, k, top_k, CCH_FMT_E4M3, CCH_ROUND_RNE, stream);
     }
     const int groups = (int)((rows + 64 * FFN_WAVES - 1) / (64 * FFN_WAVES));
-    auto kern = groups <= 1 ? moe_dispatch_kernel<1> : groups <= 2 ? moe_dispatch_kernel<2> : groups <= 4 ? moe_dispatch_kernel<4> : moe_dispatch_kernel<8>;
+    const bool hint = 1.5 * (double)k * (double)n * experts > FFN_CACHED_WEIGHTS;   // (the down projection has half as many as the up projection)
+    auto kern = groups <= 1   ? (hint ? moe_dispatch_kernel<1, true> : moe_dispatch_kernel<1, false>)
+                : groups <= 2 ? (hint ? moe_dispatch_kernel<2, true> : moe_dispatch_kernel<2, false>)
+                : groups <= 4 ? (hint ? moe_dispatch_kernel<4, true> : moe_dispatch_kernel<4, false>)
+                              : (hint ? moe_dispatch_kernel<8, true> : moe_dispatch_kernel<8, false>);
     hipLaunchKernelGGL(kern, dim3((unsigned)workgroups), dim3(64 * FFN_WAVES), 0, static_cast<hipStream_t>(stream),
                        static_cast<const uint16_t *>(x), expert_idx, (int)m, top_k, experts, route_key_bits(experts), src_to_dst, expert_tokens,
                        static_cast<uint8_t *>(packed), (int)k, (int)pitch, (int)ppr, (int)(k - (ppr - 1) * 1024), (int)tpw);
@@ -220,7 +229,7 @@ extern "C" int cch_moe_ffn_mxfp8(const void *x, const int32_t *expert_idx, const
     uint8_t *p = static_cast<uint8_t *>(workspace);
     int32_t *s2d = reinterpret_cast<int32_t *>(p + w.s2d), *cnt = reinterpret_cast<int32_t *>(p + w.cnt);
     const int64_t pitch = ffn_pitch(rows, k);
-    int rc = ffn_dispatch(x, expert_idx, m, k, top_k, (int)num_experts, reinterpret_cast<int32_t *>(p + w.d2s), s2d, cnt, p + w.packed, pitch, p + w.route,
+    int rc = ffn_dispatch(x, expert_idx, m, k, top_k, (int)num_experts, reinterpret_cast<int32_t *>(p + w.d2s), s2d, cnt, p + w.packed, pitch, n, p + w.route,
                           w.route_bytes, stream);
     if (rc == CCH_OK)
         rc = mx_gmm_swiglu_mx_rows(p + w.packed, pitch, w1, sw1, cnt, p + w.act, p + w.scales, num_experts, rows, n, k, CCH_FMT_E4M3, trans_b, CCH_FMT_E4M3, stream);

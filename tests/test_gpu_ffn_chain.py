@@ -103,6 +103,8 @@ def test_ffn_chain_against_oracle_chain(cfg):
     (8192, 64, 128, 5, 1, True),       # 8192 routes to one expert each
     (5016, 4160, 128, 5, 1, True),     # 1672 workgroups of three tokens of five pieces look at 5016 routes: 2^23 in all but for some
     (5019, 4160, 128, 5, 1, True),     # and 1673 at 5019, more: two launches
+    (70, 2048, 1024, 96, 4, True),     # more weights than the caches hold: rows of whole pieces are stored with the non-temporal hint
+    (70, 1984, 1024, 96, 4, True),     # and of partial ones
     (5, 17472, 128, 2, 2, False),      # 18 pieces a token, more than a workgroup's waves
     (6, 512, 128, 257, 3, True),       # more experts than MAX: refused
 ])
