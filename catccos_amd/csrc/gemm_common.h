@@ -16,9 +16,10 @@ enum GemmKind { KIND_I8 = 0, KIND_F8 = 1, KIND_F4 = 2 };
 enum GemmEpilogue { EPI_PLAIN = 0, EPI_DEQUANT = 1, EPI_DEQUANT_SWIGLU = 2, EPI_SWIGLU = 3 };
 
 // The tiled MFMA kernels, numbered as the switch "gemm_kernel" names them: 256 x 256 tiles (gemm_tile_kernel.h), 64 x 128, 128 x 128 and
-// 128 x 256 tiles (gemm_mid_kernel.h), tiles of 32 x 64 whose 4 or 8 waves split K (gemm_stream_kernel.h), and 256 x 256 tiles with
-// a second launch of 64 x 128 ones for a grouped problem's last round (gemm_tail.h).
-enum GemmPath { PATH_TILE, PATH_MID1, PATH_MID2, PATH_MID3, PATH_STREAM4, PATH_STREAM8, NUM_KERNELS, PATH_TILE_TAIL = NUM_KERNELS, NUM_PATHS };
+// 128 x 256 tiles (gemm_mid_kernel.h), tiles of 32 x 64 whose 4 or 8 waves split K (gemm_stream_kernel.h), 256 x 256 tiles with
+// a second launch of 64 x 128 ones for a grouped problem's last round (gemm_tail.h); and 192 x 192 tiles (gemm_mid_kernel.h), which have a
+// switch of their own, "gemm_192_tiles".
+enum GemmPath { PATH_TILE, PATH_MID1, PATH_MID2, PATH_MID3, PATH_STREAM4, PATH_STREAM8, NUM_KERNELS, PATH_TILE_TAIL = NUM_KERNELS, NUM_PATHS, PATH_MID192 = NUM_PATHS };
 
 constexpr int MAX_GROUPS = 256;
 constexpr int TAIL_TILES = 256;   // most tiles that the second launch of a grouped problem may have (gemm_tail.h): one to a CU

@@ -222,6 +222,13 @@ static bool takes_192(const GemmProblem &p, int kind, int epi, int cus)
     return p.kernel < 0 && p.group_sizes == nullptr && tiles(128) > 2 * cus && tiles(192) <= cus;
 }
 
+// The kernel that a problem runs on; one that "gemm_kernel" names has passed path_refuses().
+static GemmPath path_of(const GemmProblem &p, int kind, int epi, int cus)
+{
+    if (takes_192(p, kind, epi, cus)) return PATH_MID192;
+    return p.kernel >= 0 ? (GemmPath)p.kernel : choose_path(p, kind, epi, cus);
+}
+
 template <int KIND, int EPI, int FMT>
 static int launch_family(const GemmProblem &p, hipStream_t stream)
 {
@@ -232,8 +239,7 @@ static int launch_family(const GemmProblem &p, hipStream_t stream)
         const char *why = path_refuses(p, KIND, p.kernel);
         if (why) return fail(CCH_ENOSUP, "gemm_kernel %d does not take this problem (T=%d N=%d K=%d trans_b=%d: %s)", p.kernel, p.T, p.N, p.K, p.trans_b, why);
     }
-    if (takes_192(p, KIND, EPI, cus)) return launch_mid_t<KIND, EPI, FMT, 1>(p, 192, 192, stream);
-    const GemmPath path = p.kernel >= 0 ? (GemmPath)p.kernel : choose_path(p, KIND, EPI, cus);
+    const GemmPath path = path_of(p, KIND, EPI, cus);
     switch (path) {
     case PATH_TILE_TAIL: {
         GemmProblem q = p;
@@ -248,6 +254,7 @@ static int launch_family(const GemmProblem &p, hipStream_t stream)
         const int rows = PATH_MODEL[path].tm, cols = PATH_MODEL[path].tn;
         return p.trans_b ? launch_mid_t<KIND, EPI, FMT, 1>(p, rows, cols, stream) : launch_mid_t<KIND, EPI, FMT, 0>(p, rows, cols, stream);
     }
+    case PATH_MID192: return launch_mid_t<KIND, EPI, FMT, 1>(p, 192, 192, stream);
     case PATH_STREAM4:
     case PATH_STREAM8: {
         const int waves = path == PATH_STREAM4 ? 4 : 8;
@@ -323,5 +330,6 @@ extern "C" int cch_gemm_kernel_for(int fmt, int swiglu, int64_t num_experts, int
     p.sld = kind == KIND_I8 ? 0 : (int)(2 * ((k + 63) / 64));
     p.b_stride = n * k / (kind == KIND_F4 ? 2 : 1);
     p.sb_stride = n * p.sld;
-    return gemm_tile_unsupported(p, kind, epi) ? -1 : (int)choose_path(p, kind, epi, cus);
+    p.kernel = p.tiles_192 = -1;
+    return gemm_tile_unsupported(p, kind, epi) ? -1 : (int)path_of(p, kind, epi, cus);
 }

@@ -387,7 +387,8 @@ int cch_dyn_quant_i8_rows_smooth(const void *x, const int32_t *src_rows, const f
 int cch_set_option(const char *name, int value);
 
 /* Tiled MFMA kernels: persistent workgroups on 256 x 256 tiles; tiles of 64 x 128, 128 x 128 and 128 x 256; tiles of 32 x 64 whose
- * 4 or 8 waves split K; 256 x 256 tiles whose mostly empty last round (grouped problems) is a second launch of 64 x 128 ones. */
+ * 4 or 8 waves split K; 256 x 256 tiles whose mostly empty last round (grouped problems) is a second launch of 64 x 128 ones; tiles
+ * of 192 x 192 (asked for with "gemm_192_tiles", not with "gemm_kernel"). */
 #define CCH_GEMM_KERNEL_256X256 0
 #define CCH_GEMM_KERNEL_64X128 1
 #define CCH_GEMM_KERNEL_128X128 2
@@ -395,7 +396,8 @@ int cch_set_option(const char *name, int value);
 #define CCH_GEMM_KERNEL_STREAM4 4
 #define CCH_GEMM_KERNEL_STREAM8 5
 #define CCH_GEMM_KERNEL_256X256_TAIL 6
-/* The kernel that a GEMM entry point chooses for aligned operands on a GPU of `cus` CUs, or -1 (the generic kernels, or no
+#define CCH_GEMM_KERNEL_192X192 7
+/* The kernel that a GEMM entry point chooses by itself (whatever the switches say) for aligned operands on a GPU of `cus` CUs, or -1 (the generic kernels, or no
  * problem at all).  fmt: CCH_FMT_E4M3, CCH_FMT_E5M2, CCH_FMT_E2M1, or -1 for int8; num_experts 0: a dense problem; n: columns of B
  * (gate and up halves together).  Host code only, no GPU needed. */
 int cch_gemm_kernel_for(int fmt, int swiglu, int64_t num_experts, int64_t t, int64_t n, int64_t k, int trans_b, int cus);

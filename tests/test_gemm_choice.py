@@ -7,7 +7,7 @@ import pytest
 
 from catccos_amd import _abi
 
-TILE, MID1, MID2, MID3, STREAM4, STREAM8, TAIL = range(7)
+TILE, MID1, MID2, MID3, STREAM4, STREAM8, TAIL, MID192 = range(8)
 I8, E4M3, E2M1 = -1, _abi.FMT_E4M3, _abi.FMT_E2M1
 
 
@@ -47,6 +47,24 @@ def test_the_switch_names_a_kernel():
         assert "gemm_kernel" in L.cch_last_error().decode()
     for v in (*range(7), -1):
         assert L.cch_set_option(b"gemm_kernel", v) == _abi.OK
+
+
+@pytest.mark.parametrize("fmt", [E4M3, _abi.FMT_E5M2, E2M1])
+def test_one_round_of_192x192_tiles(fmt):
+    """Dense products with [N, K] weights: more than two 128 x 128 tiles to a CU and at most one of 192 x 192, at either bound."""
+    for t, n, k in ((3000, 3000, 448 if fmt != E2M1 else 384), (2881, 3072, 128), (1335, 6856, 256), (5466, 1528, 5120)):
+        assert chosen(fmt, 0, 0, t, n, k, 1) == MID192
+    assert chosen(fmt, 0, 0, 16 * 192, 16 * 192, 1024, 1) == MID192              # 256 tiles of 192 x 192
+    assert chosen(fmt, 0, 0, 16 * 192 + 1, 16 * 192, 1024, 1) != MID192          # 272
+    assert chosen(fmt, 0, 0, 128 * 27, 128 * 19, 1024, 1) == MID192              # 513 of 128 x 128, 234 of 192 x 192
+    assert chosen(fmt, 0, 0, 128 * 32, 128 * 16, 1024, 1) != MID192              # 512
+    for other in (chosen(fmt, 0, 0, 3000, 3000, 1024, 0), chosen(fmt, 0, 1, 3000, 3000, 1024, 1), chosen(fmt, 1, 0, 3000, 3008, 1024, 1),
+                  chosen(fmt, 1, 16, 3000, 3008, 1024, 1), chosen(I8, 0, 0, 3000, 3000, 1024, 1)):
+        assert other != MID192                                                   # [K, N], groups, SwiGLU, int8
+
+
+def test_192x192_tiles_and_mxfp4_scale_rows_off_dwords():
+    assert chosen(E2M1, 0, 0, 3000, 3000, 1984, 1) != MID192 and chosen(E4M3, 0, 0, 3000, 3000, 1984, 1) == MID192
 
 
 def test_a_last_round_of_short_tiles_is_a_second_launch():
