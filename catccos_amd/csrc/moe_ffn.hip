@@ -215,6 +215,7 @@ extern "C" int cch_moe_ffn_mxfp8(const void *x, const int32_t *expert_idx, const
                                  void *stream)
 {
     using namespace cch;
+    clear_error();
     CCH_REQUIRE(m >= 0 && k >= 0 && n >= 0 && !(m >> 31) && !(k >> 30) && !(n >> 31), "cch_moe_ffn_mxfp8: bad shape m=%lld k=%lld n=%lld", (long long)m, (long long)k, (long long)n);
     CCH_REQUIRE(top_k >= 1 && top_k <= FFN_MAX_TOPK, "cch_moe_ffn_mxfp8: top_k=%d outside 1..%d", top_k, FFN_MAX_TOPK);
     CCH_REQUIRE(num_experts >= 1 && !(num_experts >> 31), "cch_moe_ffn_mxfp8: num_experts=%lld", (long long)num_experts);
@@ -231,9 +232,13 @@ extern "C" int cch_moe_ffn_mxfp8(const void *x, const int32_t *expert_idx, const
     const int64_t pitch = ffn_pitch(rows, k);
     int rc = ffn_dispatch(x, expert_idx, m, k, top_k, (int)num_experts, reinterpret_cast<int32_t *>(p + w.d2s), s2d, cnt, p + w.packed, pitch, n, p + w.route,
                           w.route_bytes, stream);
-    if (rc == CCH_OK)
+    char note[512] = "";   // that the up projection ran on the generic kernels, if it did: the down projection's call empties the message
+    if (rc == CCH_OK) {
         rc = mx_gmm_swiglu_mx_rows(p + w.packed, pitch, w1, sw1, cnt, p + w.act, p + w.scales, num_experts, rows, n, k, CCH_FMT_E4M3, trans_b, CCH_FMT_E4M3, stream);
+        snprintf(note, sizeof(note), "%s", cch_last_error());
+    }
     if (rc == CCH_OK) rc = cch_mx_gmm(p + w.act, p + w.scales, w2, sw2, cnt, p + w.y, num_experts, rows, k, h, CCH_FMT_E4M3, trans_b, stream);
+    if (rc == CCH_OK && note[0] && !cch_last_error()[0]) fail(CCH_OK, "%s", note);
     if (rc == CCH_OK) rc = cch_moe_token_unpermute(p + w.y, s2d, probs, out, rows, m, k, top_k, stream);
     return rc;
 }

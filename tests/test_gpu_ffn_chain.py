@@ -92,6 +92,29 @@ def test_ffn_chain_against_oracle_chain(cfg):
     assert np.sqrt(np.mean((got - want) ** 2)) <= 2e-2 * rms and np.abs(got - want).max() <= 0.12 * rms
 
 
+@pytest.mark.parametrize("n,k,note", [
+    (96, 128, "MX-quantised output"),     # the up projection alone: 48 columns are no whole MX blocks
+    (128, 132, "16-byte stores"),         # both: K of the up projection, and columns of the down projection, whose note is the later one
+    (128, 128, ""),
+])
+def test_ffn_reports_a_projection_on_the_generic_kernels(n, k, note):
+    """cch_last_error() names the precondition when either projection of the call ran on the one-thread-per-element kernels, and nothing of older calls."""
+    L = cc._abi.lib()
+    m, e, h = 8, 2, n // 2
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    x, idx = torch.randn(m, k, device="cuda", generator=g).bfloat16(), torch.randint(0, e, (m, 2), device="cuda", generator=g, dtype=torch.int32)
+    probs = torch.rand(m, 2, device="cuda", generator=g)
+    w1, sw1, w2, sw2 = (torch.stack([cc.mx_quant(torch.randn(r, c, device="cuda", generator=g).bfloat16())[i] for _ in range(e)])
+                        for r, c in ((n, k), (k, h)) for i in (0, 1))
+    cc.mx_matmul(*cc.mx_quant(torch.randn(4, 40, device="cuda").bfloat16()), *cc.mx_quant(torch.randn(16, 40, device="cuda").bfloat16()), trans_b=1)
+    assert b"generic" in L.cch_last_error() or b"note" in L.cch_last_error()
+    cc.moe_ffn_mxfp8(x[:0], idx[:0], probs[:0], w1, sw1, w2, sw2)     # no tokens: nothing ran, and no note of the call before is left
+    assert L.cch_last_error() == b""
+    out = cc.moe_ffn_mxfp8(x, idx, probs, w1, sw1, w2, sw2)
+    got = L.cch_last_error().decode()
+    assert torch.isfinite(out.float()).all() and (note in got if note else got == ""), got
+
+
 @pytest.mark.parametrize("m,k,n,e,topk,dropped", [
     (1, 64, 128, 1, 1, False),         # one route, one piece of one pair of blocks
     (37, 960, 256, 3, 2, True),        # K an odd multiple of 64, dropped entries of either sign
