@@ -43,7 +43,8 @@ int mx_gmm_swiglu_mx_rows(const void *packed_a, int64_t row_pitch, const void *b
 constexpr int FFN_WAVES = 16;
 constexpr int FFN_MAX_TOPK = 8;
 constexpr int FFN_TOKENS_ROUTES = FFN_WAVES * FFN_MAX_TOPK;   // of one workgroup's tokens
-constexpr int FFN_MAX_GROUPS = 8, FFN_MAX_ROUTES = FFN_MAX_GROUPS * 64 * FFN_WAVES, FFN_MAX_EXPERTS = 256;   // of a call in one launch
+constexpr int FFN_MAX_GROUPS = 8, FFN_MAX_ROUTES = FFN_MAX_GROUPS * 64 * FFN_WAVES;   // of a call in one launch
+constexpr int FFN_MAX_EXPERTS = 256;   // as many groups as the projections take
 constexpr int64_t FFN_MAX_COUNTED = (int64_t)1 << 23;
 constexpr double FFN_CACHED_WEIGHTS = 256e6;
 
@@ -159,8 +160,8 @@ static int ffn_dispatch(const void *x, const int32_t *expert_idx, int64_t m, int
                         int32_t *expert_tokens, void *packed, int64_t pitch, int64_t n, void *route_ws, int64_t route_bytes, void *stream)
 {
     const int64_t rows = m * top_k, ppr = (k + 1023) / 1024, tpw = std::max<int64_t>(1, FFN_WAVES / ppr), workgroups = (m + tpw - 1) / tpw;
-    const bool one_launch = rows <= FFN_MAX_ROUTES && workgroups * rows <= FFN_MAX_COUNTED && experts <= FFN_MAX_EXPERTS && top_k <= FFN_MAX_TOPK &&
-                            k % 64 == 0 && pitch % 16 == 0 && aligned(x, 16) && aligned(packed, 16) && !g_route_three_launches.load(std::memory_order_relaxed);
+    const bool one_launch = rows <= FFN_MAX_ROUTES && workgroups * rows <= FFN_MAX_COUNTED && k % 64 == 0 && pitch % 16 == 0 && aligned(x, 16) &&
+                            aligned(packed, 16) && !g_route_three_launches.load(std::memory_order_relaxed);
     if (!one_launch) {
         const int rc = cch_moe_init_routing(expert_idx, rows, experts, dst_to_src, src_to_dst, expert_tokens, 0, route_ws, route_bytes, stream);
         return rc ? rc : quant_scatter(x, src_to_dst, packed, rows, pitch, m, k, top_k, CCH_FMT_E4M3, CCH_ROUND_RNE, stream);
@@ -218,13 +219,14 @@ extern "C" int cch_moe_ffn_mxfp8(const void *x, const int32_t *expert_idx, const
     clear_error();
     CCH_REQUIRE(m >= 0 && k >= 0 && n >= 0 && !(m >> 31) && !(k >> 30) && !(n >> 31), "cch_moe_ffn_mxfp8: bad shape m=%lld k=%lld n=%lld", (long long)m, (long long)k, (long long)n);
     CCH_REQUIRE(top_k >= 1 && top_k <= FFN_MAX_TOPK, "cch_moe_ffn_mxfp8: top_k=%d outside 1..%d", top_k, FFN_MAX_TOPK);
-    CCH_REQUIRE(num_experts >= 1 && !(num_experts >> 31), "cch_moe_ffn_mxfp8: num_experts=%lld", (long long)num_experts);
+    CCH_REQUIRE(num_experts >= 1 && num_experts <= FFN_MAX_EXPERTS, "cch_moe_ffn_mxfp8: num_experts=%lld outside 1..%d", (long long)num_experts, FFN_MAX_EXPERTS);
     CCH_REQUIRE(n % 2 == 0, "cch_moe_ffn_mxfp8: n=%lld must be even (gate | up halves)", (long long)n);
+    CCH_REQUIRE(trans_b == 0 || trans_b == 1, "cch_moe_ffn_mxfp8: trans_b %d", trans_b);
     const int64_t rows = m * top_k, h = n / 2;
     CCH_REQUIRE(!(rows >> 31), "cch_moe_ffn_mxfp8: %lld routes", (long long)rows);
     if (m == 0 || k == 0) return CCH_OK;
     const FfnWorkspace w = ffn_workspace(m, k, top_k, num_experts, n);
-    CCH_REQUIRE(x && expert_idx && probs && out, "cch_moe_ffn_mxfp8: null pointer");
+    CCH_REQUIRE(x && expert_idx && probs && out && (n == 0 || (w1 && sw1 && w2 && sw2)), "cch_moe_ffn_mxfp8: null pointer");
     CCH_REQUIRE(workspace && aligned(workspace, 512) && workspace_bytes >= w.end, "cch_moe_ffn_mxfp8: workspace of %lld bytes, need %lld on a 512-byte boundary",
                 (long long)workspace_bytes, (long long)w.end);
     uint8_t *p = static_cast<uint8_t *>(workspace);

@@ -102,6 +102,34 @@ def test_routing_and_unpermute_arguments():
         assert L.cch_set_option(name, default) == _abi.OK, name
 
 
+def test_ffn_arguments():
+    L = _abi.lib()
+
+    def call(m=4, k=128, top_k=2, e=3, n=64, trans_b=1, ws=P, ws_bytes=1 << 40, x=P, w=P):
+        return L.cch_moe_ffn_mxfp8(x, P, P, w, P, w, P, P, m, k, top_k, e, n, trans_b, ws, ws_bytes, None)
+    for m in (4, 0):   # also where there is nothing to do, as the stages called one by one
+        rejected(call(m=m, top_k=0), "top_k")
+        rejected(call(m=m, top_k=9), "top_k")
+        rejected(call(m=m, e=0), "num_experts")
+        rejected(call(m=m, e=257), "num_experts", "256")
+        rejected(call(m=m, n=63), "even")
+        rejected(call(m=m, trans_b=2), "trans_b")
+    rejected(call(m=-1), "shape")
+    rejected(call(k=1 << 30), "shape")
+    rejected(call(m=1 << 29, top_k=4), "routes")
+    rejected(call(x=None), "null")
+    rejected(call(w=None), "null")
+    need = L.cch_moe_ffn_mxfp8_workspace_bytes(4, 128, 2, 3, 64)
+    rejected(call(ws_bytes=need - 1), "workspace", str(need))
+    rejected(call(ws=P + 256), "512-byte")
+    rejected(call(ws=None), "workspace")
+    assert call(m=0, ws=None, x=None) == call(k=0, ws=None, x=None) == _abi.OK
+    assert L.cch_moe_ffn_mxfp8_workspace_bytes(-1, 128, 2, 3, 64) == L.cch_moe_ffn_mxfp8_workspace_bytes(4, 128, 0, 3, 64) == 0
+    rejected(L.cch_set_option(b"gemm_192_tiles", 2), "gemm_192_tiles")
+    rejected(L.cch_set_option(b"gemm_192_tiles", -2), "gemm_192_tiles")
+    assert L.cch_set_option(b"gemm_192_tiles", -1) == _abi.OK
+
+
 def test_empty_problems_succeed_without_a_device():
     L = _abi.lib()
     assert L.cch_gemm_i8_dequant(None, None, None, None, None, 0, 8, 8, 0, None) == _abi.OK
