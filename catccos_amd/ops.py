@@ -513,8 +513,8 @@ def moe_ffn_mxfp8(x, expert_idx, probs, w1, sw1, w2, sw2, trans_b=1):
         raise ValueError("top_k must be 1..8")
     if expert_idx.dtype != torch.int32 or probs.dtype != torch.float32:
         raise ValueError("expert_idx must be int32 and probs float32")
-    if w1.dim() != 3 or w2.dim() != 3 or any(w.dtype != torch.uint8 for w in (w1, sw1, w2, sw2)):
-        raise ValueError("w1, w2 must be 3-D uint8 tensors, sw1, sw2 uint8")
+    if w1.dim() != 3 or w2.dim() != 3 or any(w.dtype != torch.uint8 for w in (w2, sw2)) or any(w.element_size() != 1 for w in (w1, sw1)):
+        raise ValueError("w1, w2 must be 3-D uint8 tensors, sw1, sw2 uint8 (w1, sw1: any type of one byte)")
     n = w1.shape[1] if trans_b else w1.shape[2]
     if n % 2 or (w1.shape[2] if trans_b else w1.shape[1]) != k or sw1.numel() != e * scale_cols(k) * n:
         raise ValueError("shape mismatch between x, w1 and sw1")

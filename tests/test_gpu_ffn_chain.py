@@ -92,6 +92,21 @@ def test_ffn_chain_against_oracle_chain(cfg):
     assert np.sqrt(np.mean((got - want) ** 2)) <= 2e-2 * rms and np.abs(got - want).max() <= 0.12 * rms
 
 
+def test_ffn_takes_up_projections_of_any_one_byte_type():
+    """The up projection's payload and scales are bytes whatever their element type is called, as in mx_grouped_matmul_swiglu_packed."""
+    m, k, n, e = 20, 128, 128, 3
+    g = torch.Generator(device="cuda").manual_seed(9)
+    x, idx = torch.randn(m, k, device="cuda", generator=g).bfloat16(), torch.randint(0, e, (m, 2), device="cuda", generator=g, dtype=torch.int32)
+    probs = torch.rand(m, 2, device="cuda", generator=g)
+    w1, sw1, w2, sw2 = (torch.stack([cc.mx_quant(torch.randn(r, c, device="cuda", generator=g).bfloat16())[i] for _ in range(e)])
+                        for r, c in ((n, k), (k, n // 2)) for i in (0, 1))
+    want = cc.moe_ffn_mxfp8(x, idx, probs, w1, sw1, w2, sw2)
+    got = cc.moe_ffn_mxfp8(x, idx, probs, w1.view(torch.float8_e4m3fn), sw1.view(torch.int8), w2, sw2)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    with pytest.raises(ValueError, match="uint8"):
+        cc.moe_ffn_mxfp8(x, idx, probs, w1, sw1, w2.view(torch.int8), sw2)
+
+
 @pytest.mark.parametrize("n,k,note", [
     (96, 128, "MX-quantised output"),     # the up projection alone: 48 columns are no whole MX blocks
     (128, 132, "16-byte stores"),         # both: K of the up projection, and columns of the down projection, whose note is the later one
