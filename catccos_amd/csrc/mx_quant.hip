@@ -306,14 +306,14 @@ static int launch_rows(const void *x, void *payload, void *scales, int64_t m, in
     const int64_t wpr = (nblk * 4 + 63) / 64;
     const bool vec = (k % 8 == 0) && aligned(x, 16) && aligned(payload, 8);
     const bool pair = vec && (k % 16 == 0) && aligned(payload, 16) && QUANT_UNROLL % 2 == 0;
-    int dev = 0, cus = 0;
-    CCH_HIP(hipGetDevice(&dev));
-    CCH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const int64_t max_blocks = (int64_t)cus * QUANT_BLOCKS_PER_CU;
     if constexpr (HWCVT) {
         const int rc = launch_rows_fast<FMT, false>(x, payload, scales, m, k, stream);
         if (rc != 1) return rc;
     }
+    int dev = 0, cus = 0;
+    CCH_HIP(hipGetDevice(&dev));
+    CCH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    const int64_t max_blocks = (int64_t)cus * QUANT_BLOCKS_PER_CU;
     const int64_t rows_per_launch = std::max<int64_t>(1, (int64_t)(1 << 30) / wpr);
     for (int64_t r0 = 0; r0 < m; r0 += rows_per_launch) {
         const int64_t rows = std::min(rows_per_launch, m - r0);
