@@ -644,7 +644,7 @@ def main():
                 extra["moe_token_unpermute_top2"]["parity"] = {"bit_exact_whole_tensor": bool(np.array_equal(
                     out_u.view(torch.int16).cpu().numpy().view(np.uint16), uh))}
             del ys, out_u
-            # routing sort of config 4's routes (8192 tokens, top-2, 16 experts): three short launches through the C ABI
+            # routing sort of config 4's routes (8192 tokens, top-2, 16 experts): one short launch through the C ABI
             rt_rows, rt_e = 8192 * 2, 16
             rt_idx = torch.randint(0, rt_e, (rt_rows,), dtype=torch.int32, device=dev)
             rt_d2s = torch.empty(rt_rows, dtype=torch.int32, device=dev)
@@ -667,7 +667,7 @@ def main():
             e1.record()
             torch.cuda.synchronize()
             extra["moe_init_routing_cfg4_routes"] = {"us": round(e0.elapsed_time(e1) * 1e3 / 100, 2), "routes": rt_rows, "experts": rt_e,
-                                                     "launches_per_call": 3}
+                                                     "launches_per_call": 1}
             if cpu:
                 t0 = time.perf_counter()
                 d2s_h, s2d_h, cnt_h = orc.moe_init_routing(rt_idx.cpu().numpy(), rt_e)
@@ -712,8 +712,8 @@ def main():
             del pu, su, pv, sv
             # The MXFP8 FFN of one rank from routing to combine, at the largest shape of the reference example's own list
             # (examples/ascend950_dispatch_ffn_combine/scripts/test_shapes.csv: 512 tokens, K 7168, N 4096) with its run.sh's
-            # 16 experts and top-6: seven launches (routing sort x3, quantise-and-scatter, GMM1 + SwiGLU + quantise, GMM2,
-            # un-permute), eager and as one HIP graph.  Weight bytes per pass: 16 x (29.4 + 14.7) MB + scales = 0.73 GB.
+            # 16 experts and top-6: one library call of five launches (routing sort and quantise-and-scatter, GMM1 + SwiGLU + quantise
+            # in two, GMM2, un-permute), eager and as one HIP graph.  Weight bytes per pass: 16 x (29.4 + 14.7) MB + scales = 0.73 GB.
             mf, ef, topf = 512, 16, 6
             xf = torch.randn(mf, K, device=dev).to(torch.bfloat16)
             idf = torch.argsort(torch.rand(mf, ef, device=dev), dim=1)[:, :topf].to(torch.int32).contiguous()

@@ -19,7 +19,7 @@ namespace cch {
 
 constexpr int ROUTE_CHUNK = 1024;       // rows per workgroup
 constexpr int ROUTE_MAX_EXPERTS = 1024;
-// cch_set_option("routing_three_launches", 1): the general path also where one workgroup would do (for tests)
+// cch_set_option("routing_three_launches", 1): the general path also where one launch would do (for tests)
 std::atomic<int> g_route_three_launches{0};
 
 // hist[e * nchunks + c] (BY_CHUNK: hist[c * experts + e]) = rows of chunk c routed to expert e; dst_to_src of the chunk's positions

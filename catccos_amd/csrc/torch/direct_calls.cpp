@@ -274,7 +274,7 @@ PyObject *MxGroupedMatmul(PyObject *, PyObject *const *v, Py_ssize_t nv)
     END_HANDLE_TH_ERRORS
 }
 
-// moe_ffn_mxfp8(x, expert_idx, probs, w1, sw1, w2, sw2, trans_b): what lies between the five launches is one allocation
+// moe_ffn_mxfp8(x, expert_idx, probs, w1, sw1, w2, sw2, trans_b): what lies between the launches is one allocation
 PyObject *MoeFfnMxfp8(PyObject *, PyObject *const *v, Py_ssize_t nv)
 {
     HANDLE_TH_ERRORS

@@ -492,7 +492,7 @@ def mx_grouped_matmul_mapped(a, sa, b, sb, group_sizes, out_row_map, out, fmt="e
 
 
 def moe_ffn_mxfp8(x, expert_idx, probs, w1, sw1, w2, sw2, trans_b=1):
-    """The MXFP8 MoE FFN of one rank that holds every expert, routing to combine, four or five launches on the current stream
+    """The MXFP8 MoE FFN of one rank that holds every expert, routing to combine, one library call on the current stream
     (the reference's Ascend950DispatchFFNCombine, examples/ascend950_dispatch_ffn_combine/ascend950_dispatch_ffn_combine_device.h:124-176):
     routing sort -> MXFP8 quantise-and-scatter -> GMM1 + SwiGLU + MXFP8 quantise -> GMM2 -> weighted un-permute.
 

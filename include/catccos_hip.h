@@ -307,7 +307,9 @@ int cch_moe_init_routing_noalloc(const int32_t *expert_idx, int64_t rows, int nu
  * Ascend950DispatchFFNCombine (examples/ascend950_dispatch_ffn_combine/
  * ascend950_dispatch_ffn_combine_device.h:124-176) with the exchanges of one rank: the stages cch_moe_init_routing,
  * cch_mx_quant_scatter_packed, cch_mx_gmm_swiglu_mx_packed, cch_mx_gmm and cch_moe_token_unpermute on one
- * stream, four or five launches (up to 8192 routes the sort and the quantiser are one).
+ * stream, launches only.  Sort and quantiser are one launch up to 8192 routes (fewer where tokens are long), a projection is one or,
+ * where its last round of tiles would be mostly empty, two.  num_experts 1..256.  After CCH_OK cch_last_error() names the precondition that
+ * kept a projection from the tiled kernels, or is empty.
  *   x           bf16 [m, k]; expert_idx int32 [m, top_k] (an entry outside [0, num_experts) is dropped)
  *   probs       fp32 [m, top_k]; top_k 1..8
  *   w1 / sw1    E4M3 payload and E8M0 scales of the up projections [num_experts] x [k, n] (gate columns first) in the

@@ -76,7 +76,7 @@ def _calls(dev="cuda"):
         out.append((cc.dynamic_quant_i8, (x, idx.reshape(-1), 2, mode), {}))
     for cumsum in (False, True):
         out.append((cc.moe_init_routing, (idx, e, cumsum), {}))
-    out.append((cc.moe_init_routing, (torch.randint(0, e, (9000,), device=dev, generator=g, dtype=torch.int32), e), {}))
+    out.append((cc.moe_init_routing, (torch.randint(0, e, (40000,), device=dev, generator=g, dtype=torch.int32), e), {}))
     q, pt = cc.dynamic_quant_i8(x)
     for tb in (0, 1):
         wi = torch.randint(-127, 128, (e, n, k) if tb else (e, k, n), dtype=torch.int8, device=dev, generator=g)

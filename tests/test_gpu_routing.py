@@ -30,8 +30,8 @@ def test_routing_exact(case, cumsum):
 
 @pytest.mark.parametrize("case", [(1, 1), (63, 3), (64, 256), (1000, 16), (4097, 200), (8192, 256), (8192, 1), (8193, 256), (500, 257)])
 def test_routing_one_workgroup_equals_three_launches(case):
-    """Up to 8192 rows and 256 experts one workgroup does the whole sort in one launch; the general path (three launches,
-    `routing_three_launches`) and the oracle give the same integers, also just past either limit and with dropped routes."""
+    """Up to 1024 rows and 256 experts one workgroup does the whole sort, up to 32768 one launch of a workgroup per 1024; the general path (three launches,
+    `routing_three_launches`) and the oracle give the same integers, also past the limit of experts and with dropped routes."""
     rows, e = case
     rng = np.random.default_rng(rows * 7 + e)
     idx = rng.integers(-1, e + 1, rows).astype(np.int32)      # -1 and e are dropped
@@ -54,7 +54,7 @@ def test_routing_one_workgroup_equals_three_launches(case):
 @pytest.mark.parametrize("rows", [1023, 1024, 1025, 2048, 2049, 4096, 4097, 8191, 8192])
 @pytest.mark.parametrize("e", [1, 64, 65, 256])
 def test_routing_one_workgroup_edges(rows, e):
-    """The one-workgroup kernel is instantiated on the 64-row groups of a wave (1, 2, 4, 8) and scans experts 64 at a time:
+    """The kernels of one launch differ in the groups of 1024 rows that they count (1, 2, 4, 8) and scan experts 64 at a time:
     the row counts and expert counts on either side of each limit, with dropped routes (which leave -1 behind the last)."""
     rng = np.random.default_rng(rows * 31 + e)
     idx = rng.integers(-1, e + 1, rows).astype(np.int32)

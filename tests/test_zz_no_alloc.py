@@ -43,8 +43,9 @@ def _case(rows, experts, seed):
 def test_noalloc_routing_matches_workspace_routing_on_two_calls():
     assert _abi.lib().cch_init(0) == 0
     # the second call is smaller in rows and in experts, so it reuses a part of what the first one left behind
-    # (up to 8192 rows and 256 experts the sort is one workgroup that needs no histogram area: the second call stays above that)
-    for (rows, experts, cumsum, seed) in ((70000, 256, 0, 1), (20000, 16, 1, 2), (5000, 16, 1, 4), (1, 1, 0, 3)):
+    # (up to 32768 rows and 256 experts the sort is one launch that needs no histogram area: the second call stays above that; the third
+    # reuses it for more experts than that launch takes; the last two do not touch it)
+    for (rows, experts, cumsum, seed) in ((70000, 256, 0, 1), (40000, 16, 1, 2), (3000, 300, 0, 5), (5000, 16, 1, 4), (1, 1, 0, 3)):
         idx = _case(rows, experts, seed) if rows > 10 else torch.zeros(rows, dtype=torch.int32, device="cuda")
         # outputs allocated before the call under test; the call itself must not allocate
         outs = (torch.full((rows,), -7, dtype=torch.int32, device="cuda"), torch.full((rows,), -7, dtype=torch.int32, device="cuda"),
